@@ -143,7 +143,12 @@ typedef struct {
     const int *src_count;      /* [nshots] */
     const int *src_nodes;      /* [sum of src_count] */
     const double *src_weight;  /* [sum of src_count][2]: u and w weights */
-    int kernel_variant;        /* 0 = default (1), 1 = packed values + 2-way gather, 2 = separate value
+    int kernel_variant;        /* 0 = chosen by the library: with shots_per_lane_group 0, row_order NULL
+                                  and block 0 or 256, meshes numbered line by line take the grid
+                                  layout (patches of rows with their neighbours' fields in LDS, the
+                                  matrices as a table of the distinct row stencils; FP64, and the FP32
+                                  forms unless 64-shot lane groups would be mostly full); else 1.
+                                  1 = packed values + 2-way gather, 2 = separate value
                                   arrays, 3 = 1 + streaming hints on data used once per step,
                                   4 = 3 + own-row fields kept from the diagonal gather and own-row
                                   accelerations (p in the FP32 forms) / Kahan terms loaded first,

@@ -1,6 +1,6 @@
 """Autotuner for the step kernel: picks the block size, the lane grouping
 (rows per wavefront vs shots per lane group), the kernel variant (with the
-sliced layouts' sorting window), the XCD block map (contiguous ranges,
+sliced layouts' sorting window; or the library's own choice), the XCD block map (contiguous ranges,
 round-robin, or stripes of Q row blocks) and the row order (node order, a
 Hilbert walk over the node coordinates, or patches of a structured mesh) by
 timing short runs of the actual problem on the GPU.
@@ -32,6 +32,8 @@ def candidates(nshots, nodes=160801, patches=False):
         return dict(shots_per_lane_group=sp, block=block, kernel_variant=variant, xcd_remap=xcd, row_order=order,
                     sell_sigma=sigma)
 
+    # the library's own choice (the grid layout on meshes numbered line by line)
+    own = [c(0, 0, 0, True, "node")]
     if nshots <= 1:
         # one row per lane: per-row layouts, the sliced layout (8) and, on meshes
         # with a line structure, the sliced layout with LDS-staged halos over
@@ -42,7 +44,7 @@ def candidates(nshots, nodes=160801, patches=False):
         if patches:
             cands += [c(1, b, 9, x, o) for b, o in ((256, "patch16x16"), (256, "patch32x8"), (64, "patch16x4"))
                       for x in (True, False)]
-        return cands
+        return own + cands
     if nshots <= 4:
         sps, blocks = [4, 16], [256]
     elif nshots <= 16:
@@ -60,7 +62,7 @@ def candidates(nshots, nodes=160801, patches=False):
     for sp in sps:
         for b in blocks:
             cands += [c(sp, b, v, q, "node") for q in stripe_widths(nodes, sp, b) if q > 1 for v in variants]
-    return cands
+    return own + cands
 
 
 def tune(op, md, src, rec, dt, f0, t0, precision, steps=40, cands=None, log=None, coords=None):

@@ -6,9 +6,11 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "seisfem_gpu.h"
@@ -205,6 +207,26 @@ extern "C" void abc_mpml(int node_num, int element_num, int element_order, int *
 // ---------------------------------------------------------------------------
 // operators
 
+// Grid layout of one operator for patches of at most `most` rows (GridArgs).
+struct GridPlan {
+    int most = 0, align = 0;    // rows of a patch; nodes that lines and patches start on a multiple of (0: any)
+    bool ok = false;            // false: the operator does not fit the layout
+    GridShape g;
+    int mode = GRID_ROWS, magic = 0;
+    int *rows = nullptr, *cls = nullptr, *slice = nullptr, *smax = nullptr, *toff = nullptr, *tlen = nullptr,
+        *trep = nullptr, *tdst = nullptr, *moff = nullptr, *sdel = nullptr;
+    int nitems = 0;             // stencils in the tables
+    long long nentries = 0;     // table entries
+    long long nslots = 0;       // slots of 64 per-row values
+    void *tab[2] = {nullptr, nullptr}, *mval[2] = {nullptr, nullptr}; // FP64, FP32
+    bool vals[2] = {false, false};
+    ~GridPlan()
+    {
+        for (int *q : {rows, cls, slice, smax, toff, tlen, trep, tdst, moff, sdel}) dfree(q);
+        for (int k = 0; k < 2; ++k) { dfree(tab[k]); dfree(mval[k]); }
+    }
+};
+
 struct sfg_operator {
     int n = 0, nnz = 0, device = 0;
     int *rp = nullptr, *ci = nullptr;
@@ -213,6 +235,12 @@ struct sfg_operator {
     float *v32 = nullptr;  // [7][nnz]
     double *p64 = nullptr; // [nnz][8]: M, S1..S6, 0 (one wide load per nonzero)
     float *p32 = nullptr;  // [nnz][8]
+    // grid layouts of this operator, built by the first run that takes one and
+    // shared by its later runs (grid_plan); freed with the operator
+    mutable std::mutex grid_mu;
+    mutable std::vector<std::unique_ptr<GridPlan>> grid;
+    mutable int grid_tried = 0;         // lines looked for
+    mutable GridShape lines;            // line, lines, hx, hy (line = 0: none)
 };
 
 static int check_csr(int n, const int *p, const int *j, int m)
@@ -298,6 +326,311 @@ extern "C" void sfg_operator_destroy(sfg_operator *op)
     delete op;
 }
 
+// Nodes per line of a mesh numbered line by line, guessed from the pattern: the
+// nearest column of a row beyond GRID_REACH is the first one on the next line,
+// at most GRID_REACH before the node above it.  Wrong guesses are caught by the
+// reach check.  Returns candidates, fewest nodes first.
+static std::vector<int> line_candidates(const sfg_operator *op)
+{
+    const int n = op->n;
+    int lo = n;
+    for (int k = 0; k < 64; ++k) {
+        const int i = (int)((long long)n * k / 64);
+        for (int q = op->hrp[i]; q < op->hrp[i + 1]; ++q) {
+            const int d = op->hci[q] - i;
+            if (d > GRID_REACH && d < lo) lo = d;
+        }
+    }
+    std::vector<int> out;
+    for (int l = lo; l <= lo + GRID_REACH; ++l)
+        if (l >= 4 * GRID_REACH && l < n && n % l == 0) out.push_back(l);
+    return out;
+}
+
+// Patch shape: the one whose blocks touch the fewest 64-byte pieces of the
+// state: 10 staged words per halo node and 28 own words per row (in and out).
+static void choose_patch(GridShape &g, int most, int align)
+{
+    double best = 1e300;
+    GridShape b = g;
+    for (int pw0 = 4; pw0 <= 64 && pw0 <= most; ++pw0) {
+        GridShape c = g;
+        c.px = (g.line + pw0 - 1) / pw0;
+        const bool even = g.hx > 1 || g.hy > 1 || align > 0;
+        if (align > 0 && pw0 % align) continue;
+        c.pw = even ? pw0 : (g.line + c.px - 1) / c.px;
+        const int ph0 = most / c.pw;
+        if (ph0 < 1) continue;
+        const int py = (g.lines + ph0 - 1) / ph0;
+        c.ph = even ? ph0 : (g.lines + py - 1) / py;
+        c.npatch = c.px * py;
+        c.W = c.pw + 2 * g.hx;
+        c.halo = c.W * (c.ph + 2 * g.hy);
+        if (c.halo > 2 * most) continue;
+        // quadratic elements alternate between kinds of nodes along and across the
+        // lines: sides that divide into whole waves of each keep waves to one class
+        if (even && (c.pw % 2 || c.ph % 2 || c.pw * c.ph != most)) continue;
+        const double cost = (double)c.npatch * ((c.ph + 2.0 * g.hy) * (c.W * 8.0 + 64.0) * 10.0 +
+                                                c.ph * (c.pw * 8.0 + 64.0) * 28.0);
+        if (cost < best) best = cost, b = c;
+    }
+    g = b;
+}
+
+// Most classes a table may hold (their entries, at most 25 each, are numbered in
+// 24 bits; a table of this size is at most 6.5 MB, and the rows of a patch use a
+// few of its classes).
+static const int kGridClasses = 4096;
+
+// Groups the rows by hash; classes in order of appearance.  false: more than kGridClasses
+static bool group_rows(const unsigned long long *h, int n, std::vector<int> &cls, std::vector<int> &rep)
+{
+    cls.resize(n);
+    rep.clear();
+    std::unordered_map<unsigned long long, int> seen;
+    unsigned long long last[4] = {0, 0, 0, 0};
+    int lastc[4] = {-1, -1, -1, -1}, at = 0;
+    for (int i = 0; i < n; ++i) {
+        int c = -1;
+        for (int k = 0; k < 4; ++k)
+            if (lastc[k] >= 0 && last[k] == h[i]) c = lastc[k];
+        if (c < 0) {
+            const auto it = seen.emplace(h[i], (int)rep.size());
+            c = it.first->second;
+            if (it.second) {
+                if ((int)rep.size() >= kGridClasses) return false;
+                rep.push_back(i);
+            }
+            last[at] = h[i];
+            lastc[at] = c;
+            at = (at + 1) & 3;
+        }
+        cls[i] = c;
+    }
+    return true;
+}
+
+// Tables of the patches, whose rows' keys (first entry of the class in a table of
+// all classes | nonzeros << 24, sorted within the patch, places without a row last
+// with key 0) are rewritten to the patch's own table.  Patches with the same
+// classes share one.  false: a patch needs more than GRID_TABLE entries, or all of
+// them more than 2^20.
+static bool patch_tables(GridShape &g, const std::vector<int> &cptr, const std::vector<int> &rep, std::vector<int> &keys,
+                         std::vector<int> &toff, std::vector<int> &tlen, std::vector<int> &trep, std::vector<int> &tdst,
+                         long long *nentries)
+{
+    std::unordered_map<std::string, std::pair<int, int>> seen; // classes -> first entry, entries
+    toff.clear();
+    tlen.clear();
+    trep.clear();
+    tdst.clear();
+    long long total = 0;
+    g.table = 0;
+    std::vector<int> have;
+    for (int p = 0; p < g.npatch; ++p) {
+        int *k = keys.data() + (size_t)p * g.most;
+        have.clear();
+        int at = 0, prev = -1, base = 0;
+        for (int q = 0; q < g.most; ++q) {
+            if (k[q] >> 24 == 0) continue;      // no row here (or a row without nonzeros)
+            if (k[q] != prev) {
+                prev = k[q];
+                base = at;
+                at += prev >> 24;
+                have.push_back(prev & 0xffffff);
+            }
+            k[q] = base | (prev & ~0xffffff);
+        }
+        if (at > GRID_TABLE) return false;
+        const auto it = seen.emplace(std::string((const char *)have.data(), sizeof(int) * have.size()),
+                                     std::make_pair((int)total, at));
+        if (it.second) {
+            int d = (int)total;
+            for (int e : have) {
+                const int c = (int)(std::upper_bound(cptr.begin(), cptr.end(), e) - cptr.begin()) - 1;
+                trep.push_back(rep[c]);
+                tdst.push_back(d);
+                d += cptr[c + 1] - cptr[c];
+            }
+            total += at;
+            if (total > 1 << 20) return false;
+        }
+        toff.push_back(it.first->second.first);
+        tlen.push_back(it.first->second.second);
+        g.table = std::max(g.table, at);
+    }
+    *nentries = total;
+    return true;
+}
+
+template <class T>
+static int upload(T **p, const std::vector<T> &v, hipStream_t st)
+{
+    int rc = dalloc(p, v.size());
+    if (rc) return rc;
+    if (!v.empty()) HIPCHK(hipMemcpyAsync(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return SFG_OK;
+}
+
+// The mesh's lines and the reach of its columns, found once per operator (the
+// caller holds grid_mu).
+static int find_lines(const sfg_operator *op, hipStream_t st)
+{
+    if (op->grid_tried) return SFG_OK;
+    int *flags = nullptr, f[4];
+    int rc = dalloc(&flags, 4);
+    if (rc) return rc;
+    hipError_t e = hipSuccess;
+    for (int l : line_candidates(op)) {
+        e = launch_fill_zero(flags, sizeof f, st);
+        if (e == hipSuccess) e = launch_grid_reach(op->n, op->rp, op->ci, l, flags, flags + 2, st);
+        if (e == hipSuccess) e = hipMemcpyAsync(f, flags, sizeof f, hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess || f[2] != 0) continue;
+        op->lines.line = l;
+        op->lines.lines = op->n / l;
+        op->lines.hx = f[0];
+        op->lines.hy = f[1];
+        break;
+    }
+    dfree(flags);
+    if (e != hipSuccess) return fail(SFG_E_HIP, "grid layout: %s", hipGetErrorString(e));
+    op->grid_tried = 1;
+    return SFG_OK;
+}
+
+static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
+{
+    const int n = op->n;
+    P.ok = false;
+    int rc = find_lines(op, st);
+    if (rc) return rc;
+    GridShape g = op->lines;
+    if (g.line == 0) return SFG_OK;
+    g.most = P.most;
+    g.pitch = P.align > 0 ? (g.line + P.align - 1) / P.align * P.align : g.line;
+    choose_patch(g, P.most, P.align);
+    if (g.npatch == 0) return SFG_OK;
+    P.magic = 65536 / g.W + 1;
+    for (int q = 0; q < GRID_HALO_MAX; ++q)
+        if ((q * P.magic) >> 16 != q / g.W) return SFG_OK;
+    P.g = g;
+    const int nw = g.npatch * (g.most / 64);
+    int f[4];
+    struct Tmp { // device scratch of this call
+        int *flags = nullptr, *key = nullptr;
+        unsigned long long *h = nullptr;
+        ~Tmp() { dfree(flags); dfree(key); dfree(h); }
+    } tmp;
+    if ((rc = dalloc(&tmp.flags, 4)) || (rc = dalloc(&tmp.h, 2 * (size_t)n)) || (rc = dalloc(&tmp.key, n)) ||
+        (rc = dalloc(&P.rows, (size_t)g.npatch * g.most)) || (rc = dalloc(&P.cls, (size_t)g.npatch * g.most)) ||
+        (rc = dalloc(&P.slice, nw)) || (rc = dalloc(&P.smax, nw)))
+        return rc;
+    // the most compact mode whose tables fit
+    std::vector<unsigned long long> h(n);
+    HIPCHK(launch_grid_hash(n, op->rp, op->ci, op->v64, (size_t)op->nnz, tmp.h, st));
+    std::vector<int> cls, rep, keys((size_t)g.npatch * g.most), cptr, toff, tlen, trep, tdst;
+    int mode = GRID_ROWS;
+    for (int m = GRID_CLASS; m < GRID_ROWS && mode == GRID_ROWS; ++m) {
+        HIPCHK(hipMemcpyAsync(h.data(), tmp.h + (m == GRID_CLASS ? n : 0), sizeof(unsigned long long) * n,
+                              hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        if (!group_rows(h.data(), n, cls, rep)) continue;
+        const int nclass = (int)rep.size();
+        cptr.assign(nclass + 1, 0);
+        for (int c = 0; c < nclass; ++c) cptr[c + 1] = cptr[c] + op->hrp[rep[c] + 1] - op->hrp[rep[c]];
+        struct Up { // device copies of rep and cptr
+            int *rep = nullptr, *cptr = nullptr;
+            ~Up() { dfree(rep); dfree(cptr); }
+        } up;
+        if ((rc = upload(&up.rep, rep, st)) || (rc = upload(&up.cptr, cptr, st))) return rc;
+        HIPCHK(launch_fill_zero(tmp.flags, 4 * sizeof(int), st));
+        HIPCHK(hipMemcpyAsync(tmp.key, cls.data(), sizeof(int) * n, hipMemcpyHostToDevice, st));
+        HIPCHK(launch_grid_check(n, op->rp, op->ci, op->v64, (size_t)op->nnz, m == GRID_CLASS ? 0 : 1, tmp.key, up.rep,
+                                 tmp.flags, st));
+        HIPCHK(launch_grid_sort(g, m, op->rp, tmp.key, up.cptr, P.rows, P.cls, P.slice, P.smax, st));
+        HIPCHK(hipMemcpyAsync(f, tmp.flags, sizeof f, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipMemcpyAsync(keys.data(), P.cls, sizeof(int) * keys.size(), hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        if (f[0] == 0 && patch_tables(g, cptr, rep, keys, toff, tlen, trep, tdst, &P.nentries)) mode = m;
+    }
+    P.mode = mode;
+    if (mode == GRID_ROWS) {
+        g.table = 0;
+        P.nentries = 0;
+        HIPCHK(launch_grid_sort(g, mode, op->rp, tmp.key, nullptr, P.rows, P.cls, P.slice, P.smax, st));
+    } else {
+        P.nitems = (int)trep.size();
+        HIPCHK(hipMemcpyAsync(P.cls, keys.data(), sizeof(int) * keys.size(), hipMemcpyHostToDevice, st));
+        if ((rc = upload(&P.toff, toff, st)) || (rc = upload(&P.tlen, tlen, st)) || (rc = upload(&P.trep, trep, st)) ||
+            (rc = upload(&P.tdst, tdst, st)))
+            return rc;
+    }
+    P.g = g;
+    HIPCHK(launch_grid_place(g, P.rows, P.cls, st));
+    if (mode != GRID_CLASS) {
+        std::vector<int> smax(nw), moff(nw);
+        HIPCHK(hipMemcpyAsync(smax.data(), P.smax, sizeof(int) * nw, hipMemcpyDeviceToHost, st));
+        HIPCHK(hipStreamSynchronize(st));
+        for (int w = 0; w < nw; ++w) {
+            moff[w] = (int)P.nslots;
+            P.nslots += smax[w];
+        }
+        if (P.nslots > 0x7fffffffLL / (7 * 64)) return SFG_OK;
+        if ((rc = upload(&P.moff, moff, st))) return rc;
+        if (mode == GRID_ROWS && (rc = dalloc(&P.sdel, (size_t)P.nslots * 64))) return rc;
+    }
+    HIPCHK(hipStreamSynchronize(st));
+    P.ok = true;
+    return SFG_OK;
+}
+
+// The operator's grid layout for patches of at most `most` rows with the values
+// of one precision, built on first use (on `st`, which it waits for).  *out =
+// null when the operator does not fit the layout (no line structure).
+static int grid_plan(const sfg_operator *op, int most, int align, bool f32, hipStream_t st, const GridPlan **out)
+{
+    *out = nullptr;
+    std::lock_guard<std::mutex> lk(op->grid_mu);
+    GridPlan *P = nullptr;
+    for (auto &p : op->grid)
+        if (p->most == most && p->align == align) P = p.get();
+    if (!P) {
+        std::unique_ptr<GridPlan> fresh(new GridPlan);
+        fresh->most = most;
+        fresh->align = align;
+        int rc = build_grid(op, *fresh, st);
+        if (rc) return rc;
+        P = fresh.get();
+        op->grid.push_back(std::move(fresh));
+    }
+    if (!P->ok) return SFG_OK;
+    const int k = f32 ? 1 : 0, w = f32 ? 4 : 8;
+    if (!P->vals[k]) {
+        const void *v = f32 ? (const void *)op->v32 : (const void *)op->v64;
+        int rc;
+        char *tv = nullptr, *mv = nullptr;
+        if ((rc = dalloc(&tv, (size_t)P->nentries * 8 * w))) return rc;
+        P->tab[k] = tv;
+        if (P->mode != GRID_CLASS) {
+            const size_t per = P->mode == GRID_ROWS ? 7 : 1;
+            if ((rc = dalloc(&mv, (size_t)P->nslots * 64 * per * w))) return rc;
+            P->mval[k] = mv;
+        }
+        if (P->nitems)
+            HIPCHK(launch_grid_table(P->nitems, P->trep, P->tdst, op->rp, op->ci, P->g.line, P->g.W, v, (size_t)op->nnz,
+                                     w, tv, st));
+        if (P->mode != GRID_CLASS)
+            HIPCHK(launch_grid_values(P->g.npatch * (P->g.most / 64), P->mode, P->rows, P->moff, P->smax, op->rp,
+                                      op->ci, P->g.line, P->g.W, v, (size_t)op->nnz, w, mv, P->sdel, st));
+        HIPCHK(hipStreamSynchronize(st));
+        P->vals[k] = true;
+    }
+    *out = P;
+    return SFG_OK;
+}
+
 // ---------------------------------------------------------------------------
 // media
 
@@ -372,6 +705,76 @@ extern "C" void sfg_medium_destroy(sfg_medium *md)
     delete md;
 }
 
+// ---- launch shape left to the library (shots_per_lane_group, kernel_variant,
+// row_order and a block other than 256 not given) ------------------------------
+
+// Whether a launch of `tiles` patches stages all fields of an M-PML patch at once:
+// one barrier less, against LDS for 24 instead of 12-14 values per halo node and, in
+// FP64, 202 instead of 174 VGPRs.  It pays while the launch has few blocks per CU.
+// us per step, at once / in two parts: Q4 100 x 100 FP64 7.7 / 8.5, Q4 200 x 200 FP64
+// 9.2 / 9.8, Q9 300 x 300 FP32 24.8 / 27.2; T6 101 x 203 FP64 22.2 / 18.4, 37 shots Q9
+// 97 x 111 FP32 130 / 124.
+static bool grid_together(int prec, int reach, long long tiles)
+{
+    return prec != 0 ? tiles <= 2048 : tiles <= (reach > 1 ? 256 : 1024);
+}
+
+// Rows of a patch: small patches spread a small mesh over more CUs; large ones have
+// the smaller halo, and for quadratic elements whole waves of each kind of node.  us
+// per step with 64 / 128 / 256: Q4 100 x 100 FP64 7.7 / 8.3 / 9.4, Q4 200 x 200 FP64
+// 9.2 / 11.3 / 10.0, Q4 400 x 400 FP32 11.1 / 12.1 / 10.4; T6 101 x 203 FP64 - / 18.4 /
+// 19.9, Q9 300 x 300 FP32 - / 30.0 / 24.8.
+static int grid_rows(int nodes, int nshots, int reach)
+{
+    const long long rows = (long long)nodes * nshots;
+    return reach > 1 ? (rows <= 131072 ? 128 : 256) : (rows <= 65536 ? 64 : 256);
+}
+
+// Whether a descriptor that leaves the launch shape to the library may take the grid
+// layout.  FP64 does for any number of shots.  In the FP32 forms 64-shot lane groups
+// that are mostly full (at least three quarters) need fewer instructions for the same
+// bytes, except for long rows (Q9: 16 nonzeros on average).  us per step, grid / best
+// lane-group launch: Q4 300 x 300 FP64 8 shots 93 / 257, 64 shots 628 / 769; FP32 +
+// Kahan (bfloat16 terms) 8 shots 28 / 85, 24 shots 98 / 170, 64 shots 251 / 233, 128
+// shots 490 / 455; Q4 200 x 200 72 shots 153 / 202, 96 shots 200 / 203; Q9 120 x 120 24
+// shots 92 / 180, 128 shots 476 / 493; T6 120 x 120 128 shots 467 / 423; a medium per
+// shot, 128 shots: Q4 200 x 200 258 / 233, Q9 100 x 100 336 / 374.
+static bool grid_default(const sfg_operator *op, const sfg_shot_desc *d)
+{
+    if (d->shots_per_lane_group != 0 || d->kernel_variant != 0 || d->row_order ||
+        (d->block != 0 && d->block != GRID_BLOCK))
+        return false;
+    const int groups = (d->nshots + 63) / 64;
+    return d->precision == 0 || 4 * d->nshots <= 3 * 64 * groups || op->nnz > 14LL * op->n;
+}
+
+// The layout the library takes for `nshots` shots (null: none).  With several shots
+// lines and patches start on 128-byte boundaries (64 with small patches): the state
+// then streams through HBM, and a line written in two parts costs its read back
+// (128 shots Q4 400 x 400 FP32 844 -> 804 us per step, 37 shots Q9 97 x 111 132 -> 124).
+static int choose_grid(const sfg_operator *op, int nshots, bool f32, hipStream_t st, const GridPlan **out)
+{
+    int rc = SFG_OK;
+    auto get = [&](int most) {
+        rc = grid_plan(op, most, nshots > 1 ? (most == 256 && f32 ? 32 : 16) : 0, f32, st, out);
+        return rc == SFG_OK && *out;
+    };
+    *out = nullptr;
+    int reach;
+    {
+        std::lock_guard<std::mutex> lk(op->grid_mu);
+        if ((rc = find_lines(op, st))) return rc;
+        if (op->lines.line == 0) return SFG_OK;
+        reach = std::max(op->lines.hx, op->lines.hy);
+    }
+    if (!get(grid_rows(op->n, nshots, reach)) && rc == SFG_OK) (void)get(256);
+    // with all seven values per row the matrices are read again for every shot, which
+    // lane groups of many shots do not (T6 120 x 120 FP64, 64 shots: 922 us per step
+    // against 687; Q9 100 x 100 FP64, 24 shots: 331 / 481)
+    if (*out && (*out)->mode == GRID_ROWS && nshots > 32) *out = nullptr;
+    return rc;
+}
+
 // ---------------------------------------------------------------------------
 // runs
 
@@ -412,6 +815,16 @@ struct sfg_run {
     bool in_multi = false;      // stepped by an sfg_multi (shares its step counter)
     StepArgs<double> a64;
     StepArgs<float> a32;
+    // grid layout (default launch shape on meshes numbered line by line): the
+    // per-step launches take launch_grid_step with these; a64 / a32 keep a
+    // per-row form that steps a single-shot run's state alike (persistent schedule)
+    const GridPlan *plan = nullptr;
+    int np = 0;                 // padded nodes per field
+    unsigned char *info = nullptr;
+    int *bkind = nullptr;
+    size_t grid_lds = 0;
+    GridArgs<double> g64;
+    GridArgs<float> g32;
 };
 
 static void run_free(sfg_run *r)
@@ -449,8 +862,13 @@ static void run_free(sfg_run *r)
     dfree(r->energy);
     dfree(r->coefp);
     dfree(r->flagp);
+    dfree(r->info);
+    dfree(r->bkind);
     delete r;
 }
+
+// nodes x shots of one field of the state, padding included
+static size_t field_stride(const sfg_run *r) { return (size_t)(r->np ? r->np : r->op->n) * r->S; }
 
 extern "C" void sfg_run_destroy(sfg_run *r)
 {
@@ -463,6 +881,11 @@ extern "C" void sfg_run_destroy(sfg_run *r)
 static int launch_one_step(sfg_run *r, int slot)
 {
     const void *args = (r->prec == 0) ? (const void *)&r->a64 : (const void *)&r->a32;
+    if (r->plan) {
+        const void *g = (r->prec == 0) ? (const void *)&r->g64 : (const void *)&r->g32;
+        HIPCHK(launch_grid_step(r->prec, r->cps, args, g, r->S, slot, r->grid_lds, r->stream));
+        return SFG_OK;
+    }
     HIPCHK(launch_step(r->prec, r->SP, r->cps, args, r->nbx, r->nby, r->block, slot, r->lds_bytes, r->stream));
     return SFG_OK;
 }
@@ -471,11 +894,14 @@ static int launch_one_step(sfg_run *r, int slot)
 static StateLayout state_layout(const sfg_run *r)
 {
     StateLayout L;
+    L.np = r->np;
+    L.line = r->plan ? r->plan->g.line : 1;
+    L.pitch = r->plan ? r->plan->g.pitch : 1;
     L.gs = node_major(r->SP) ? (r->SP >= 64 ? 64 : r->SP) : 0;
     L.ng = L.gs ? r->S / L.gs : 0;
     L.nf = NFIELD;
     L.S = r->S;
-    L.F = (size_t)r->op->n * r->S;
+    L.F = field_stride(r);
     return L;
 }
 
@@ -563,8 +989,27 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     r->rec_num = d->rec_num;
     r->guard_every = d->guard_every > 0 ? d->guard_every : 50;
     r->use_graph = d->use_graph != 0;
+    hipError_t es = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
+    if (es != hipSuccess) {
+        run_free(r);
+        return fail(SFG_E_HIP, "run setup: %s", hipGetErrorString(es));
+    }
     // lane grouping: shots per lane group and the padded shot stride
     int sp = d->shots_per_lane_group;
+    if (n < 1 << 28 && grid_default(op, d)) {
+        int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan);
+        if (rc) {
+            run_free(r);
+            return rc;
+        }
+        // (padded lines may exceed the index range where lane groups do not)
+        if (r->plan && (size_t)r->plan->g.pitch * r->plan->g.lines * d->nshots >= (size_t)1 << 31) r->plan = nullptr;
+    }
+    const int variant = d->kernel_variant, xcd = d->xcd_remap;
+    if (r->plan) {
+        sp = 1;
+        r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
+    }
     if (sp == 0) sp = d->nshots <= 1 ? 1 : d->nshots <= 4 ? 4 : d->nshots <= 16 ? 16 : 64;
     if (sp != 1 && sp != 4 && sp != 16 && sp != 32 && sp != 64) {
         run_free(r);
@@ -575,7 +1020,7 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     r->SP = sp;
     r->S = sp * ((d->nshots + sp - 1) / sp);
     r->nby = r->S / sp;
-    if ((size_t)n * r->S >= (size_t)1 << 31) {
+    if (field_stride(r) >= (size_t)1 << 31) {
         run_free(r);
         return fail(SFG_E_ARG, "run: node_num * padded shots must stay below 2^31");
     }
@@ -667,14 +1112,14 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         }
     }
 
-    const size_t F = (size_t)n * r->S;
+    const size_t F = field_stride(r);
     const size_t w = r->prec == 0 ? 8 : 4;
     const size_t seis_n = (size_t)r->S * d->max_steps * std::max(d->rec_num, 1);
 
     // LDS-staged gathers: the halo (distinct columns) of each block of rows
     std::vector<int> hptr, hnode, kslot, rslot;
     int lds_stride = 0;
-    if (d->kernel_variant == 7) {
+    if (variant == 7) {
         if (!node_major(sp)) {
             run_free(r);
             return fail(SFG_E_ARG, "run: kernel_variant 7 (LDS-staged gathers) needs 16, 32 or 64 shots per lane group");
@@ -729,15 +1174,15 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     // windows lie inside blocks (default: one window per block), and the slots
     // hold the columns' positions in the block's sorted halo list.
     std::vector<int> srow, soff, sci, ssrc, sown;
-    if (d->kernel_variant == 8 || d->kernel_variant == 9) {
-        const bool staged = d->kernel_variant == 9;
+    if (variant == 8 || variant == 9) {
+        const bool staged = variant == 9;
         const int R = r->block;                                  // rows per block (one per lane)
         const int win = d->sell_sigma > 0 ? d->sell_sigma : 64;
         if (sp != 1 || win % 64 || (staged && R % win)) {
             run_free(r);
             return fail(SFG_E_ARG, "run: kernel_variant %d (sliced layout) needs one shot per lane group and a "
                         "sorting window of a multiple of 64 rows%s (got %d shots per group, window %d)",
-                        d->kernel_variant, staged ? " dividing the block" : "", sp, win);
+                        variant, staged ? " dividing the block" : "", sp, win);
         }
         const size_t nslices = (size_t)r->nbx * (R / 64);
         std::vector<int> logical(n);
@@ -842,7 +1287,8 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     hipError_t e = hipSuccess;
     if ((rc = dalloc((char **)&r->state, 2 * NFIELD * F * w)) ||
         (r->prec >= 2 && (rc = dalloc((char **)&r->comp, 2 * comp_fields(r->prec) * F * w))) ||
-        (r->prec != 0 && ((rc = dalloc((char **)&r->uw, 2 * 2 * F * w)) || (rc = dalloc(&r->pml, n)))) ||
+        ((r->prec != 0 || r->plan) && ((rc = dalloc((char **)&r->uw, 2 * 2 * F * w)) || (rc = dalloc(&r->pml, n)))) ||
+        (r->plan && ((rc = dalloc(&r->info, (size_t)r->plan->g.npatch * r->plan->g.most)) || (rc = dalloc(&r->bkind, r->plan->g.npatch)))) ||
         (rc = dalloc(&r->ctrl, 1)) ||
         (rc = dalloc(&r->active, d->max_steps)) || (rc = dalloc(&r->shot_steps, r->S)) ||
         (rc = dalloc(&r->src, n + 1)) ||
@@ -856,8 +1302,7 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         run_free(r);
         return rc;
     }
-    e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreate(&r->ev0);
+    e = hipEventCreate(&r->ev0);
     if (e == hipSuccess) e = hipEventCreate(&r->ev1);
     if (e == hipSuccess) e = launch_fill_zero(r->state, 2 * NFIELD * F * w, r->stream);
     if (e == hipSuccess && r->comp) e = launch_fill_zero(r->comp, 2 * comp_fields(r->prec) * F * w, r->stream);
@@ -930,20 +1375,36 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
             csrc[s] = r->prec == 0 ? (const void *)m->coef64 : (const void *)m->coef32;
             fsrc[s] = m->flag;
         }
-        const void **dsrc = nullptr;
-        if ((rc = dalloc((char **)&r->coefp, (size_t)NCOEF * F * w)) || (rc = dalloc(&r->flagp, F)) ||
-            (rc = dalloc((char **)&dsrc, sizeof(void *) * 2 * d->nshots))) {
+        if (r->plan) {
+            // shot-major, each shot's arrays as its medium holds them
+            const size_t nc = (size_t)NCOEF * n;
+            if ((rc = dalloc((char **)&r->coefp, nc * r->S * w)) || (rc = dalloc(&r->flagp, (size_t)n * r->S))) {
+                run_free(r);
+                return rc;
+            }
+            for (int s = 0; s < d->nshots && e == hipSuccess; ++s) {
+                e = hipMemcpyAsync((char *)r->coefp + s * nc * w, csrc[s], nc * w, hipMemcpyDeviceToDevice, r->stream);
+                if (e == hipSuccess)
+                    e = hipMemcpyAsync(r->flagp + (size_t)s * n, fsrc[s], sizeof(int) * (size_t)n,
+                                       hipMemcpyDeviceToDevice, r->stream);
+            }
+            if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+        } else {
+            const void **dsrc = nullptr;
+            if ((rc = dalloc((char **)&r->coefp, (size_t)NCOEF * F * w)) || (rc = dalloc(&r->flagp, F)) ||
+                (rc = dalloc((char **)&dsrc, sizeof(void *) * 2 * d->nshots))) {
+                dfree(dsrc);
+                run_free(r);
+                return rc;
+            }
+            e = hipMemcpy(dsrc, csrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
+            if (e == hipSuccess)
+                e = hipMemcpy(dsrc + d->nshots, fsrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
+            if (e == hipSuccess) e = launch_pack_per_shot(dsrc, d->nshots, NCOEF, n, r->S, (int)w, r->coefp, r->stream);
+            if (e == hipSuccess) e = launch_pack_per_shot(dsrc + d->nshots, d->nshots, 1, n, r->S, 4, r->flagp, r->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
             dfree(dsrc);
-            run_free(r);
-            return rc;
         }
-        e = hipMemcpy(dsrc, csrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
-        if (e == hipSuccess)
-            e = hipMemcpy(dsrc + d->nshots, fsrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
-        if (e == hipSuccess) e = launch_pack_per_shot(dsrc, d->nshots, NCOEF, n, r->S, (int)w, r->coefp, r->stream);
-        if (e == hipSuccess) e = launch_pack_per_shot(dsrc + d->nshots, d->nshots, 1, n, r->S, 4, r->flagp, r->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-        dfree(dsrc);
         if (e != hipSuccess) {
             run_free(r);
             return fail(SFG_E_HIP, "run setup (per-shot media): %s", hipGetErrorString(e));
@@ -952,8 +1413,17 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
 
     if (r->pml) {
         // rows outside every damping layer (for all shots) take the short gather
-        e = launch_pml_rows(r->prec, r->cps ? r->coefp : (const void *)md->coef32, n, r->cps ? r->S : 1, op->rp,
-                            op->ci, r->pml, r->stream);
+        const void *coef = r->cps ? r->coefp : r->prec == 0 ? (const void *)md->coef64 : (const void *)md->coef32;
+        // [coef][node], per-shot media [coef][node][shot] or (grid layout) [shot][coef][node]
+        if (!r->cps)
+            e = launch_pml_rows(r->prec, coef, n, 1, n, 1, 0, op->rp, op->ci, r->pml, r->stream);
+        else if (r->plan)
+            e = launch_pml_rows(r->prec, coef, n, r->S, n, 1, (size_t)NCOEF * n, op->rp, op->ci, r->pml, r->stream);
+        else
+            e = launch_pml_rows(r->prec, coef, n, r->S, (size_t)n * r->S, r->S, 1, op->rp, op->ci, r->pml, r->stream);
+        if (e == hipSuccess && r->plan)
+            e = launch_grid_info(r->plan->g, r->plan->rows, r->pml, r->src, r->rec_ptr,
+                                 r->cps ? nullptr : md->flag, r->info, r->bkind, r->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
         if (e != hipSuccess) {
             run_free(r);
@@ -968,8 +1438,8 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         a.S = r->S;
         a.rows_per_block = rows_per_block;
         a.nsteps_max = d->max_steps;
-        a.xcd_remap = d->xcd_remap == 0 ? 1 : 0;
-        a.xcd_stripe = d->xcd_remap > 0 ? d->xcd_remap : 0;
+        a.xcd_remap = xcd == 0 ? 1 : 0;
+        a.xcd_stripe = xcd > 0 ? xcd : 0;
         a.sp = r->SP;
         a.cps = r->cps ? 1 : 0;
         a.nbx = r->nbx;
@@ -988,7 +1458,7 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         for (int m = 0; m < 7; ++m) a.A[m] = vals + (size_t)m * op->nnz;
         // descriptor variant -> kernel variant (see step_tile)
         static const int kv[10] = {1, 1, 0, 2, 3, 4, 5, 6, 7, 8};
-        a.variant = kv[d->kernel_variant];
+        a.variant = kv[variant];
         a.coef = r->cps ? (decltype(coef))r->coefp : coef;
         a.flag = r->cps ? r->flagp : md->flag;
         a.state = state;
@@ -998,7 +1468,8 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         // the LDS-staged walk reads every neighbour's split fields, so it keeps them on all
         // rows; one row per lane (lane groups of 1 or 4 shots) mixes row kinds in a wave
         // and measured slower with summed rows
-        a.agg = (r->prec != 0 && d->kernel_variant != 7 && node_major(r->SP)) ? 1 : 0;
+        // (the grid layout's patches are mostly of one kind, so its runs do)
+        a.agg = (r->prec != 0 && variant != 7 && (node_major(r->SP) || r->plan)) ? 1 : 0;
         a.fstride = F;
         a.active = r->active;
         a.src_ptr = r->src;
@@ -1025,6 +1496,37 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     else
         fill(r->a32, (float *)r->state, (float *)r->comp, op->v32, md->coef32, [](double v) { return (float)v; }),
             r->a32.Ap = op->p32, r->a32.sell_val = (const float *)r->sell_val;
+
+    if (const GridPlan *P = r->plan) {
+        auto fill_grid = [&](auto &g, int k, auto *tab, auto *mval) {
+            g.g = P->g;
+            g.mode = P->mode;
+            g.toff = P->toff;
+            g.tlen = P->tlen;
+            g.np = r->np;
+            g.magic = P->magic;
+            g.steps0 = r->steps_int[0];
+            g.rows = P->rows;
+            g.cls = P->cls;
+            g.slice = P->slice;
+            g.moff = P->moff;
+            g.sdel = P->sdel;
+            g.info = r->info;
+            g.bkind = r->bkind;
+            g.tab = (decltype(tab))P->tab[k];
+            g.mval = (decltype(mval))P->mval[k];
+        };
+        if (r->prec == 0) fill_grid(r->g64, 0, (const double *)nullptr, (const double *)nullptr);
+        else fill_grid(r->g32, 1, (const float *)nullptr, (const float *)nullptr);
+        const bool tog = grid_together(r->prec, std::max(P->g.hx, P->g.hy), (long long)P->g.npatch * r->S);
+        r->g64.together = r->g32.together = tog;
+        r->grid_lds = grid_lds_bytes(P->g, tog, w);
+        if (r->grid_lds > 65536) e = allow_grid_lds();
+        if (e != hipSuccess) {
+            run_free(r);
+            return fail(SFG_E_HIP, "run: LDS size %zu: %s", r->grid_lds, hipGetErrorString(e));
+        }
+    }
 
     // captured graphs of guard_every steps followed by the energy guard: one
     // per parity of the first step (a second one only when guard_every is odd)
@@ -1117,7 +1619,7 @@ extern "C" int sfg_run_reset(sfg_run *r)
     g_err.clear();
     if (!r) return fail(SFG_E_ARG, "reset: null run");
     if (r->in_multi) return fail(SFG_E_ARG, "reset: this run is stepped by a multi-run");
-    const size_t F = (size_t)r->op->n * r->S;
+    const size_t F = field_stride(r);
     const size_t w = r->prec == 0 ? 8 : 4;
     const size_t seis_n = (size_t)r->S * r->max_steps * std::max(r->rec_num, 1);
     // the same zero fills as at creation (elastic_wave.c:466-502), on the run's stream
@@ -1319,7 +1821,8 @@ struct MultiGroup {
     std::vector<sfg_run *> runs;
     int ntiles = 0;
     int xcd_remap = 1;          // the group's tile map: 0 round-robin, 1 contiguous, Q + 1 stripes of Q
-    size_t lds_bytes = 0;       // dynamic LDS of the launch (LDS-staged group)
+    size_t lds_bytes = 0;       // dynamic LDS of the launch (LDS-staged and grid groups)
+    bool together = false;      // grid group: GridArgs::together
     void *args = nullptr;       // device StepArgs<T>[runs]
     int *tile_start = nullptr;  // device [runs + 1]
 };
@@ -1332,17 +1835,20 @@ struct sfg_multi {
     // chip on its own takes its own step launch (the single-run kernel, with its
     // compaction of finished shot groups), reading the shared counter; then one
     // launch of the smaller batched runs (grp[0]), one of the single-shot runs in
-    // the per-row or sliced layouts (grp[1], a kernel with only those forms) and
-    // one of the single-shot runs with LDS-staged halos (grp[2]), each only when
-    // it has runs.
+    // the per-row or sliced layouts (grp[1], a kernel with only those forms), one
+    // of the single-shot runs with LDS-staged halos (grp[2]) and one of the runs in
+    // the grid layout with each patch size (grid[]), each only when it has runs.
     std::vector<sfg_run *> solo;
     std::vector<StepArgs<double>> solo64;   // their arguments with the shared counter
     std::vector<StepArgs<float>> solo32;
     MultiGroup grp[3];
+    MultiGroup grid[3];         // grid layout, by patch size: 64, 128, 256 rows
+    MultiGroup mixed;           // persistent schedule of grp[1] and grid[] together, in their per-row forms
     // persistent schedule (sfg_multi_set_persistent): resident blocks of one
     // cooperative launch per guard interval, or 0 for the per-step launches
     int persist_blocks = 0;
-    int persist_group = -1;
+    const MultiGroup *persist = nullptr;
+    bool persist_single = false; // only single-shot runs
     int *queue = nullptr;       // device int[16]: tile queues by step parity and XCD
     hipStream_t stream = nullptr;
     hipGraphExec_t graph[2] = {nullptr, nullptr}; // by parity of the first step
@@ -1360,9 +1866,9 @@ static void multi_free(sfg_multi *m)
     if (m->stream) (void)hipStreamDestroy(m->stream);
     dfree(m->ctrl);
     dfree(m->queue);
-    for (MultiGroup &g : m->grp) {
-        dfree(g.args);
-        dfree(g.tile_start);
+    for (MultiGroup *g : {&m->grp[0], &m->grp[1], &m->grp[2], &m->grid[0], &m->grid[1], &m->grid[2], &m->mixed}) {
+        dfree(g->args);
+        dfree(g->tile_start);
     }
     delete m;
 }
@@ -1384,6 +1890,10 @@ static int multi_launch_step(sfg_multi *m, int slot)
     if (!g2.runs.empty())
         HIPCHK(launch_multi_step_lds(m->prec, g2.args, g2.tile_start, (int)g2.runs.size(), g2.ntiles, m->block,
                                      g2.xcd_remap, slot, g2.lds_bytes, m->stream));
+    for (const MultiGroup &g : m->grid)
+        if (!g.runs.empty())
+            HIPCHK(launch_multi_grid(m->prec, g.args, g.tile_start, (int)g.runs.size(), g.ntiles, g.runs[0]->plan->g.most,
+                                     g.xcd_remap, slot, g.lds_bytes, g.together, m->stream));
     return SFG_OK;
 }
 
@@ -1394,6 +1904,56 @@ static int multi_launch_guards(sfg_multi *m)
         if (rc) return rc;
     }
     return SFG_OK;
+}
+
+// Argument table and tile starts of a group's runs: each run's own arguments
+// with the shared step counter (grid: GridRun entries, one tile per patch and
+// shot; else StepArgs, one per row block and shot group).
+template <class T>
+static int fill_group_t(sfg_multi *m, MultiGroup &g, bool grid)
+{
+    const int n = (int)g.runs.size();
+    std::vector<int> ts(n + 1, 0);
+    std::vector<StepArgs<T>> sa;
+    std::vector<GridRun<T>> ga;
+    for (int k = 0; k < n; ++k) {
+        const sfg_run *r = g.runs[k];
+        StepArgs<T> a;
+        if constexpr (sizeof(T) == 8) a = r->a64;
+        else a = r->a32;
+        a.ctrl = m->ctrl;
+        if (k == 0) g.xcd_remap = a.xcd_stripe > 0 ? a.xcd_stripe + 1 : a.xcd_remap; // the group's tile map
+        if (grid) {
+            GridRun<T> e;
+            e.a = a;
+            if constexpr (sizeof(T) == 8) e.g = r->g64;
+            else e.g = r->g32;
+            ga.push_back(e);
+        } else {
+            sa.push_back(a);
+        }
+        ts[k + 1] = ts[k] + (grid ? r->plan->g.npatch * r->S : r->nbx * r->nby);
+        if (!grid) g.lds_bytes = std::max(g.lds_bytes, r->lds_bytes);
+    }
+    g.ntiles = ts[n];
+    int reach = 1;
+    for (int k = 0; grid && k < n; ++k) reach = std::max({reach, g.runs[k]->plan->g.hx, g.runs[k]->plan->g.hy});
+    g.together = grid && grid_together(m->prec, reach, g.ntiles);
+    for (int k = 0; grid && k < n; ++k)
+        g.lds_bytes = std::max(g.lds_bytes, grid_lds_bytes(g.runs[k]->plan->g, g.together, sizeof(T)));
+    const size_t bytes = grid ? sizeof(GridRun<T>) * n : sizeof(StepArgs<T>) * n;
+    int rc;
+    if ((rc = dalloc((char **)&g.args, bytes)) || (rc = dalloc(&g.tile_start, n + 1))) return rc;
+    HIPCHK(hipMemcpyAsync(g.args, grid ? (const void *)ga.data() : (const void *)sa.data(), bytes, hipMemcpyHostToDevice,
+                          m->stream));
+    HIPCHK(hipMemcpyAsync(g.tile_start, ts.data(), sizeof(int) * ts.size(), hipMemcpyHostToDevice, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+    return SFG_OK;
+}
+
+static int fill_group(sfg_multi *m, MultiGroup &g, bool grid)
+{
+    return m->prec == 0 ? fill_group_t<double>(m, g, grid) : fill_group_t<float>(m, g, grid);
 }
 
 extern "C" int sfg_multi_create(sfg_multi **out, sfg_run *const *runs, int nruns)
@@ -1420,7 +1980,8 @@ extern "C" int sfg_multi_create(sfg_multi **out, sfg_run *const *runs, int nruns
     for (int k = 0; k < nruns; ++k) {
         sfg_run *r = runs[k];
         m->runs.push_back(r);
-        if (r->SP == 1) m->grp[staged(r) ? 2 : 1].runs.push_back(r);
+        if (r->plan) m->grid[r->plan->g.most / 128].runs.push_back(r);
+        else if (r->SP == 1) m->grp[staged(r) ? 2 : 1].runs.push_back(r);
         else if ((r->SP == 32 || r->SP == 64) && r->nbx * r->nby < 256 && r->lds_bytes == 0) m->grp[0].runs.push_back(r);
         else m->solo.push_back(r);
     }
@@ -1438,59 +1999,21 @@ extern "C" int sfg_multi_create(sfg_multi **out, sfg_run *const *runs, int nruns
             m->solo32.back().ctrl = m->ctrl;
         }
     }
-    const size_t asz = m->prec == 0 ? sizeof(StepArgs<double>) : sizeof(StepArgs<float>);
-    std::vector<std::vector<char>> tabs(3);
-    std::vector<std::vector<int>> tss(3);
-    for (int gi = 0; gi < 3; ++gi) {
-        MultiGroup &g = m->grp[gi];
-        const int n = (int)g.runs.size();
-        if (n == 0) continue;
-        {
-            // the group's first run sets its tile map
-            const sfg_run *f = g.runs[0];
-            const int remap = f->prec == 0 ? f->a64.xcd_remap : f->a32.xcd_remap;
-            const int stripe = f->prec == 0 ? f->a64.xcd_stripe : f->a32.xcd_stripe;
-            g.xcd_remap = stripe > 0 ? stripe + 1 : remap;
-        }
-        std::vector<int> &ts = tss[gi];
-        ts.assign(n + 1, 0);
-        for (int k = 0; k < n; ++k) {
-            ts[k + 1] = ts[k] + g.runs[k]->nbx * g.runs[k]->nby;
-            g.lds_bytes = std::max(g.lds_bytes, g.runs[k]->lds_bytes);
-        }
-        g.ntiles = ts[n];
-        if ((rc = dalloc((char **)&g.args, asz * n)) || (rc = dalloc(&g.tile_start, n + 1))) {
-            multi_free(m);
-            return rc;
-        }
-        // argument table: each run's own arguments with the shared step counter
-        std::vector<char> &tab = tabs[gi];
-        tab.resize(asz * n);
-        for (int k = 0; k < n; ++k) {
-            if (m->prec == 0) {
-                StepArgs<double> a = g.runs[k]->a64;
-                a.ctrl = m->ctrl;
-                std::memcpy(tab.data() + asz * k, &a, asz);
-            } else {
-                StepArgs<float> a = g.runs[k]->a32;
-                a.ctrl = m->ctrl;
-                std::memcpy(tab.data() + asz * k, &a, asz);
-            }
-        }
-    }
     hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
+    for (int gi = 0; gi < 3 && e == hipSuccess && rc == SFG_OK; ++gi) {
+        if (!m->grp[gi].runs.empty()) rc = fill_group(m, m->grp[gi], false);
+        if (rc == SFG_OK && !m->grid[gi].runs.empty()) rc = fill_group(m, m->grid[gi], true);
+    }
+    if (rc != SFG_OK) {
+        multi_free(m);
+        return rc;
+    }
+    for (const MultiGroup &g : m->grid)
+        if (e == hipSuccess && g.lds_bytes > 65536) e = allow_grid_lds();
     if (e == hipSuccess && !m->grp[2].runs.empty()) e = allow_multi_step_lds(m->prec, m->grp[2].lds_bytes);
     if (e == hipSuccess) e = hipEventCreate(&m->ev0);
     if (e == hipSuccess) e = hipEventCreate(&m->ev1);
     if (e == hipSuccess) e = launch_fill_zero(m->ctrl, sizeof(Ctrl), m->stream);
-    for (int gi = 0; gi < 3; ++gi) {
-        if (m->grp[gi].runs.empty()) continue;
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(m->grp[gi].args, tabs[gi].data(), tabs[gi].size(), hipMemcpyHostToDevice, m->stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(m->grp[gi].tile_start, tss[gi].data(), sizeof(int) * tss[gi].size(),
-                               hipMemcpyHostToDevice, m->stream);
-    }
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     if (e != hipSuccess) {
         multi_free(m);
@@ -1521,10 +2044,10 @@ extern "C" int sfg_multi_advance(sfg_multi *m, int nsteps)
     HIPCHK(hipEventRecord(m->ev0, m->stream));
     while (todo > 0 && m->persist_blocks > 0) {
         // one cooperative launch up to the next guard
-        const MultiGroup &g = m->grp[m->persist_group];
+        const MultiGroup &g = *m->persist;
         const int seg = std::min(todo, m->guard_every - m->executed % m->guard_every);
         HIPCHK(launch_multi_persistent(m->prec, g.args, g.tile_start, (int)g.runs.size(), g.ntiles, m->block,
-                                       m->persist_blocks, m->executed & 1, seg, m->queue, m->persist_group == 1,
+                                       m->persist_blocks, m->executed & 1, seg, m->queue, m->persist_single,
                                        m->stream));
         m->executed += seg;
         todo -= seg;
@@ -1571,17 +2094,25 @@ extern "C" int sfg_multi_set_persistent(sfg_multi *m, int blocks_per_cu)
         m->persist_blocks = 0;
         return SFG_OK;
     }
-    int gi = -1, groups = 0;
-    for (int k = 0; k < 3; ++k)
-        if (!m->grp[k].runs.empty()) {
-            gi = k;
-            ++groups;
+    // the runs of one shared launch: batched runs only, or single-shot runs in the
+    // per-row, sliced and grid layouts (the last in their per-row form)
+    const MultiGroup *g = nullptr;
+    bool ok = m->solo.empty() && m->grp[2].runs.empty();
+    bool grid = false;
+    for (const MultiGroup &q : m->grid)
+        for (const sfg_run *r : q.runs) {
+            grid = true;
+            ok = ok && r->S == 1;
         }
-    if (!m->solo.empty() || groups != 1 || gi == 2)
+    if (ok && m->grp[1].runs.empty() && !grid) g = &m->grp[0];
+    else if (ok && m->grp[0].runs.empty()) g = grid ? &m->mixed : &m->grp[1];
+    else ok = false;
+    if (!ok)
         return fail(SFG_E_ARG, "multi persistent: needs every run in one shared launch (single-shot runs in the "
-                               "per-row or sliced layouts, or batched runs too small to fill the GPU alone)");
+                               "per-row, sliced or grid layouts, or batched runs too small to fill the GPU alone)");
+    const bool single = g != &m->grp[0];
     int per_cu = 0, dev = 0, cus = 0;
-    HIPCHK(multi_persistent_blocks_per_cu(m->prec, gi == 1, m->block, &per_cu));
+    HIPCHK(multi_persistent_blocks_per_cu(m->prec, single, m->block, &per_cu));
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     if (blocks_per_cu > per_cu)
@@ -1592,7 +2123,18 @@ extern "C" int sfg_multi_set_persistent(sfg_multi *m, int blocks_per_cu)
         HIPCHK(launch_fill_zero(m->queue, 16 * sizeof(int), m->stream));
         HIPCHK(hipStreamSynchronize(m->stream));
     }
-    m->persist_group = gi;
+    if (g == &m->mixed && !m->mixed.args) {
+        for (sfg_run *r : m->runs) m->mixed.runs.push_back(r);
+        int rc = fill_group(m, m->mixed, false);
+        if (rc) {
+            m->mixed.runs.clear();
+            dfree(m->mixed.args);
+            dfree(m->mixed.tile_start);
+            return rc;
+        }
+    }
+    m->persist = g;
+    m->persist_single = single;
     m->persist_blocks = blocks_per_cu * cus;
     return SFG_OK;
 }

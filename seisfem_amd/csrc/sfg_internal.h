@@ -59,7 +59,11 @@ __device__ __forceinline__ int executed_steps(const Ctrl *c)
 // group], for groups of 16, 32 or 64 shots, so that a wave's gather of one
 // neighbour reads all that node's fields from one contiguous block instead of
 // one short piece from each of 20 arrays tens of MB apart.
+// Grid-layout runs (GridArgs) are shot-major, [shot][field][padded node]: each
+// shot's fields are those of a single-shot run.
 struct StateLayout {
+    int np;         // > 0: shot-major with this padded node count,
+    int line, pitch; // lines of `line` nodes `pitch` nodes apart
     int gs;         // shots per group when node-major, 0 = field-major
     int ng;         // shot groups (node-major)
     int nf;         // fields per node in this array (26 state, 6 Kahan terms)
@@ -69,6 +73,7 @@ struct StateLayout {
 
 __host__ __device__ inline size_t state_index(const StateLayout &L, int i, int f, int s)
 {
+    if (L.np) return ((size_t)s * L.nf + f) * L.np + (L.pitch == L.line ? i : i / L.line * L.pitch + i % L.line);
     if (L.gs) return (((size_t)i * L.ng + s / L.gs) * L.nf + f) * L.gs + s % L.gs;
     return (size_t)f * L.F + (size_t)i * L.S + s;
 }
@@ -122,6 +127,7 @@ struct StepArgs {
     // profiles of row i is nonzero for some shot, 1 when row i is a column of
     // such a row, else 0.  Rows below 2 gather only U, W and the 8 memory
     // fields of their neighbours; rows at 0 keep no velocity (null in exact mode).
+    // (FP64 runs in the grid layout keep uw and pml too.)
     T *uw;
     const int *pml;
     // 1: rows of kind 0 (their split fields are gathered by no M-PML row) keep
@@ -143,6 +149,103 @@ struct StepArgs {
     double *seis_u, *seis_w; // [S][nsteps_max][rec_num]
     Ctrl *ctrl;
 };
+
+// ---- grid layout --------------------------------------------------------------
+// Operators of meshes numbered line by line (every column within GRID_REACH
+// nodes and lines of its row) are stepped in patches of pw nodes x ph lines,
+// one patch of one shot per block, one row per thread.  Rows are grouped by class:
+// rows whose stencils (relative columns and values) are identical bit for bit.  A
+// patch's rows are sorted by class, so that most waves hold one class, and the
+// stencils of its classes (few on a uniform mesh) are its table, which patches with
+// the same classes share: the matrices are then hardly read at all.
+//   GRID_CLASS    M, S1..S6 from the class table
+//   GRID_CLASS_S  S1..S6 from the class table, M per row (a density that varies
+//                 from row to row)
+//   GRID_ROWS     all seven per row (S too varies: distorted meshes); the rows of
+//                 a patch are then sorted by length
+enum GridMode : int { GRID_CLASS = 0, GRID_CLASS_S = 1, GRID_ROWS = 2 };
+constexpr int GRID_REACH = 2;
+constexpr int GRID_BLOCK = 256;         // most rows of a patch
+constexpr int GRID_HALO_MAX = 2 * GRID_BLOCK;  // most halo nodes of a patch (two per thread)
+constexpr int GRID_TABLE = 384;         // most table entries of a patch
+// bits of GridArgs::info
+enum GridInfo : int { GI_KIND = 3, GI_SRC = 4, GI_REC = 8, GI_CLAMP = 16 };
+
+struct GridShape {
+    int line = 0, lines = 0;    // nodes per line, lines
+    int pitch = 0;              // nodes from one line to the next in the state (>= line)
+    int hx = 0, hy = 0;         // reach of the columns
+    int most = 0;               // places for rows in a patch: 64, 128 or 256
+    int pw = 0, ph = 0, px = 0, npatch = 0;
+    int W = 0, halo = 0;        // halo width and nodes
+    int table = 0;              // most table entries of a patch
+};
+
+template <class T>
+struct GridArgs {
+    GridShape g;
+    int mode;
+    int np;                     // padded nodes: field stride of a shot
+    int magic;                  // q / W == q * magic >> 16 for halo positions q
+    int together;               // 1: a patch stages all its fields at once (FP64; the FP32 forms always do)
+    int steps0;                 // executed steps of shot 0 (single-shot runs)
+    const int *rows;            // [npatch * most] row at each place, -1 = none
+    const int *cls;             // [npatch * most] first entry of the row's class in its patch's table | its
+                                // halo position << 12 | its nonzeros << 24
+    const int *slice;           // [npatch * most / 64] longest row of the wave, + 0x100 if all its rows are of one class
+    const int *toff, *tlen;     // [npatch] first entry of the patch's table in tab, its entries
+    const T *tab;               // [entry][8]: M, S1..S6, halo position of the column relative to the row's own
+    const int *moff;            // [npatch * most / 64] first slot of the wave's per-row values
+    const T *mval;              // slot k of lane l: GRID_CLASS_S mval[64 k + l] = M, GRID_ROWS mval[(7 k + m) 64 + l]
+    const int *sdel;            // GRID_ROWS: [64 k + l] halo position relative to the row's own
+    const unsigned char *info;  // [npatch * most] kind, source / receiver / clamp bits of the lane's row in this run
+    const int *bkind;           // [npatch] largest kind of the patch's rows
+};
+
+// Argument table entry of a multi-run's grid launch
+template <class T>
+struct GridRun {
+    StepArgs<T> a;
+    GridArgs<T> g;
+};
+
+hipError_t launch_grid_step(int precision, bool cps, const void *step_args, const void *grid_args, int nshots, int slot,
+                            size_t lds_bytes, hipStream_t st);
+// runs of one patch size `most`
+hipError_t launch_multi_grid(int precision, const void *runs_dev, const int *tile_start_dev, int nruns, int ntiles,
+                             int most, int xcd_remap, int slot, size_t lds_bytes, bool together, hipStream_t st);
+// LDS of a patch: its table, and per halo node part A and (together) part B, else
+// the larger of the two (see LDS_A, LDS_B)
+inline size_t grid_lds_bytes(const GridShape &g, bool together, size_t w)
+{
+    const size_t a = w == 4 ? 12 : 10, b = w == 4 ? 12 : 14;
+    return ((size_t)g.table * 8 + (size_t)g.halo * (together ? a + b : b)) * w;
+}
+hipError_t allow_grid_lds(); // lets the FP64 kernels take more than 64 KB
+// Plan building (one-off per operator; see GridPlan in sfg_api.hip)
+// *bad |= 1 when a column lies beyond GRID_REACH of its row under `line`; reach[0..1] = largest |dx|, |dy|
+hipError_t launch_grid_reach(int n, const int *rp, const int *ci, int line, int *reach, int *bad, hipStream_t st);
+// per row: hash of relative columns and S1..S6 (h[i]), and of M as well (h[n + i])
+hipError_t launch_grid_hash(int n, const int *rp, const int *ci, const double *v64, size_t nnz,
+                            unsigned long long *h, hipStream_t st);
+// *bad |= 1 when row i and the representative rep[cls[i]] differ in a relative column or a value (m0 .. 6)
+hipError_t launch_grid_check(int n, const int *rp, const int *ci, const double *v64, size_t nnz, int m0, const int *cls,
+                             const int *rep, int *bad, hipStream_t st);
+// sorts each patch's rows by class key[row] (first table entry cptr[key]; GRID_ROWS: descending length);
+// smax[w] = longest row of wave w
+hipError_t launch_grid_sort(const GridShape &g, int mode, const int *rp, const int *key, const int *cptr,
+                            int *rows, int *cls, int *slice, int *smax, hipStream_t st);
+// adds each place's halo position to its key
+hipError_t launch_grid_place(const GridShape &g, const int *rows, int *cls, hipStream_t st);
+// table items: the stencil of row rep[c] at entries dst[c] ..
+hipError_t launch_grid_table(int nitems, const int *rep, const int *dst, const int *rp, const int *ci, int line, int W,
+                             const void *vals, size_t nnz, int elem, void *tab, hipStream_t st);
+hipError_t launch_grid_values(int nwaves, int mode, const int *rows, const int *moff, const int *smax, const int *rp,
+                              const int *ci, int line, int W, const void *vals, size_t nnz, int elem, void *mval,
+                              int *sdel, hipStream_t st);
+// info and bkind of a run; flag may be null (per-shot flags)
+hipError_t launch_grid_info(const GridShape &g, const int *rows, const int *pml, const int *src_ptr,
+                            const int *rec_ptr, const int *flag, unsigned char *info, int *bkind, hipStream_t st);
 
 // Launchers (defined in sfg_kernels.hip).  precision: 0 exact FP64, 1 FP32, 2 FP32+Kahan,
 // 3 FP32+Kahan with the compensation terms stored as bfloat16.
@@ -190,10 +293,11 @@ hipError_t launch_fill_zero(void *p, size_t bytes, hipStream_t st);
 hipError_t launch_sell_values(const void *vals, size_t nnz, const int *src, size_t nslots, int elem, void *out,
                               hipStream_t st);
 // pml[i] = 2 when coefficient DX..DYYP of row i is nonzero for one of the ns
-// shots (coef is [NCOEF][n][ns]; ns = 1: one medium for every shot), 1 when
-// row i is a column of such a row in the pattern rp/ci, else 0
-hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, const int *rp, const int *ci, int *pml,
-                           hipStream_t st);
+// shots (coefficient c of row i and shot s at coef[c cs + i is + s ss]; ns = 1:
+// one medium for every shot), 1 when row i is a column of such a row in the
+// pattern rp/ci, else 0
+hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, size_t cs, size_t is, size_t ss,
+                           const int *rp, const int *ci, int *pml, hipStream_t st);
 // dst[c][i][s] = srcs[min(s, nsrc-1)][c*n + i] for c < ncoef, i < n, s < S; elem = 4 or 8 bytes
 hipError_t launch_pack_per_shot(const void *const *srcs_dev, int nsrc, int ncoef, int n, int S, int elem,
                                 void *dst, hipStream_t st);

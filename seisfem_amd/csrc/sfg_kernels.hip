@@ -23,56 +23,9 @@
 //   2  FP32 with a Kahan-compensated displacement update.
 #include <hip/hip_cooperative_groups.h>
 
-#include "sfg_internal.h"
+#include "sfg_device.h"
 
 namespace sfg {
-
-template <bool EXACT, class T>
-__device__ __forceinline__ T mac(T acc, T a, T x)
-{
-    if constexpr (EXACT) return acc + a * x;
-    else return __builtin_fmaf(a, x, acc);
-}
-
-// Loads and stores of data no other lane of this step touches again (a row's
-// own accelerations, the Kahan terms, every output) may carry the streaming
-// (nontemporal) hint, so the lines they occupy do not push the neighbours'
-// fields, which nine rows gather, out of L2.
-template <bool NT, class T>
-__device__ __forceinline__ T ld_once(const T *p)
-{
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-
-template <bool NT, class T>
-__device__ __forceinline__ void st_once(T *p, T v)
-{
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
-
-// bfloat16 halves of a 32-bit word (precision 3 keeps the Kahan terms of two
-// displacement fields per word): the low half is field 2k, the high half 2k+1.
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-// round to nearest even (the terms are finite: a Kahan term is the rounding
-// error of an FP32 sum)
-__device__ __forceinline__ uint32_t bf16_bits(float f)
-{
-    const uint32_t u = __float_as_uint(f);
-    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
-
-// Read-only arrays of a step (pattern, values, coefficients, schedules) are
-// read through the constant address space: they do not change during a
-// launch, which lets wave-uniform reads (one row per wave) go through the
-// scalar unit instead of the vector-memory path the gathers saturate.
-template <class T>
-__device__ __forceinline__ const __attribute__((address_space(4))) T *ro(const T *p)
-{
-    return (const __attribute__((address_space(4))) T *)p;
-}
 
 // 16-byte vector of T (staging copies into LDS)
 template <class T> struct vec16;
@@ -82,41 +35,6 @@ template <> struct vec16<double> { using type = double2; };
 // Position of state field f among the 20 gathered fields (U1..W3, U1t..W3t,
 // Lx1..Ly4; the accelerations are not gathered).
 __device__ __forceinline__ constexpr int gathered_slot(int f) { return f < U1TT ? f : f - 6; }
-
-// Workgroups are dispatched round-robin over the 8 XCDs; this map makes each
-// XCD walk one contiguous range of logical blocks (shot chunk, row block), so
-// neighbouring rows share that XCD's L2.  A bijection on [0, nb) for any nb.
-__device__ __forceinline__ unsigned int xcd_contiguous(unsigned int bid, unsigned int nb)
-{
-    const unsigned int q = nb / 8, r = nb % 8;
-    const unsigned int x = bid % 8, l = bid / 8;
-    return x * q + (x < r ? x : r) + l;
-}
-
-// Stripes: tiles are taken in runs of 8*Q; within a run XCD x (workgroup ids
-// x, x+8, ...) steps tiles x*Q .. x*Q+Q-1.  All XCDs then sweep the rows
-// together, each keeping one stripe of consecutive row blocks, so a row's
-// neighbours on the adjacent grid lines were fetched into the same XCD's L2.
-// A bijection on [0, nb): the ids past the last whole run map to themselves.
-__device__ __forceinline__ unsigned int xcd_striped(unsigned int bid, unsigned int nb, unsigned int q)
-{
-    const unsigned int span = 8u * q;
-    if (bid >= (nb / span) * span) return bid;
-    const unsigned int x = bid % 8, k = bid / 8;
-    return (k / q) * span + x * q + k % q;
-}
-
-// Step number of a launch with the given slot; the first thread of the grid
-// hands t + 1 to the next launch (the other slot).  One store per launch: a
-// per-block completion count on one address serialises tens of thousands of
-// atomics per step at one L2 channel.
-__device__ __forceinline__ int begin_step(Ctrl *ctrl, int slot)
-{
-    const int t = __hip_atomic_load(&ctrl->step[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0)
-        __hip_atomic_store(&ctrl->step[slot ^ 1], t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return t;
-}
 
 // One tile (logical block bx of rows, shot chunk by) of step t.
 // Variant V: 0 separate value arrays; 1 values packed per nonzero, gather loop
@@ -711,6 +629,13 @@ __device__ __forceinline__ void step_tile(const StepArgs<T> &a, int t, int bx, i
             const size_t ob = uw_base(row);
             st_once<NT>(uwout + ob, sum_u);
             st_once<NT>(uwout + ob + FS, sum_w);
+        } else if constexpr (SP == 1) {
+            // an FP64 run of the grid layout keeps U and W too (StepArgs::uw)
+            if (a.uw) {
+                T *uo = a.uw + (size_t)((t + 1) & 1) * 2 * F + uw_base(row);
+                uo[0] = sum_u;
+                uo[FS] = sum_w;
+            }
         }
 
         // ---- receivers sitting on this node --------------------------------
@@ -1092,7 +1017,8 @@ __global__ __launch_bounds__(256) void guard_kernel(const T *state, const T *uw,
     __shared__ double red_u[256], red_w[256];
     const int t = executed_steps(ctrl);
     const int S = L.S;
-    const int sg = S < 64 ? S : 64;                 // shots covered by one block
+    // shots covered by one block: shots innermost, or (shot-major) one
+    const int sg = L.np ? 1 : S < 64 ? S : 64;
     const int rstep = blockDim.x / sg;
     const int sl = threadIdx.x % sg, rl = threadIdx.x / sg;
     const int s = blockIdx.y * sg + sl;
@@ -1142,7 +1068,7 @@ hipError_t launch_guard(int precision, const void *state, const void *uw, int n,
                         hipStream_t st)
 {
     const int npb = 2048;
-    const int sg = L.S < 64 ? L.S : 64;
+    const int sg = L.np ? 1 : L.S < 64 ? L.S : 64;
     const dim3 g((n + npb - 1) / npb, (L.S + sg - 1) / sg);
     if (precision == 0)
         hipLaunchKernelGGL(guard_kernel<double>, g, dim3(256), 0, st, (const double *)state, (const double *)uw,
@@ -1310,13 +1236,12 @@ __global__ void fill_zero_kernel(uint32_t *p, size_t nwords)
 }
 
 template <class T>
-__global__ void pml_rows_kernel(const T *coef, int n, int ns, int *pml)
+__global__ void pml_rows_kernel(const T *coef, int n, int ns, size_t cs, size_t is, size_t ss, int *pml)
 {
-    const size_t cs = (size_t)n * ns;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         int any = 0;
         for (int c = DX; c <= DYYP; ++c)
-            for (int s = 0; s < ns; ++s) any |= coef[c * cs + (size_t)i * ns + s] != T(0);
+            for (int s = 0; s < ns; ++s) any |= coef[c * cs + i * is + s * ss] != T(0);
         pml[i] = any ? 2 : 0;
     }
 }
@@ -1334,15 +1259,17 @@ __global__ void pml_ring_kernel(int n, const int *rp, const int *ci, int *pml)
     }
 }
 
-hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, const int *rp, const int *ci, int *pml,
-                           hipStream_t st)
+hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, size_t cs, size_t is, size_t ss,
+                           const int *rp, const int *ci, int *pml, hipStream_t st)
 {
     const int blocks = (n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096;
     if (n <= 0) return hipSuccess;
     if (precision == 0)
-        hipLaunchKernelGGL(pml_rows_kernel<double>, dim3(blocks), dim3(256), 0, st, (const double *)coef, n, ns, pml);
+        hipLaunchKernelGGL(pml_rows_kernel<double>, dim3(blocks), dim3(256), 0, st, (const double *)coef, n, ns, cs,
+                           is, ss, pml);
     else
-        hipLaunchKernelGGL(pml_rows_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float *)coef, n, ns, pml);
+        hipLaunchKernelGGL(pml_rows_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float *)coef, n, ns, cs,
+                           is, ss, pml);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(pml_ring_kernel, dim3(blocks), dim3(256), 0, st, n, rp, ci, pml);
