@@ -748,6 +748,25 @@ static bool grid_default(const sfg_operator *op, const sfg_shot_desc *d)
     return d->precision == 0 || 4 * d->nshots <= 3 * 64 * groups || op->nnz > 14LL * op->n;
 }
 
+// Variant and XCD map of 64-shot lane groups whose launch shape is left to the
+// library, on meshes numbered line by line: XCD stripes of an eighth of a line (a
+// row's neighbours on the adjacent lines then come from the same L2); streaming
+// hints on large meshes of few nonzeros a row, three nonzeros in flight elsewhere.  us
+// per step, FP32 + Kahan (bfloat16 terms): variant 1 in contiguous ranges 855, 3 in
+// stripes 759, 5 in stripes 812 (128 shots Q4 400 x 400); 3 / 5 in stripes 455 / 487
+// (Q4 300 x 300), 92 / 88 (Q4 100 x 120), 499 / 493 (Q9 120 x 120), 426 / 423 (T6 120 x
+// 120), and 246 / 233 with a medium per shot (Q4 200 x 200).
+static void batched_default(const sfg_operator *op, const sfg_shot_desc *d, bool media, int *variant, int *xcd)
+{
+    if (d->shots_per_lane_group != 0 || d->kernel_variant != 0 || d->xcd_remap != 0 || d->row_order || d->nshots <= 16 ||
+        (d->block != 0 && d->block != 256))
+        return;
+    const std::vector<int> line = line_candidates(op);
+    if (line.empty()) return;
+    *variant = (media || op->nnz > 10LL * op->n || op->n < 65536) ? 5 : 3;
+    *xcd = std::max(1, (line[0] + 16) / 32);     // 4 rows a block, 8 XCDs
+}
+
 // The layout the library takes for `nshots` shots (null: none).  With several shots
 // lines and patches start on 128-byte boundaries (64 with small patches): the state
 // then streams through HBM, and a line written in two parts costs its read back
@@ -1005,7 +1024,8 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
         // (padded lines may exceed the index range where lane groups do not)
         if (r->plan && (size_t)r->plan->g.pitch * r->plan->g.lines * d->nshots >= (size_t)1 << 31) r->plan = nullptr;
     }
-    const int variant = d->kernel_variant, xcd = d->xcd_remap;
+    int variant = d->kernel_variant, xcd = d->xcd_remap;
+    if (!r->plan) batched_default(op, d, nmedia > 1, &variant, &xcd);
     if (r->plan) {
         sp = 1;
         r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
