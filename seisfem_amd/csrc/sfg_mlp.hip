@@ -94,6 +94,7 @@ struct EpiArgs {
     float *W = nullptr, *Mw = nullptr, *Vw = nullptr;
     uint16_t *W16 = nullptr;
     int arows = 0, acols = 0;
+    bool stream = false; // EPI_ADAM: the STREAM form of the kernel
     AdamArgs ad{};
     // a product split over K (gridDim.z > 1): 0 = the parts are added into C with
     // atomics; > 0 = part z is stored (EPI_STORE) at C + z * slice
@@ -103,6 +104,25 @@ struct EpiArgs {
     // with bw updates the bias bw by Adam (moments bm, bv; arguments ad) from it
     float *db = nullptr, *bw = nullptr, *bm = nullptr, *bv = nullptr;
 };
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <bool STREAM>
+__device__ __forceinline__ float4 load4(const float *p)
+{
+    const f32x4 *q = reinterpret_cast<const f32x4 *>(p);
+    f32x4 v;
+    if constexpr (STREAM) v = __builtin_nontemporal_load(q);
+    else v = *q;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+template <bool STREAM>
+__device__ __forceinline__ void store4(float *p, const float4 &v)
+{
+    const f32x4 w = {v.x, v.y, v.z, v.w};
+    f32x4 *q = reinterpret_cast<f32x4 *>(p);
+    if constexpr (STREAM) __builtin_nontemporal_store(w, q);
+    else *q = w;
+}
 
 // ---- C = A . B^T, bf16 in, fp32 out -----------------------------------------
 // Block tile BM x BN, K in steps of BK = 64, NW waves in (NW / WN) x WN, each
@@ -117,8 +137,10 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int BK = 64, LDK = BK + 8;
 
 // TB: B is stored [K][N] (ldb >= N) instead of [N][K]; it is read along N in
-// 16-byte pieces and transposed while it is written into the LDS tile.
-template <int BM, int BN, int NW, int WN, bool TB>
+// 16-byte pieces and transposed while it is written into the LDS tile.  STREAM: the
+// weights and moments of EPI_ADAM carry the streaming (nontemporal) hint (a template
+// parameter: a run-time choice between the two kinds of access is merged into the plain one).
+template <int BM, int BN, int NW, int WN, bool TB, bool STREAM = false>
 __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, int kchunk, const uint16_t *__restrict__ A,
                                                       int lda, const uint16_t *__restrict__ B, int ldb,
                                                       float *__restrict__ C, int ldc, const EpiArgs ep)
@@ -345,9 +367,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
 #pragma unroll
                 for (int i = 0; i < PL; ++i) {
                     const size_t o = (size_t)min(r0 + a * 32 + i * RS, ep.arows - 1) * ldc + min(col, N - 4);
-                    aw[i] = *reinterpret_cast<const float4 *>(ep.W + o);
-                    am[i] = *reinterpret_cast<const float4 *>(ep.Mw + o);
-                    av[i] = *reinterpret_cast<const float4 *>(ep.Vw + o);
+                    aw[i] = load4<STREAM>(ep.W + o);
+                    am[i] = load4<STREAM>(ep.Mw + o);
+                    av[i] = load4<STREAM>(ep.Vw + o);
                 }
             }
             __syncthreads();
@@ -365,9 +387,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                     for (int e = 0; e < 4; ++e)
                         if (col + e < ep.acols) pw[e] = adam_update(pw[e], pg[e], pm[e], pv[e], ep.ad);
                     const size_t o = (size_t)row * ldc + col;
-                    *reinterpret_cast<float4 *>(ep.W + o) = w4;
-                    *reinterpret_cast<float4 *>(ep.Mw + o) = m4;
-                    *reinterpret_cast<float4 *>(ep.Vw + o) = v4;
+                    store4<STREAM>(ep.W + o, w4);
+                    store4<STREAM>(ep.Mw + o, m4);
+                    store4<STREAM>(ep.Vw + o, v4);
                     *reinterpret_cast<uint2 *>(ep.W16 + o) = make_uint2(f2bf(w4.x) | ((uint32_t)f2bf(w4.y) << 16),
                                                                         f2bf(w4.z) | ((uint32_t)f2bf(w4.w) << 16));
                     continue;
@@ -651,7 +673,10 @@ int mfail(int code, const char *fmt, ...)
 // Tiles: 256 x 128 (eight waves of 64 x 64, one block per CU) for a product whose M
 // is one or two tiles of the batch (256 x 32000 x 1024: 28.7 us against 31.0 us for
 // 128 x 128); 128 x 128 (four waves of 64 x 64) for other large products (dW of the
-// output layer, M = 32000: faster than 256 x 128); 64 x 64 below 256 tiles, the
+// output layer, M = 32000, when it is stored); 64 x 64 for dW with the Adam step, which
+// its epilogue bounds (12 bytes of weight and moments read and 14 written per element:
+// four blocks per CU keep more of them in flight than two; 32000 x 1024, batch 256:
+// 0.446 -> 0.417 ms per training step, batch 1024 0.947 -> 0.931), and below 256 tiles, the
 // K = 32000 product (dX of the output layer) split 8 ways (faster than 256 x 128 split
 // 63, and than 128 x 128 split 32: 0.520 against 0.511 ms per training step; and
 // than 16 parts: 0.474 against 0.469 ms).
@@ -663,7 +688,7 @@ struct GemmShape {
 GemmShape gemm_shape(int M, int N, int K, int kind)
 {
     GemmShape g;
-    g.big = (long)((M + 127) / 128) * ((N + 127) / 128) >= 256;
+    g.big = kind != EPI_ADAM && (long)((M + 127) / 128) * ((N + 127) / 128) >= 256;
     g.wide = g.big && M % 256 == 0 && M <= 512;
     g.bm = g.wide ? 256 : g.big ? 128 : 64;
     g.bn = g.big ? 128 : 64;
@@ -684,6 +709,7 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
     if (K % 8 || lda % 8 || ldb % 8 || M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
     if (tb && N % 8) return hipErrorInvalidValue;
     if (ep.kind == EPI_MSE && !ep.H) return hipErrorInvalidValue;
+    if (ep.stream && (ep.kind != EPI_ADAM || tb)) return hipErrorInvalidValue;
     if (ep.kind == EPI_ADAM) {
         // the row-piece epilogue must apply: 16-byte rows of C (unused), W and its moments
         auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -719,6 +745,9 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
                                ldb, C, ldc, ep);
     } else if (big) {
         if (tb) SFG_GEMM(128, true); else SFG_GEMM(128, false);
+    } else if (ep.stream) {
+        hipLaunchKernelGGL((gemm_nt_kernel<64, 64, 4, 2, false, true>), g, dim3(256), 0, st, M, N, K, kchunk, A, lda, B,
+                           ldb, C, ldc, ep);
     } else {
         if (tb) SFG_GEMM(64, true); else SFG_GEMM(64, false);
     }
@@ -1014,6 +1043,10 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
             ep.W16 = m->W16[l];
             ep.arows = m->dout[l];
             ep.acols = m->din[l];
+            // weights and moments that do not stay in the 256 MB Infinity Cache until the
+            // next step stream past it (32000 x 1024, 393 MB: 0.417 -> 0.396 ms per step;
+            // 8000 x 1024, 98 MB, would slow down, 0.216 -> 0.223)
+            ep.stream = (size_t)m->pout[l] * m->pin[l] * 12 > (size_t)192 << 20;
             ep.ad = *ad;
             MCHK(gemm(m->st, m->pout[l], m->pin[l], B, m->dzT16[l], B, m->hT16[l], B, m->G[l], m->pin[l], ep));
         } else {
