@@ -15,6 +15,7 @@
 
 #include "seisfem_gpu.h"
 #include "seisfem_host.h"
+#include "sfg_copy.h"
 #include "sfg_internal.h"
 
 using namespace sfg;
@@ -827,6 +828,7 @@ struct sfg_run {
     double *src_wt = nullptr;
     double *wavelet = nullptr, *seis_u = nullptr, *seis_w = nullptr, *energy = nullptr;
     hipStream_t stream = nullptr;
+    std::shared_ptr<Staging> staging = sfg::staging();
     hipGraphExec_t graph[2] = {nullptr, nullptr}; // guard_every steps + guard, by parity of the first step
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int executed = 0;
@@ -1682,13 +1684,10 @@ extern "C" int sfg_run_seismograms(sfg_run *r, double *u, double *w)
     HIPCHK(hipStreamSynchronize(r->stream));
     const size_t per = (size_t)r->max_steps * r->rec_num;
     if (per == 0) return SFG_OK;
-    std::vector<double> hu(per * r->S), hw(per * r->S);
-    HIPCHK(hipMemcpy(hu.data(), r->seis_u, sizeof(double) * hu.size(), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(hw.data(), r->seis_w, sizeof(double) * hw.size(), hipMemcpyDeviceToHost));
-    for (int s = 0; s < r->nshots; ++s) {
-        std::memcpy(u + per * r->perm[s], hu.data() + per * s, sizeof(double) * per);
-        std::memcpy(w + per * r->perm[s], hw.data() + per * s, sizeof(double) * per);
-    }
+    HIPCHK(download(r->staging, u, r->seis_u, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
+                    r->stream));
+    HIPCHK(download(r->staging, w, r->seis_w, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
+                    r->stream));
     return SFG_OK;
 }
 

