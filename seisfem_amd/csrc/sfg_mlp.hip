@@ -86,6 +86,9 @@ struct EpiArgs {
     const float *bias = nullptr;
     uint16_t *H = nullptr;
     int ldh = 0;
+    // EPI_BIAS_GELU (row-piece epilogue, M a multiple of 8): H transposed as well, HT[col][row]
+    uint16_t *HT = nullptr;
+    int ldht = 0;
     const float *T = nullptr;
     const int *tidx = nullptr;
     int ldt = 0;
@@ -138,10 +141,15 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int BK = 64, LDK = BK + 8;
 
 // TB: B is stored [K][N] (ldb >= N) instead of [N][K]; it is read along N in
-// 16-byte pieces and transposed while it is written into the LDS tile.  STREAM: the
+// 16-byte pieces and transposed while it is written into the LDS tile.  KIND: the
+// epilogue (a template parameter: with all epilogues in one kernel, chosen at run time,
+// the 256 x 128 tiles spilled, the 128 x 128 tiles ran one block per CU and every product
+// paid for the registers of the largest; training step at 32000 x 1024, batch 256, 0.392
+// -> 0.357 ms with the passes below fused as well, batch 1024 0.99 -> 0.80).  STREAM: the
 // weights and moments of EPI_ADAM carry the streaming (nontemporal) hint (a template
-// parameter: a run-time choice between the two kinds of access is merged into the plain one).
-template <int BM, int BN, int NW, int WN, bool TB, bool STREAM = false>
+// parameter too: a run-time choice between the two kinds of access is merged into the
+// plain one).
+template <int BM, int BN, int NW, int WN, int KIND, bool TB = false, bool STREAM = false>
 __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, int kchunk, const uint16_t *__restrict__ A,
                                                       int lda, const uint16_t *__restrict__ B, int ldb,
                                                       float *__restrict__ C, int ldc, const EpiArgs ep)
@@ -153,8 +161,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
     static_assert(TM >= 1 && TN >= 1 && LA >= 1 && LB >= 1, "tile shape");
     __shared__ __align__(16) uint16_t As[2][BM * LDK];
     __shared__ __align__(16) uint16_t Bs[2][BN * LDK];
+    __shared__ int Ti[KIND == EPI_MSE ? BM : 1]; // EPI_MSE: the sample of each row (read long before it is needed)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
+    if constexpr (KIND == EPI_MSE)
+        for (int i = tid; i < BM; i += NW * 64) Ti[i] = ep.tidx[min((int)blockIdx.y * BM + i, M - 1)];
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
     const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
     f32x16 acc[TM][TN];
@@ -310,17 +321,18 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
     };
     // row of register r in a tile whose lane rows start at rb
 #define SFG_ROW(r) (rb + ((r) >> 2) * 8 + ((r) & 3))
-    if (gridDim.z > 1) C += (size_t)blockIdx.z * ep.slice;
-    if (gridDim.z > 1 && ep.slice == 0) {
+    if constexpr (KIND == EPI_STORE)
+        if (gridDim.z > 1) C += (size_t)blockIdx.z * ep.slice;
+    if (KIND == EPI_STORE && gridDim.z > 1 && ep.slice == 0) {
         tiles([&](const f32x16 &t, int col, int rb) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (col < N && SFG_ROW(r) < M) atomicAdd(&C[(size_t)SFG_ROW(r) * ldc + col], t[r]);
         });
     } else if (N % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 &&
-               (ep.kind == EPI_STORE || (reinterpret_cast<uintptr_t>(ep.bias) & 15) == 0) &&
+               (KIND == EPI_STORE || (reinterpret_cast<uintptr_t>(ep.bias) & 15) == 0) &&
                (!ep.H || (ep.ldh % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.H) & 7) == 0)) &&
-               (ep.kind != EPI_MSE ||
+               (KIND != EPI_MSE ||
                 (ep.ldt % 4 == 0 && ep.nvalid % 4 == 0 && (reinterpret_cast<uintptr_t>(ep.T) & 15) == 0))) {
         // Each wave turns its tile rows round in LDS (the A buffers, idle after the
         // last step's barrier), 32 rows at a time, so that the epilogue reads and
@@ -336,13 +348,24 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
         // lane: columns col .. col + 3 of rows r0 + a * 32 + i * RS
         const int pc = lane % PR, pr = lane / PR;
         const int col = n0 + wn * WC + pc * 4, r0 = m0 + wm * (BM / WM) + pr;
-        const bool mse = ep.kind == EPI_MSE, act = ep.kind == EPI_BIAS_GELU;
+        constexpr bool mse = KIND == EPI_MSE, act = KIND == EPI_BIAS_GELU;
         const int nv = mse ? ep.nvalid : N; // a multiple of 4: a piece is all valid or all not
-        const bool adam = ep.kind == EPI_ADAM, biased = ep.kind != EPI_STORE && !adam;
+        constexpr bool adam = KIND == EPI_ADAM, biased = KIND != EPI_STORE && !adam;
         float4 bc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (biased) bc = *reinterpret_cast<const float4 *>(&ep.bias[min(col, N - 4)]);
+        if constexpr (biased) bc = *reinterpret_cast<const float4 *>(&ep.bias[min(col, N - 4)]);
         double lsum = 0.0;
         float cs[4] = {0.0f, 0.0f, 0.0f, 0.0f}; // the lane's column sums of the loss gradient (ep.db)
+        // targets: the 16-byte pieces of all passes, all in flight together (from clamped
+        // columns; what lies past an edge is not used)
+        float4 tv[TM][PL];
+        if constexpr (mse) {
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+#pragma unroll
+                for (int i = 0; i < PL; ++i)
+                    tv[a][i] = *reinterpret_cast<const float4 *>(ep.T + (size_t)Ti[r0 - m0 + a * 32 + i * RS] * ep.ldt +
+                                                                 min(col, nv - 4));
+        }
 #pragma unroll
         for (int a = 0; a < TM; ++a) {
 #pragma unroll
@@ -350,21 +373,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     S[((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * SLD + b * 32 + (lane & 31)] = acc[a][b][r];
-            // targets: the pass's sample indices, then its 16-byte target pieces, all
-            // from in-bounds addresses (clamped; what lies past an edge is not used),
-            // all in flight together
-            float4 tv[PL];
-            if (mse) {
-                int ti[PL];
-#pragma unroll
-                for (int i = 0; i < PL; ++i) ti[i] = ep.tidx[min(r0 + a * 32 + i * RS, M - 1)];
-#pragma unroll
-                for (int i = 0; i < PL; ++i)
-                    tv[i] = *reinterpret_cast<const float4 *>(ep.T + (size_t)ti[i] * ep.ldt + min(col, nv - 4));
-            }
             // Adam: the pass's weights and moments, likewise all issued before any store
             float4 aw[PL], am[PL], av[PL];
-            if (adam) {
+            if constexpr (adam) {
 #pragma unroll
                 for (int i = 0; i < PL; ++i) {
                     const size_t o = (size_t)min(r0 + a * 32 + i * RS, ep.arows - 1) * ldc + min(col, N - 4);
@@ -379,7 +390,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                 const int row = r0 + a * 32 + i * RS;
                 const float4 v = *reinterpret_cast<const float4 *>(&S[(pr + i * RS) * SLD + pc * 4]);
                 if (row >= M || col >= N) continue;
-                if (adam) {
+                if constexpr (adam) {
                     if (row >= ep.arows) continue;
                     float4 w4 = aw[i], m4 = am[i], v4 = av[i];
                     float *pw = &w4.x, *pm = &m4.x, *pv = &v4.x;
@@ -396,9 +407,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                     continue;
                 }
                 float4 o = v;
-                if (biased) o = make_float4(v.x + bc.x, v.y + bc.y, v.z + bc.z, v.w + bc.w);
-                if (mse) {
-                    const float d[4] = {o.x - tv[i].x, o.y - tv[i].y, o.z - tv[i].z, o.w - tv[i].w};
+                if constexpr (biased) o = make_float4(v.x + bc.x, v.y + bc.y, v.z + bc.z, v.w + bc.w);
+                if constexpr (mse) {
+                    const float d[4] = {o.x - tv[a][i].x, o.y - tv[a][i].y, o.z - tv[a][i].z, o.w - tv[a][i].w};
                     float g[4] = {0.0f, 0.0f, 0.0f, 0.0f};
                     if (col < nv) {
 #pragma unroll
@@ -410,17 +421,37 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                     }
                     o = make_float4(g[0], g[1], g[2], g[3]);
                 }
-                if (!ep.db) *reinterpret_cast<float4 *>(&C[(size_t)row * ldc + col]) = o;
-                if (ep.H) {
+                if (!(mse && ep.db)) *reinterpret_cast<float4 *>(&C[(size_t)row * ldc + col]) = o;
+                if (biased && ep.H) {
                     const float h[4] = {act ? gelu(o.x) : o.x, act ? gelu(o.y) : o.y, act ? gelu(o.z) : o.z,
                                         act ? gelu(o.w) : o.w};
-                    *reinterpret_cast<uint2 *>(&ep.H[(size_t)row * ep.ldh + col]) =
+                    const uint2 hv =
                         make_uint2(f2bf(h[0]) | ((uint32_t)f2bf(h[1]) << 16), f2bf(h[2]) | ((uint32_t)f2bf(h[3]) << 16));
+                    *reinterpret_cast<uint2 *>(&ep.H[(size_t)row * ep.ldh + col]) = hv;
+                    // the slab's piece has been read (by this lane): its first half takes the bf16 copy
+                    if (act && ep.HT) *reinterpret_cast<uint2 *>(&S[(pr + i * RS) * SLD + pc * 4]) = hv;
                 }
             }
             __syncthreads();
+            if (act && ep.HT) {
+                // each lane gathers RL rows of one column and writes them as 16-byte pieces
+                constexpr int RL = WC / 2;
+                const int c = lane % WC, rl = lane / WC * RL, rt = m0 + wm * (BM / WM) + a * 32 + rl;
+                const int gc = n0 + wn * WC + c;
+                const uint16_t *src = reinterpret_cast<const uint16_t *>(&S[rl * SLD + (c >> 2) * 4]) + (c & 3);
+                uint32_t h[RL];
+#pragma unroll
+                for (int r = 0; r < RL; ++r) h[r] = src[r * SLD * 2];
+#pragma unroll
+                for (int r = 0; r < RL; r += 8)
+                    if (gc < N && rt + r < M)
+                        *reinterpret_cast<uint4 *>(&ep.HT[(size_t)gc * ep.ldht + rt + r]) =
+                            make_uint4(h[r] | (h[r + 1] << 16), h[r + 2] | (h[r + 3] << 16), h[r + 4] | (h[r + 5] << 16),
+                                       h[r + 6] | (h[r + 7] << 16));
+                __syncthreads();
+            }
         }
-        if (mse) {
+        if constexpr (mse) {
             // one atomic per block: the waves' sums meet in LDS (free after the last
             // pass's barrier); so do the column sums of the gradient (ep.db): first
             // over the lanes that hold the same columns, then over the WM waves
@@ -455,13 +486,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                 }
             }
         }
-    } else if (ep.kind == EPI_STORE) {
+    } else if constexpr (KIND == EPI_STORE) {
         tiles([&](const f32x16 &t, int col, int rb) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (col < N && SFG_ROW(r) < M) C[(size_t)SFG_ROW(r) * ldc + col] = t[r];
         });
-    } else if (ep.kind == EPI_MSE) {
+    } else if constexpr (KIND == EPI_MSE) {
         double lsum = 0.0;
         tiles([&](const f32x16 &t, int col, int rb) __attribute__((always_inline)) {
             const bool cv = col < ep.nvalid;
@@ -469,7 +500,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
             int ti[16];
             float tv[16];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) ti[r] = (cv && SFG_ROW(r) < M) ? ep.tidx[SFG_ROW(r)] : 0;
+            for (int r = 0; r < 16; ++r) ti[r] = (cv && SFG_ROW(r) < M) ? Ti[SFG_ROW(r) - m0] : 0;
 #pragma unroll
             for (int r = 0; r < 16; ++r) tv[r] = (cv && SFG_ROW(r) < M) ? ep.T[(size_t)ti[r] * ep.ldt + col] : 0.0f;
 #pragma unroll
@@ -488,8 +519,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
         });
         for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o, 64);
         if (lane == 0) atomicAdd(ep.loss, lsum);
-    } else if (ep.kind != EPI_ADAM) { // (the host sends EPI_ADAM only where the row pieces apply)
-        const bool act = ep.kind == EPI_BIAS_GELU;
+    } else if constexpr (KIND != EPI_ADAM) { // (the host sends EPI_ADAM only where the row pieces apply)
+        constexpr bool act = KIND == EPI_BIAS_GELU;
         tiles([&](const f32x16 &t, int col, int rb) __attribute__((always_inline)) {
             const float bc = col < N ? ep.bias[col] : 0.0f;
 #pragma unroll
@@ -538,34 +569,34 @@ __global__ void zero_list_kernel(ZeroList z)
     if (t0 < n - 4 * n4) p[4 * n4 + t0] = 0.0f;
 }
 
-// dst[c][r] = src[r][c] for r < rows, c < cols (bf16), for two such matrices in
-// one launch (both operands of a weight gradient): blocks 0 .. nb0 - 1 take the
-// 32 x 32 tiles of the first, row of tiles by row, the rest those of the second
-struct Transpose {
-    int rows, cols;
-    const uint16_t *src;
-    int lds;
-    uint16_t *dst;
-    int ldd;
-};
-__global__ void transpose_bf16_kernel(Transpose t0, Transpose t1, int nb0)
+// dst[c][r] = src[r][c] (bf16; rows and cols, the row strides' lengths too, multiples of
+// 8), by 64 x 64 tiles, in 16-byte pieces on both sides: 256 x 32000 in 8 us, where 32 x
+// 32 tiles of single elements took 13
+__global__ __launch_bounds__(256) void transpose_bf16_kernel(int rows, int cols, const uint16_t *__restrict__ src,
+                                                             int lds, uint16_t *__restrict__ dst, int ldd)
 {
-    const bool second = (int)blockIdx.x >= nb0;
-    const Transpose &t = second ? t1 : t0;
-    const int rows = t.rows, cols = t.cols, lds = t.lds, ldd = t.ldd;
-    const uint16_t *src = t.src;
-    uint16_t *dst = t.dst;
-    const int b = (int)blockIdx.x - (second ? nb0 : 0), tx = (cols + 31) / 32;
-    const int c0 = (b % tx) * 32, r0 = (b / tx) * 32;
-    __shared__ uint16_t tile[32][33];
-    for (int j = threadIdx.y; j < 32; j += blockDim.y) {
-        const int r = r0 + j, c = c0 + threadIdx.x;
-        tile[j][threadIdx.x] = (r < rows && c < cols) ? src[(size_t)r * lds + c] : (uint16_t)0;
+    const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
+    __shared__ uint32_t tile[64][33];
+    for (int k = threadIdx.x; k < 512; k += 256) {
+        const int r = k >> 3, c = k & 7;
+        if (r0 + r < rows && c0 + 8 * c < cols) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(src + (size_t)(r0 + r) * lds + c0 + 8 * c);
+            uint32_t *t = &tile[r][4 * c];
+            t[0] = v.x;
+            t[1] = v.y;
+            t[2] = v.z;
+            t[3] = v.w;
+        }
     }
     __syncthreads();
-    for (int j = threadIdx.y; j < 32; j += blockDim.y) {
-        const int c = c0 + j, r = r0 + threadIdx.x;
-        if (c < cols && r < rows) dst[(size_t)c * ldd + r] = tile[threadIdx.x][j];
+    for (int k = threadIdx.x; k < 512; k += 256) {
+        const int c = k >> 3, r = 8 * (k & 7), sh = 16 * (c & 1);
+        if (c0 + c >= cols || r0 + r >= rows) continue;
+        uint32_t h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            h[i] = ((tile[r + 2 * i][c >> 1] >> sh) & 0xffffu) | ((tile[r + 2 * i + 1][c >> 1] >> sh) << 16);
+        *reinterpret_cast<uint4 *>(dst + (size_t)(c0 + c) * ldd + r0 + r) = make_uint4(h[0], h[1], h[2], h[3]);
     }
 }
 
@@ -575,49 +606,145 @@ __global__ void f32_to_bf16_kernel(size_t n, const float *src, uint16_t *dst)
         dst[i] = f2bf(src[i]);
 }
 
-// rows of X (nin wide) for the given sample indices -> bf16 [batch][ldx], zero padded
-// (and *zero = 0, the batch's loss accumulator, by the first thread)
+// rows of X (width wide) for the given sample indices -> bf16 dst[batch][ld], zero padded,
+// and, with dstT, its transpose dstT[ld][batch] (and *zero = 0, the batch's loss
+// accumulator, by the first thread)
 __global__ void gather_rows_kernel(int batch, int width, int ld, const float *src, const int *idx, uint16_t *dst,
-                                   float *dstf, double *zero)
+                                   uint16_t *dstT, double *zero)
 {
     const int b = blockIdx.y;
     if (zero && b == 0 && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0.0;
     if (b >= batch) return;
     const size_t s = (size_t)idx[b];
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ld; c += gridDim.x * blockDim.x) {
-        const float v = c < width ? src[s * width + c] : 0.0f;
-        if (dst) dst[(size_t)b * ld + c] = f2bf(v);
-        if (dstf) dstf[(size_t)b * ld + c] = v;
+        const uint16_t v = f2bf(c < width ? src[s * width + c] : 0.0f);
+        dst[(size_t)b * ld + c] = v;
+        if (dstT) dstT[(size_t)c * batch + b] = v;
     }
 }
 
-// dz = dh * gelu'(z) (fp32 and bf16 copies), dh the sum of the nparts parts of
-// a product split over K (part p at parts + p * slice), added in part order
-__global__ void gelu_back_kernel(size_t n, const float *parts, int nparts, size_t slice, const float *z, float *dz,
-                                 uint16_t *dz16)
+// What lies between two products of a hidden layer, rows = the batch, cols the layer's
+// padded width (row stride of everything but T), from the nparts parts of a product
+// split over K (part p at parts + p * slice, added in part order):
+//   forward   z = sum + bias[col], H = bf16(gelu(z))
+//   BACK      dz = sum * gelu'(z), H = bf16(dz); db[col] = the sum of dz over the batch
+//             (col < valid), and with bw the bias's Adam step from it
+// and with T the transpose of H, T[col][row] (rows a multiple of 8), which the dW
+// product reads.  A block takes 16 columns of the whole batch, HR rows at a time in LDS,
+// so that the column sums and the transpose cost no further pass: 9 us for 256 x 1024
+// backward in 8 parts, where GELU, column sums and transpose as separate kernels took 17.
+// What is left is the latency of the loads on a quarter of the chip.  HR = 256 (1024
+// threads, one pass for a batch of 256) is the faster form alone (13 us with HR = 64);
+// beside a kernel that fills the chip such a block waits for a whole CU to drain (150 us),
+// and HR = 64 (256 threads) starts in any free slot (20 to 30 us).
+constexpr int HC = 16, HLD = HC + 1, HP = 8;
+template <bool BACK, int HR>
+__global__ __launch_bounds__(4 * HR) void hidden_kernel(int rows, int cols, int valid, const float *__restrict__ parts,
+                                                    int nparts, size_t slice, float *__restrict__ z,
+                                                    uint16_t *__restrict__ H, uint16_t *__restrict__ T,
+                                                    const float *__restrict__ bias, float *db, float *bw, float *bm,
+                                                    float *bv, AdamArgs ad)
 {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        float dh = parts[i];
-        for (int p = 1; p < nparts; ++p) dh += parts[p * slice + i];
-        const float g = dh * gelu_grad(z[i]);
-        dz[i] = g;
-        dz16[i] = f2bf(g);
+    __shared__ float tile[2][HR * HLD];
+    __shared__ float chain[16 * HC];
+    const int tid = threadIdx.x, c0 = blockIdx.x * HC;
+    const int q = tid & 3, lr = tid >> 2, col = c0 + 4 * q;
+    // column sums: thread tid < 256 takes column tid % 16 and the rows j, j + 16, ..  (j = tid
+    // / 16 = y + 4 u, u < 4) below the last whole group of its y; y's chains are added as
+    // (0 + 1) + (2 + 3), the rows left over to chain 0, and the four y the same way
+    const int j = tid >> 4, sc = tid & 15, y = j & 3;
+    const int whole = rows > y + 12 ? (rows - y - 13) / 16 + 1 : 0;
+    float sum = 0.0f;
+    float4 bc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (!BACK) bc = *reinterpret_cast<const float4 *>(bias + col);
+    // a pass's first HP parts and z (clamped addresses, no branch), a pass ahead of their use
+    struct Pass {
+        float4 w[HP], z;
+    };
+    auto load = [&](Pass &x, int r0) __attribute__((always_inline)) {
+        const size_t o = (size_t)min(r0 + lr, rows - 1) * cols + col;
+#pragma unroll
+        for (int k = 0; k < HP; ++k)
+            x.w[k] = *reinterpret_cast<const float4 *>(parts + min(k, nparts - 1) * slice + o);
+        if (BACK) x.z = *reinterpret_cast<const float4 *>(z + o);
+    };
+    auto add = [](const float4 &a, const float4 &b) __attribute__((always_inline)) {
+        return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+    };
+    auto pass = [&](const Pass &x, int r0, float *t0) __attribute__((always_inline)) {
+        const int row = r0 + lr;
+        if (row < rows) {
+            const size_t o = (size_t)row * cols + col;
+            float4 v = x.w[0];
+#pragma unroll
+            for (int k = 1; k < HP; ++k)
+                if (k < nparts) v = add(v, x.w[k]);
+            for (int p = HP; p < nparts; p += HP) {
+                float4 w[HP];
+#pragma unroll
+                for (int k = 0; k < HP; ++k)
+                    w[k] = *reinterpret_cast<const float4 *>(parts + min(p + k, nparts - 1) * slice + o);
+#pragma unroll
+                for (int k = 0; k < HP; ++k)
+                    if (p + k < nparts) v = add(v, w[k]);
+            }
+            float4 h;
+            if (BACK) {
+                v = make_float4(v.x * gelu_grad(x.z.x), v.y * gelu_grad(x.z.y), v.z * gelu_grad(x.z.z),
+                                v.w * gelu_grad(x.z.w));
+                h = v;
+            } else {
+                v = add(v, bc);
+                *reinterpret_cast<float4 *>(z + o) = v;
+                h = make_float4(gelu(v.x), gelu(v.y), gelu(v.z), gelu(v.w));
+            }
+            *reinterpret_cast<uint2 *>(H + o) =
+                make_uint2(f2bf(h.x) | ((uint32_t)f2bf(h.y) << 16), f2bf(h.z) | ((uint32_t)f2bf(h.w) << 16));
+            float *t = t0 + lr * HLD + 4 * q;
+            t[0] = h.x;
+            t[1] = h.y;
+            t[2] = h.z;
+            t[3] = h.w;
+        }
+        __syncthreads(); // (one barrier a pass: the next one fills the other tile)
+        if (T) {
+            const int c = tid / (HR / 4), rr = 4 * (tid % (HR / 4));
+            if (r0 + rr < rows) {
+                const float *t = t0 + rr * HLD + c;
+                *reinterpret_cast<uint2 *>(T + (size_t)(c0 + c) * rows + r0 + rr) =
+                    make_uint2(f2bf(t[0]) | ((uint32_t)f2bf(t[HLD]) << 16),
+                               f2bf(t[2 * HLD]) | ((uint32_t)f2bf(t[3 * HLD]) << 16));
+            }
+        }
+        if (BACK && j < 16) {
+            const int end = min(whole, (r0 + HR) / 16);
+            for (int k = r0 / 16; k < end; ++k) sum += t0[(j + 16 * k - r0) * HLD + sc];
+            if (j < 4 && r0 + HR >= rows)
+                for (int r = y + 16 * whole; r < rows; r += 4) sum += t0[(r - r0) * HLD + sc];
+        }
+    };
+    Pass a, b;
+    load(a, 0);
+    for (int r0 = 0; r0 < rows; r0 += 2 * HR) {
+        load(b, r0 + HR);
+        pass(a, r0, tile[0]);
+        if (r0 + HR >= rows) break;
+        load(a, r0 + 2 * HR);
+        pass(b, r0 + HR, tile[1]);
     }
-}
-
-// A hidden layer's forward epilogue after a product split over K: z = (sum of the
-// nparts parts, in part order) + bias[c], h = bf16(gelu(z)); rows x cols, row
-// stride cols for all of them
-__global__ void bias_gelu_parts_kernel(int rows, int cols, const float *parts, int nparts, size_t slice,
-                                       const float *bias, float *z, uint16_t *h)
-{
-    const int n = rows * cols;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        float v = parts[i];
-        for (int p = 1; p < nparts; ++p) v += parts[p * slice + i];
-        const float zz = v + bias[i % cols];
-        z[i] = zz;
-        h[i] = f2bf(gelu(zz));
+    if (!BACK) return;
+    if (j < 16) chain[j * HC + sc] = sum;
+    __syncthreads();
+    if (tid < HC && c0 + tid < valid) {
+        float s[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            s[k] = (chain[k * HC + tid] + chain[(k + 4) * HC + tid]) +
+                   (chain[(k + 8) * HC + tid] + chain[(k + 12) * HC + tid]);
+        const float g = (s[0] + s[1]) + (s[2] + s[3]);
+        const int c = c0 + tid;
+        db[c] = g;
+        if (bw) bw[c] = adam_update(bw[c], g, bm[c], bv[c], ad);
     }
 }
 
@@ -708,9 +835,16 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
                 int ldc, const EpiArgs &ep, bool tb = false, bool zeroed = false)
 {
     if (K % 8 || lda % 8 || ldb % 8 || M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
-    if (tb && N % 8) return hipErrorInvalidValue;
+    if (tb && (N % 8 || ep.kind != EPI_STORE)) return hipErrorInvalidValue;
     if (ep.kind == EPI_MSE && !ep.H) return hipErrorInvalidValue;
-    if (ep.stream && (ep.kind != EPI_ADAM || tb)) return hipErrorInvalidValue;
+    if (ep.HT) {
+        // the row-piece epilogue must apply
+        auto al = [](const void *p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; };
+        if (ep.kind != EPI_BIAS_GELU || M % 8 || ep.ldht % 8 || ep.ldht < M || !al(ep.HT, 16) || !ep.H || N % 4 ||
+            ldc % 4 || !al(C, 16) || !ep.bias || !al(ep.bias, 16) || ep.ldh % 4 || !al(ep.H, 8))
+            return hipErrorInvalidValue;
+    }
+    if (ep.stream && ep.kind != EPI_ADAM) return hipErrorInvalidValue;
     if (ep.kind == EPI_ADAM) {
         // the row-piece epilogue must apply: 16-byte rows of C (unused), W and its moments
         auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
@@ -734,32 +868,29 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
     if (splits > 1 && !zeroed && !ep.slice)
         hipLaunchKernelGGL(fill_zero_f32_kernel, dim3(1024), dim3(256), 0, st, M, N, ldc, C);
     const dim3 g((N + bn - 1) / bn, (M + bm - 1) / bm, splits);
-#define SFG_GEMM(BMV, TBV)                                                                                        \
-    hipLaunchKernelGGL((gemm_nt_kernel<BMV, BMV, 4, 2, TBV>), g, dim3(256), 0, st, M, N, K, kchunk, A, lda, B, ldb, C, \
-                       ldc, ep)
-    if (wide) {
-        if (tb)
-            hipLaunchKernelGGL((gemm_nt_kernel<256, 128, 8, 2, true>), g, dim3(512), 0, st, M, N, K, kchunk, A, lda, B,
-                               ldb, C, ldc, ep);
-        else
-            hipLaunchKernelGGL((gemm_nt_kernel<256, 128, 8, 2, false>), g, dim3(512), 0, st, M, N, K, kchunk, A, lda, B,
-                               ldb, C, ldc, ep);
-    } else if (big) {
-        if (tb) SFG_GEMM(128, true); else SFG_GEMM(128, false);
-    } else if (ep.stream) {
-        hipLaunchKernelGGL((gemm_nt_kernel<64, 64, 4, 2, false, true>), g, dim3(256), 0, st, M, N, K, kchunk, A, lda, B,
-                           ldb, C, ldc, ep);
-    } else {
-        if (tb) SFG_GEMM(64, true); else SFG_GEMM(64, false);
+#define SFG_GEMM(...)                                                                                              \
+    hipLaunchKernelGGL((gemm_nt_kernel<__VA_ARGS__>), g, dim3(bm == 256 ? 512 : 256), 0, st, M, N, K, kchunk, A, lda, B, \
+                       ldb, C, ldc, ep)
+#define SFG_GEMM_TILES(...)                                                                                        \
+    do {                                                                                                           \
+        if (wide) SFG_GEMM(256, 128, 8, 2, __VA_ARGS__);                                                           \
+        else if (big) SFG_GEMM(128, 128, 4, 2, __VA_ARGS__);                                                       \
+        else SFG_GEMM(64, 64, 4, 2, __VA_ARGS__);                                                                  \
+    } while (0)
+    switch (ep.kind) {
+    case EPI_BIAS: SFG_GEMM_TILES(EPI_BIAS); break;
+    case EPI_BIAS_GELU: SFG_GEMM_TILES(EPI_BIAS_GELU); break;
+    case EPI_MSE: SFG_GEMM_TILES(EPI_MSE); break;
+    case EPI_ADAM:
+        if (ep.stream) SFG_GEMM(64, 64, 4, 2, EPI_ADAM, false, true);
+        else SFG_GEMM(64, 64, 4, 2, EPI_ADAM);
+        break;
+    default:
+        if (tb) SFG_GEMM_TILES(EPI_STORE, true);
+        else SFG_GEMM_TILES(EPI_STORE);
     }
+#undef SFG_GEMM_TILES
 #undef SFG_GEMM
-    return hipGetLastError();
-}
-
-hipError_t transpose2(hipStream_t st, const Transpose &a, const Transpose &b)
-{
-    const int nb0 = ((a.cols + 31) / 32) * ((a.rows + 31) / 32), nb1 = ((b.cols + 31) / 32) * ((b.rows + 31) / 32);
-    hipLaunchKernelGGL(transpose_bf16_kernel, dim3(nb0 + nb1), dim3(32, 8), 0, st, a, b, nb0);
     return hipGetLastError();
 }
 
@@ -790,11 +921,33 @@ struct sfg_mlp {
     int ndata = 0;
     long step = 0;
     hipStream_t st = nullptr;
+    // With `beside` the output layer's dW and Adam step run on stream st2 beside the rest
+    // of the backward pass and the next forward pass up to that layer (which fills the spare
+    // of the transposed input that dW reads).  Taken where that step streams through more
+    // weights and moments than the caches hold (EpiArgs::stream) and so leaves the matrix
+    // cores and most latencies of the others uncovered: 32000 x 1024, batch 256, 0.357 ->
+    // 0.336 ms per step (batch 64 0.291 -> 0.258, batch 1024 0.797 -> 0.763); the waits for
+    // each other cost more than that where it is short: 8000 x 1024 0.197 -> 0.213 ms.
+    bool beside = false;
+    hipStream_t st2 = nullptr;
+    hipEvent_t dz_ready = nullptr, w_ready = nullptr;
+    bool pending = false;  // st does not yet wait for w_ready
+    uint16_t *hT16_spare = nullptr;
     std::shared_ptr<sfg::Staging> staging = sfg::staging();
 };
 
+// Weights and moments of a layer that do not stay in the 256 MB Infinity Cache until the
+// next step stream past it (32000 x 1024, 393 MB: 0.417 -> 0.396 ms per step; 8000 x
+// 1024, 98 MB, would slow down, 0.216 -> 0.223)
+static bool streams(const sfg_mlp *m, int l)
+{
+    return (size_t)m->pout[l] * m->pin[l] * 12 > (size_t)192 << 20;
+}
+
 static void mlp_free(sfg_mlp *m)
 {
+    for (hipStream_t x : {m->st2, m->st})
+        if (x) (void)hipStreamSynchronize(x);
     auto F = [](auto &vec) {
         for (auto *p : vec)
             if (p) (void)hipFree(p);
@@ -805,6 +958,10 @@ static void mlp_free(sfg_mlp *m)
     for (void *p : {(void *)m->y, (void *)m->part, (void *)m->loss, (void *)m->idx, (void *)m->order, (void *)m->Xd,
                     (void *)m->Yd})
         if (p) (void)hipFree(p);
+    if (m->hT16_spare) (void)hipFree(m->hT16_spare);
+    for (hipEvent_t x : {m->dz_ready, m->w_ready})
+        if (x) (void)hipEventDestroy(x);
+    if (m->st2) (void)hipStreamDestroy(m->st2);
     if (m->st) (void)hipStreamDestroy(m->st);
     delete m;
 }
@@ -835,7 +992,11 @@ extern "C" int sfg_mlp_create(sfg_mlp **out, int nin, int hidden, int nhidden_la
         m->pin.push_back(pad32(m->din.back()));
         m->pout.push_back(pad32(m->dout.back()));
     }
+    m->beside = streams(m, m->nl - 1);
     hipError_t e = hipStreamCreateWithFlags(&m->st, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&m->st2, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&m->dz_ready, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&m->w_ready, hipEventDisableTiming);
     // He-style uniform init from a fixed-seed generator, on the host
     uint64_t s = seed * 0x9E3779B97F4A7C15ull + 1;
     auto rnd = [&]() {
@@ -871,13 +1032,15 @@ extern "C" int sfg_mlp_create(sfg_mlp **out, int nin, int hidden, int nhidden_la
         e = zalloc(&h, (size_t)batch * m->pin[l]);
         if (e == hipSuccess) e = zalloc(&hT, (size_t)batch * m->pin[l]);
         if (e == hipSuccess) e = zalloc(&zz, (size_t)batch * m->pout[l]);
-        if (e == hipSuccess) e = zalloc(&dd, (size_t)batch * m->pout[l]);
+        dd = nullptr; // only the output layer's gradient is kept in FP32 as well
+        if (e == hipSuccess && l == m->nl - 1) e = zalloc(&dd, (size_t)batch * m->pout[l]);
         if (e == hipSuccess) e = zalloc(&dhh, (size_t)batch * m->pin[l]);
         if (e == hipSuccess) e = zalloc(&d16, (size_t)batch * m->pout[l]);
         if (e == hipSuccess) e = zalloc(&dT, (size_t)batch * m->pout[l]);
         m->h16.push_back(h); m->hT16.push_back(hT); m->z.push_back(zz); m->dz.push_back(dd);
         m->dh.push_back(dhh); m->dz16.push_back(d16); m->dzT16.push_back(dT);
     }
+    if (e == hipSuccess) e = zalloc(&m->hT16_spare, (size_t)batch * m->pin.back());
     if (e == hipSuccess) e = zalloc(&m->y, (size_t)batch * m->pout.back());
     // room for the parts of the largest product split over K
     for (int l = 0; l < m->nl; ++l) {
@@ -918,6 +1081,14 @@ extern "C" long long sfg_mlp_param_count(const sfg_mlp *m)
     return c;
 }
 
+// stream st waits for the output layer's last Adam step
+static hipError_t join(sfg_mlp *m)
+{
+    if (!m->pending) return hipSuccess;
+    m->pending = false;
+    return hipStreamWaitEvent(m->st, m->w_ready, 0);
+}
+
 // forward of the current batch (h16[0] holds its input, loaded by load_batch,
 // which also zeroes *loss).  Without targets the output goes to y; with targets
 // Y (rows by the batch's sample indices idx, on the device) the output layer's
@@ -927,6 +1098,7 @@ extern "C" long long sfg_mlp_param_count(const sfg_mlp *m)
 static int forward(sfg_mlp *m, const float *Y = nullptr, const int *idx = nullptr, const AdamArgs *ad = nullptr)
 {
     m->out_db = false;
+    const bool trans = Y && m->batch % 8 == 0; // the dW products' transposed operands too
     for (int l = 0; l < m->nl; ++l) {
         const bool last = l == m->nl - 1;
         if (!last) {
@@ -937,12 +1109,16 @@ static int forward(sfg_mlp *m, const float *Y = nullptr, const int *idx = nullpt
                 ep.slice = (size_t)m->batch * m->pout[l];
                 MCHK(gemm(m->st, m->batch, m->pout[l], m->pin[l], m->h16[l], m->pin[l], m->W16[l], m->pin[l], m->part,
                           m->pout[l], ep));
-                hipLaunchKernelGGL(bias_gelu_parts_kernel, dim3(1024), dim3(256), 0, m->st, m->batch, m->pout[l],
-                                   m->part, gs.splits, ep.slice, m->b[l], m->z[l], m->h16[l + 1]);
+                hipLaunchKernelGGL((m->beside ? hidden_kernel<false, 64> : hidden_kernel<false, 256>),
+                                   dim3(m->pout[l] / HC), dim3(m->beside ? 256 : 1024), 0, m->st, m->batch,
+                                   m->pout[l], m->dout[l], m->part, gs.splits, ep.slice, m->z[l], m->h16[l + 1],
+                                   trans ? m->hT16[l + 1] : nullptr, m->b[l], nullptr, nullptr, nullptr, nullptr,
+                                   AdamArgs{});
                 MCHK(hipGetLastError());
                 continue;
             }
         }
+        if (last) MCHK(join(m));
         EpiArgs ep;
         ep.bias = m->b[l];
         float *C = m->z[l];
@@ -950,6 +1126,10 @@ static int forward(sfg_mlp *m, const float *Y = nullptr, const int *idx = nullpt
             ep.kind = EPI_BIAS_GELU;
             ep.H = m->h16[l + 1];
             ep.ldh = m->pin[l + 1];
+            if (trans) {
+                ep.HT = m->hT16[l + 1];
+                ep.ldht = m->batch;
+            }
         } else if (!Y) {
             ep.kind = EPI_BIAS;
             C = m->y;
@@ -992,7 +1172,7 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
     const int B = m->batch;
     // without an Adam step, the dW products split over K (narrow layers) add into
     // their outputs: all of those are zeroed by one launch up front (the dX
-    // products split over K store their parts, which gelu_back adds up)
+    // products split over K store their parts, which hidden_kernel adds up)
     ZeroList zl{};
     std::vector<char> zw(m->nl, 0);
     for (int l = m->nl - 1; l >= 0 && zl.count < 8; --l) {
@@ -1006,10 +1186,50 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
         hipLaunchKernelGGL(zero_list_kernel, dim3(256, zl.count), dim3(256), 0, m->st, zl);
         MCHK(hipGetLastError());
     }
-    for (int l = m->nl - 1; l >= 0; --l) {
+    // dW = dz^T . h from transposed copies (A = dz^T [pout][B], B = h^T [pin][B]); K = batch.
+    // Reading both operands k-major instead measured 2.4x slower (transposing into LDS
+    // element by element costs as much as the products at this small K).  With ad the
+    // Adam step is in the product's epilogue (the gradient is never stored), which writes
+    // the bf16 weights to W16.
+    auto weights = [&](hipStream_t st, int l) {
+        EpiArgs ep;
+        if (ad) {
+            ep.kind = EPI_ADAM;
+            ep.W = m->W[l];
+            ep.Mw = m->Mw[l];
+            ep.Vw = m->Vw[l];
+            ep.W16 = m->W16[l];
+            ep.arows = m->dout[l];
+            ep.acols = m->din[l];
+            ep.stream = streams(m, l);
+            ep.ad = *ad;
+        }
+        return gemm(st, m->pout[l], m->pin[l], B, m->dzT16[l], B, m->hT16[l], B, m->G[l], m->pin[l], ep, false, zw[l]);
+    };
+    const int L = m->nl - 1;
+    if (!m->out_db) { // (else formed in the forward pass's loss epilogue)
+        hipLaunchKernelGGL(bias_grad_kernel, dim3((m->pout[L] + 63) / 64), dim3(256), 0, m->st, B, m->dout[L],
+                           m->pout[L], m->dz[L], m->gb[L], ad ? m->b[L] : nullptr, m->Mb[L], m->Vb[L],
+                           ad ? *ad : AdamArgs{});
+        MCHK(hipGetLastError());
+    }
+    // the output layer's dW needs nothing of what follows dX, and nothing before the next
+    // forward pass's output layer needs its result
+    const bool over = ad && m->beside;
+    const hipStream_t so = over ? m->st2 : m->st;
+    if (over) {
+        MCHK(hipEventRecord(m->dz_ready, m->st));
+        MCHK(hipStreamWaitEvent(m->st2, m->dz_ready, 0));
+    }
+    if (B % 8 == 0) { // (gemm refuses other K)
+        hipLaunchKernelGGL(transpose_bf16_kernel, dim3((m->pout[L] + 63) / 64, (B + 63) / 64), dim3(256), 0, so, B,
+                           m->pout[L], m->dz16[L], m->pout[L], m->dzT16[L], B);
+        MCHK(hipGetLastError());
+    }
+    for (int l = L; l >= 0; --l) {
         if (l > 0) {
             // dh = dz . W (W [pout][pin] read k-major as stored) ; dz_{l-1} = dh * gelu'(z_{l-1});
-            // split over K, the product's parts go to m->part and gelu_back adds them up
+            // split over K, the product's parts go to m->part and hidden_kernel adds them up
             const GemmShape gs = gemm_shape(B, m->pin[l], m->pout[l], EPI_STORE);
             const size_t n = (size_t)B * m->pin[l];
             EpiArgs ep;
@@ -1020,41 +1240,21 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
             }
             MCHK(gemm(m->st, B, m->pin[l], m->pout[l], m->dz16[l], m->pout[l], m->W16[l], m->pin[l], dh, m->pin[l], ep,
                       true));
-            hipLaunchKernelGGL(gelu_back_kernel, dim3(1024), dim3(256), 0, m->st, n, dh, gs.splits, ep.slice,
-                               m->z[l - 1], m->dz[l - 1], m->dz16[l - 1]);
+            if (l == L && over) { // (dX has read the bf16 weights)
+                MCHK(hipEventRecord(m->dz_ready, m->st));
+                MCHK(hipStreamWaitEvent(m->st2, m->dz_ready, 0));
+                MCHK(weights(m->st2, L));
+                MCHK(hipEventRecord(m->w_ready, m->st2));
+                m->pending = true;
+                std::swap(m->hT16[L], m->hT16_spare);
+            }
+            hipLaunchKernelGGL((m->beside ? hidden_kernel<true, 64> : hidden_kernel<true, 256>), dim3(m->pin[l] / HC),
+                               dim3(m->beside ? 256 : 1024), 0, m->st, B, m->pin[l], m->din[l], dh, gs.splits, ep.slice, m->z[l - 1], m->dz16[l - 1],
+                               B % 8 ? nullptr : m->dzT16[l - 1], nullptr, m->gb[l - 1], ad ? m->b[l - 1] : nullptr,
+                               m->Mb[l - 1], m->Vb[l - 1], ad ? *ad : AdamArgs{});
             MCHK(hipGetLastError());
         }
-        if (!(l == m->nl - 1 && m->out_db)) { // (else formed in the forward pass's loss epilogue)
-            hipLaunchKernelGGL(bias_grad_kernel, dim3((m->pout[l] + 63) / 64), dim3(256), 0, m->st, B, m->dout[l],
-                               m->pout[l], m->dz[l], m->gb[l], ad ? m->b[l] : nullptr, m->Mb[l], m->Vb[l],
-                               ad ? *ad : AdamArgs{});
-            MCHK(hipGetLastError());
-        }
-        // dW = dz^T . h from transposed copies (A = dz^T [pout][B], B = h^T [pin][B]); K = batch.
-        // Reading both operands k-major instead measured 2.4x slower (transposing into LDS
-        // element by element costs as much as the products at this small K)
-        MCHK(transpose2(m->st, Transpose{B, m->pout[l], m->dz16[l], m->pout[l], m->dzT16[l], B},
-                        Transpose{B, m->pin[l], m->h16[l], m->pin[l], m->hT16[l], B}));
-        if (ad) {
-            // the weights' Adam step in the dW product's epilogue: the gradient is never stored
-            EpiArgs ep;
-            ep.kind = EPI_ADAM;
-            ep.W = m->W[l];
-            ep.Mw = m->Mw[l];
-            ep.Vw = m->Vw[l];
-            ep.W16 = m->W16[l];
-            ep.arows = m->dout[l];
-            ep.acols = m->din[l];
-            // weights and moments that do not stay in the 256 MB Infinity Cache until the
-            // next step stream past it (32000 x 1024, 393 MB: 0.417 -> 0.396 ms per step;
-            // 8000 x 1024, 98 MB, would slow down, 0.216 -> 0.223)
-            ep.stream = (size_t)m->pout[l] * m->pin[l] * 12 > (size_t)192 << 20;
-            ep.ad = *ad;
-            MCHK(gemm(m->st, m->pout[l], m->pin[l], B, m->dzT16[l], B, m->hT16[l], B, m->G[l], m->pin[l], ep));
-        } else {
-            MCHK(gemm(m->st, m->pout[l], m->pin[l], B, m->dzT16[l], B, m->hT16[l], B, m->G[l], m->pin[l], EpiArgs{},
-                      false, zw[l]));
-        }
+        if (!(l == L && over)) MCHK(weights(m->st, l));
     }
     return SFG_OK;
 }
@@ -1070,10 +1270,10 @@ static int upload_idx(sfg_mlp *m, const int *idx_host, int nsrc)
 }
 
 // rows idx[batch] (device) of X -> bf16 input h16[0]
-static int load_batch(sfg_mlp *m, const int *idx, const float *X)
+static int load_batch(sfg_mlp *m, const int *idx, const float *X, bool train)
 {
     hipLaunchKernelGGL(gather_rows_kernel, dim3(1, m->batch), dim3(64), 0, m->st, m->batch, m->nin, m->pin[0], X,
-                       idx, m->h16[0], (float *)nullptr, m->loss);
+                       idx, m->h16[0], train ? m->hT16[0] : nullptr, m->loss);
     MCHK(hipGetLastError());
     return SFG_OK;
 }
@@ -1120,11 +1320,12 @@ extern "C" int sfg_mlp_train_step(sfg_mlp *m, const int *idx, float lr, double *
     g_mlp_err.clear();
     if (!m || !idx || !m->Xd) return mfail(SFG_E_ARG, "mlp train: no data");
     int rc = upload_idx(m, idx, m->ndata);
-    if (!rc) rc = load_batch(m, m->idx, m->Xd);
+    if (!rc) rc = load_batch(m, m->idx, m->Xd, true);
     AdamArgs ad{};
     if (!rc) ad = next_adam(m, lr);
     if (!rc) rc = forward(m, m->Yd, m->idx, &ad);
     if (!rc) rc = backward(m, &ad);
+    MCHK(join(m));
     double h = 0.0;
     if (!rc) rc = read_loss(m, &h); // also ends the host index buffer's use
     if (!rc && loss) *loss = h;
@@ -1163,14 +1364,18 @@ extern "C" int sfg_mlp_train(sfg_mlp *m, int epochs, float lr0, long long total_
             const double prog = std::min(1.0, (double)(m->step) / (double)T);
             const float lr = (float)(lr0 * 0.5 * (1.0 + std::cos(M_PI * prog)));
             const int *idx = m->order + (size_t)k * B;
-            int rc = load_batch(m, idx, m->Xd);
+            int rc = load_batch(m, idx, m->Xd, true);
             AdamArgs ad{};
             if (!rc) ad = next_adam(m, lr);
             if (!rc) rc = forward(m, m->Yd, idx, &ad);
             if (!rc) rc = backward(m, &ad);
-            if (rc) return rc;
+            if (rc) {
+                (void)join(m);
+                return rc;
+            }
             ++done;
         }
+        MCHK(join(m));
         MCHK(hipStreamSynchronize(m->st));
     }
     MCHK(hipEventRecord(e1, m->st));
@@ -1206,7 +1411,7 @@ extern "C" int sfg_mlp_predict(sfg_mlp *m, const float *X, int n, float *Y, doub
         const int cnt = std::min(B, n - s0);
         for (int b = 0; b < B; ++b) idx[b] = s0 + std::min(b, cnt - 1);
         int rc = upload_idx(m, idx.data(), n);
-        if (!rc) rc = load_batch(m, m->idx, Xd);
+        if (!rc) rc = load_batch(m, m->idx, Xd, false);
         MCHK(hipEventRecord(e0, m->st));
         if (!rc) rc = forward(m);
         MCHK(hipEventRecord(e1, m->st));
@@ -1240,7 +1445,7 @@ extern "C" int sfg_mlp_gradients(sfg_mlp *m, const float *Xb, const float *Yb, d
     std::vector<int> idx(m->batch);
     for (int b = 0; b < m->batch; ++b) idx[b] = b;
     int rc = upload_idx(m, idx.data(), m->batch);
-    if (!rc) rc = load_batch(m, m->idx, Xd);
+    if (!rc) rc = load_batch(m, m->idx, Xd, true);
     if (!rc) rc = forward(m, Yd, m->idx);
     if (!rc) rc = backward(m);
     double h = 0.0;
