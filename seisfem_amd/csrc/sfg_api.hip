@@ -223,7 +223,7 @@ struct GridPlan {
     bool vals[2] = {false, false};
     ~GridPlan()
     {
-        for (int *q : {rows, cls, slice, smax, toff, tlen, trep, tdst, moff, sdel}) dfree(q);
+        for (int *q : {rows, cls, slice, smax, toff, moff, sdel}) dfree(q); // (toff holds tlen, trep and tdst too)
         for (int k = 0; k < 2; ++k) { dfree(tab[k]); dfree(mval[k]); }
     }
 };
@@ -518,20 +518,23 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
         if ((q * P.magic) >> 16 != q / g.W) return SFG_OK;
     P.g = g;
     const int nw = g.npatch * (g.most / 64);
-    int f[4];
-    struct Tmp { // device scratch of this call
-        int *flags = nullptr, *key = nullptr;
+    const size_t nrows = (size_t)g.npatch * g.most;
+    struct Tmp { // device scratch of this call: hashes; rows' classes, classes' first rows and entries
+        int *key = nullptr;
         unsigned long long *h = nullptr;
-        ~Tmp() { dfree(flags); dfree(key); dfree(h); }
+        ~Tmp() { dfree(key); dfree(h); }
     } tmp;
-    if ((rc = dalloc(&tmp.flags, 4)) || (rc = dalloc(&tmp.h, 2 * (size_t)n)) || (rc = dalloc(&tmp.key, n)) ||
-        (rc = dalloc(&P.rows, (size_t)g.npatch * g.most)) || (rc = dalloc(&P.cls, (size_t)g.npatch * g.most)) ||
-        (rc = dalloc(&P.slice, nw)) || (rc = dalloc(&P.smax, nw)))
+    // (transfers of a plan are small and each costs its latency: what goes together is
+    // packed.  The flags of the check lie behind the keys that come back with them.)
+    if ((rc = dalloc(&tmp.h, 2 * (size_t)n)) || (rc = dalloc(&tmp.key, (size_t)n + 2 * kGridClasses + 1)) ||
+        (rc = dalloc(&P.rows, nrows)) || (rc = dalloc(&P.cls, nrows + 4)) || (rc = dalloc(&P.slice, nw)) ||
+        (rc = dalloc(&P.smax, nw)))
         return rc;
+    int *const flags = P.cls + nrows;
     // the most compact mode whose tables fit
     std::vector<unsigned long long> h(n);
     HIPCHK(launch_grid_hash(n, op->rp, op->ci, op->v64, (size_t)op->nnz, tmp.h, st));
-    std::vector<int> cls, rep, keys((size_t)g.npatch * g.most), cptr, toff, tlen, trep, tdst;
+    std::vector<int> cls, rep, keys(nrows + 4), packed, cptr, toff, tlen, trep, tdst;
     int mode = GRID_ROWS;
     for (int m = GRID_CLASS; m < GRID_ROWS && mode == GRID_ROWS; ++m) {
         HIPCHK(hipMemcpyAsync(h.data(), tmp.h + (m == GRID_CLASS ? n : 0), sizeof(unsigned long long) * n,
@@ -541,20 +544,18 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
         const int nclass = (int)rep.size();
         cptr.assign(nclass + 1, 0);
         for (int c = 0; c < nclass; ++c) cptr[c + 1] = cptr[c] + op->hrp[rep[c] + 1] - op->hrp[rep[c]];
-        struct Up { // device copies of rep and cptr
-            int *rep = nullptr, *cptr = nullptr;
-            ~Up() { dfree(rep); dfree(cptr); }
-        } up;
-        if ((rc = upload(&up.rep, rep, st)) || (rc = upload(&up.cptr, cptr, st))) return rc;
-        HIPCHK(launch_fill_zero(tmp.flags, 4 * sizeof(int), st));
-        HIPCHK(hipMemcpyAsync(tmp.key, cls.data(), sizeof(int) * n, hipMemcpyHostToDevice, st));
-        HIPCHK(launch_grid_check(n, op->rp, op->ci, op->v64, (size_t)op->nnz, m == GRID_CLASS ? 0 : 1, tmp.key, up.rep,
-                                 tmp.flags, st));
-        HIPCHK(launch_grid_sort(g, m, op->rp, tmp.key, up.cptr, P.rows, P.cls, P.slice, P.smax, st));
-        HIPCHK(hipMemcpyAsync(f, tmp.flags, sizeof f, hipMemcpyDeviceToHost, st));
+        packed = cls;
+        packed.insert(packed.end(), rep.begin(), rep.end());
+        packed.insert(packed.end(), cptr.begin(), cptr.end());
+        int *const drep = tmp.key + n, *const dcptr = drep + nclass;
+        HIPCHK(launch_fill_zero(flags, 4 * sizeof(int), st));
+        HIPCHK(hipMemcpyAsync(tmp.key, packed.data(), sizeof(int) * packed.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(launch_grid_check(n, op->rp, op->ci, op->v64, (size_t)op->nnz, m == GRID_CLASS ? 0 : 1, tmp.key, drep,
+                                 flags, st));
+        HIPCHK(launch_grid_sort(g, m, op->rp, tmp.key, dcptr, P.rows, P.cls, P.slice, P.smax, st));
         HIPCHK(hipMemcpyAsync(keys.data(), P.cls, sizeof(int) * keys.size(), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-        if (f[0] == 0 && patch_tables(g, cptr, rep, keys, toff, tlen, trep, tdst, &P.nentries)) mode = m;
+        if (keys[nrows] == 0 && patch_tables(g, cptr, rep, keys, toff, tlen, trep, tdst, &P.nentries)) mode = m;
     }
     P.mode = mode;
     if (mode == GRID_ROWS) {
@@ -563,10 +564,13 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
         HIPCHK(launch_grid_sort(g, mode, op->rp, tmp.key, nullptr, P.rows, P.cls, P.slice, P.smax, st));
     } else {
         P.nitems = (int)trep.size();
-        HIPCHK(hipMemcpyAsync(P.cls, keys.data(), sizeof(int) * keys.size(), hipMemcpyHostToDevice, st));
-        if ((rc = upload(&P.toff, toff, st)) || (rc = upload(&P.tlen, tlen, st)) || (rc = upload(&P.trep, trep, st)) ||
-            (rc = upload(&P.tdst, tdst, st)))
-            return rc;
+        HIPCHK(hipMemcpyAsync(P.cls, keys.data(), sizeof(int) * nrows, hipMemcpyHostToDevice, st));
+        packed = toff;
+        for (const std::vector<int> *v : {&tlen, &trep, &tdst}) packed.insert(packed.end(), v->begin(), v->end());
+        if ((rc = upload(&P.toff, packed, st))) return rc;
+        P.tlen = P.toff + toff.size();
+        P.trep = P.tlen + tlen.size();
+        P.tdst = P.trep + trep.size();
     }
     P.g = g;
     HIPCHK(launch_grid_place(g, P.rows, P.cls, st));
