@@ -301,10 +301,11 @@ hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, size_
 // dst[c][i][s] = srcs[min(s, nsrc-1)][c*n + i] for c < ncoef, i < n, s < S; elem = 4 or 8 bytes
 hipError_t launch_pack_per_shot(const void *const *srcs_dev, int nsrc, int ncoef, int n, int S, int elem,
                                 void *dst, hipStream_t st);
-hipError_t launch_elastic_apply(int n, const int *rp, const int *ci, const double *A, size_t nnz,
-                                const double *coef, const int *flag, const double *x, double *y,
-                                double *sumsq, hipStream_t st);
-hipError_t launch_scale(size_t n, double *x, const double *sumsq, hipStream_t st);
+hipError_t launch_elastic_slices(int n, const int *rp, const int *ci, const double *A, size_t nnz, const int *off,
+                                 size_t nslots, int *cols, double *vals, hipStream_t st);
+hipError_t launch_elastic_apply(int n, const int *rp, const int *off, size_t nslots, const int *cols,
+                                const double *vals, const double *coef, const int *flag, const double *x,
+                                const double *xsumsq, double *y, double *sumsq, hipStream_t st);
 hipError_t launch_stream_copy(const void *src, void *dst, size_t n16, hipStream_t st);
 
 } // namespace sfg
