@@ -149,10 +149,10 @@ constexpr int BK = 64, LDK = BK + 8;
 // weights and moments of EPI_ADAM carry the streaming (nontemporal) hint (a template
 // parameter too: a run-time choice between the two kinds of access is merged into the
 // plain one).
-template <int BM, int BN, int NW, int WN, int KIND, bool TB = false, bool STREAM = false>
-__global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, int kchunk, const uint16_t *__restrict__ A,
-                                                      int lda, const uint16_t *__restrict__ B, int ldb,
-                                                      float *__restrict__ C, int ldc, const EpiArgs ep)
+template <int BM, int BN, int NW, int WN, int KIND, bool TB, bool STREAM>
+__device__ __forceinline__ void gemm_nt_tile(int bx, int by, int bz, int nz, int M, int N, int K, int kchunk,
+                                             const uint16_t *__restrict__ A, int lda, const uint16_t *__restrict__ B,
+                                             int ldb, float *__restrict__ C, int ldc, const EpiArgs &ep)
 {
     constexpr int WM = NW / WN;                         // waves along M and N
     constexpr int TM = BM / WM / 32, TN = BN / WN / 32; // 32 x 32 tiles per wave
@@ -165,9 +165,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WN, wn = wave % WN;
     if constexpr (KIND == EPI_MSE)
-        for (int i = tid; i < BM; i += NW * 64) Ti[i] = ep.tidx[min((int)blockIdx.y * BM + i, M - 1)];
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
+        for (int i = tid; i < BM; i += NW * 64) Ti[i] = ep.tidx[min(by * BM + i, M - 1)];
+    const int m0 = by * BM, n0 = bx * BN;
+    const int kb = bz * kchunk, ke = min(K, kb + kchunk);
     f32x16 acc[TM][TN];
 #pragma unroll
     for (int a = 0; a < TM; ++a)
@@ -322,8 +322,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
     // row of register r in a tile whose lane rows start at rb
 #define SFG_ROW(r) (rb + ((r) >> 2) * 8 + ((r) & 3))
     if constexpr (KIND == EPI_STORE)
-        if (gridDim.z > 1) C += (size_t)blockIdx.z * ep.slice;
-    if (KIND == EPI_STORE && gridDim.z > 1 && ep.slice == 0) {
+        if (nz > 1) C += (size_t)bz * ep.slice;
+    if (KIND == EPI_STORE && nz > 1 && ep.slice == 0) {
         tiles([&](const f32x16 &t, int col, int rb) __attribute__((always_inline)) {
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -534,6 +534,39 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
         });
     }
 #undef SFG_ROW
+}
+
+template <int BM, int BN, int NW, int WN, int KIND, bool TB = false, bool STREAM = false>
+__global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, int kchunk, const uint16_t *__restrict__ A,
+                                                      int lda, const uint16_t *__restrict__ B, int ldb,
+                                                      float *__restrict__ C, int ldc, const EpiArgs ep)
+{
+    gemm_nt_tile<BM, BN, NW, WN, KIND, TB, STREAM>(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z, M, N, K, kchunk, A,
+                                                   lda, B, ldb, C, ldc, ep);
+}
+
+// Several products with the Adam step (64 x 64 tiles) in one launch: block b takes a tile
+// of the product whose blocks first .. hold it.  The dW of the hidden layers, each too
+// small to fill the chip for longer than a launch takes.
+struct AdamProduct {
+    int M, N, K, first, gx, lda, ldb, ldc;
+    const uint16_t *A, *B;
+    float *C;
+    EpiArgs ep;
+};
+struct AdamGroup {
+    static constexpr int MOST = 6;
+    int count;
+    AdamProduct p[MOST];
+};
+__global__ __launch_bounds__(256) void gemm_adam_group_kernel(const AdamGroup g)
+{
+    int i = 0;
+    while (i + 1 < g.count && (int)blockIdx.x >= g.p[i + 1].first) ++i;
+    const AdamProduct &p = g.p[i];
+    const int b = (int)blockIdx.x - p.first;
+    gemm_nt_tile<64, 64, 4, 2, EPI_ADAM, false, false>(b % p.gx, b / p.gx, 0, 1, p.M, p.N, p.K, p.K, p.A, p.lda, p.B,
+                                                       p.ldb, p.C, p.ldc, p.ep);
 }
 
 // C[r][c] = 0 for r < rows, c < cols (row stride ld)
@@ -829,12 +862,24 @@ GemmShape gemm_shape(int M, int N, int K, int kind)
     return g;
 }
 
+// sizes and strides that the products take; for EPI_ADAM also that the row-piece epilogue
+// applies: 16-byte rows of C (unused), W and its moments
+bool products_ok(int M, int N, int K, int lda, int ldb, const float *C, int ldc, const EpiArgs &ep)
+{
+    if (K % 8 || lda % 8 || ldb % 8 || M <= 0 || N <= 0 || K <= 0) return false;
+    if (ep.kind != EPI_ADAM) return true;
+    auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    return !(N % 4 || ldc % 4 || !a16(C) || !ep.W || !a16(ep.W) || !ep.Mw || !a16(ep.Mw) || !ep.Vw || !a16(ep.Vw) ||
+             !ep.W16 || (reinterpret_cast<uintptr_t>(ep.W16) & 7) || ep.H || ep.arows < 1 || ep.arows > M ||
+             ep.acols < 1 || ep.acols > N);
+}
+
 // C = A . B^T with the epilogue ep.  A product split over K adds its partial
 // products into C: zeroed here first, unless the caller has (zeroed).
 hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda, const uint16_t *B, int ldb, float *C,
                 int ldc, const EpiArgs &ep, bool tb = false, bool zeroed = false)
 {
-    if (K % 8 || lda % 8 || ldb % 8 || M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
+    if (!products_ok(M, N, K, lda, ldb, C, ldc, ep)) return hipErrorInvalidValue;
     if (tb && (N % 8 || ep.kind != EPI_STORE)) return hipErrorInvalidValue;
     if (ep.kind == EPI_MSE && !ep.H) return hipErrorInvalidValue;
     if (ep.HT) {
@@ -845,14 +890,6 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
             return hipErrorInvalidValue;
     }
     if (ep.stream && ep.kind != EPI_ADAM) return hipErrorInvalidValue;
-    if (ep.kind == EPI_ADAM) {
-        // the row-piece epilogue must apply: 16-byte rows of C (unused), W and its moments
-        auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-        if (N % 4 || ldc % 4 || !a16(C) || !ep.W || !a16(ep.W) || !ep.Mw || !a16(ep.Mw) || !ep.Vw || !a16(ep.Vw) ||
-            !ep.W16 || (reinterpret_cast<uintptr_t>(ep.W16) & 7) || ep.H || ep.arows < 1 || ep.arows > M ||
-            ep.acols < 1 || ep.acols > N)
-            return hipErrorInvalidValue;
-    }
     const GemmShape gs = gemm_shape(M, N, K, ep.kind);
     if (ep.db) {
         // the row-piece loss epilogue must apply, in blocks that hold every row
@@ -891,6 +928,13 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
     }
 #undef SFG_GEMM_TILES
 #undef SFG_GEMM
+    return hipGetLastError();
+}
+
+hipError_t launch_group(hipStream_t st, AdamGroup &g, int blocks)
+{
+    hipLaunchKernelGGL(gemm_adam_group_kernel, dim3(blocks), dim3(256), 0, st, g);
+    g.count = 0;
     return hipGetLastError();
 }
 
@@ -1191,7 +1235,13 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
     // element by element costs as much as the products at this small K).  With ad the
     // Adam step is in the product's epilogue (the gradient is never stored), which writes
     // the bf16 weights to W16.
-    auto weights = [&](hipStream_t st, int l) {
+    // Those of the hidden layers are collected and launched together (13 x 1024 and two of
+    // 1024 x 1024: one launch instead of three; with 32000 outputs, batch 256, 0.338 -> 0.327 ms
+    // per step, with 8000 0.198 -> 0.189, 512 wide 0.166 -> 0.153).
+    AdamGroup group;
+    group.count = 0;
+    int blocks = 0;
+    auto weights = [&](hipStream_t st, int l) -> hipError_t {
         EpiArgs ep;
         if (ad) {
             ep.kind = EPI_ADAM;
@@ -1204,7 +1254,20 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
             ep.stream = streams(m, l);
             ep.ad = *ad;
         }
-        return gemm(st, m->pout[l], m->pin[l], B, m->dzT16[l], B, m->hT16[l], B, m->G[l], m->pin[l], ep, false, zw[l]);
+        const int M = m->pout[l], N = m->pin[l];
+        if (l < m->nl - 1 && ad && !ep.stream) { // collected
+            if (!products_ok(M, N, B, B, B, m->G[l], N, ep)) return hipErrorInvalidValue;
+            if (group.count == AdamGroup::MOST) {
+                const hipError_t e = launch_group(st, group, blocks);
+                if (e != hipSuccess) return e;
+            }
+            if (group.count == 0) blocks = 0;
+            group.p[group.count++] = AdamProduct{M, N, B, blocks, (N + 63) / 64, B, B, N, m->dzT16[l], m->hT16[l],
+                                                 m->G[l], ep};
+            blocks += ((N + 63) / 64) * ((M + 63) / 64);
+            return hipSuccess;
+        }
+        return gemm(st, M, N, B, m->dzT16[l], B, m->hT16[l], B, m->G[l], N, ep, false, zw[l]);
     };
     const int L = m->nl - 1;
     if (!m->out_db) { // (else formed in the forward pass's loss epilogue)
@@ -1256,6 +1319,7 @@ static int backward(sfg_mlp *m, const AdamArgs *ad = nullptr)
         }
         if (!(l == L && over)) MCHK(weights(m->st, l));
     }
+    if (group.count) MCHK(launch_group(m->st, group, blocks));
     return SFG_OK;
 }
 
