@@ -616,6 +616,8 @@ static int grid_plan(const sfg_operator *op, int most, int align, bool f32, hipS
         const void *v = f32 ? (const void *)op->v32 : (const void *)op->v64;
         int rc;
         char *tv = nullptr, *mv = nullptr;
+        dfree(P->tab[k]); // (of an attempt that ran out of memory)
+        dfree(P->mval[k]);
         if ((rc = dalloc(&tv, (size_t)P->nentries * 8 * w))) return rc;
         P->tab[k] = tv;
         if (P->mode != GRID_CLASS) {
@@ -960,8 +962,8 @@ static int capture_graph(hipStream_t st, hipGraphExec_t *out, F launches)
     return rc;
 }
 
-static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medium *const *media, int nmedia,
-                           const sfg_shot_desc *d)
+static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium *const *media, int nmedia,
+                         const sfg_shot_desc *d, bool grid)
 {
     g_err.clear();
     if (!out || !op || !media || nmedia <= 0 || !d) return fail(SFG_E_ARG, "run: bad arguments");
@@ -1021,7 +1023,7 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     }
     // lane grouping: shots per lane group and the padded shot stride
     int sp = d->shots_per_lane_group;
-    if (n < 1 << 28 && grid_default(op, d)) {
+    if (grid && n < 1 << 28 && grid_default(op, d)) {
         int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan);
         if (rc) {
             run_free(r);
@@ -1572,6 +1574,18 @@ static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medi
     return SFG_OK;
 }
 
+// (the grid layout's tables and padded lines may need more memory than lane groups do)
+static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medium *const *media, int nmedia,
+                           const sfg_shot_desc *d)
+{
+    int rc = run_create_as(out, op, media, nmedia, d, true);
+    if (rc == SFG_E_NOMEM) {
+        (void)hipGetLastError();
+        rc = run_create_as(out, op, media, nmedia, d, false);
+    }
+    return rc;
+}
+
 extern "C" int sfg_run_create(sfg_run **out, const sfg_operator *op, const sfg_medium *md,
                               const sfg_shot_desc *d)
 {
@@ -1818,7 +1832,7 @@ extern "C" int sfg_estimate_dt(const sfg_operator *op, const sfg_medium *md, int
     }
     // (a few rows far longer than the others would pad the slices to many times the matrix:
     // such an operator is read in the order of its CSR arrays)
-    const bool sliced = nslots * 64 <= 4 * (size_t)op->nnz;
+    bool sliced = nslots * 64 <= 4 * (size_t)op->nnz;
     struct Tmp { // device memory of this call
         double *x = nullptr, *y = nullptr, *sums = nullptr, *vals = nullptr;
         int *off = nullptr, *cols = nullptr;
@@ -1827,10 +1841,16 @@ extern "C" int sfg_estimate_dt(const sfg_operator *op, const sfg_medium *md, int
     int rc = dalloc(&t.x, n2);
     if (!rc) rc = dalloc(&t.y, n2);
     if (!rc) rc = dalloc(&t.sums, 2 * most + 1);
-    if (!rc && sliced) rc = dalloc(&t.vals, 4 * nslots * 64);
-    if (!rc && sliced) rc = dalloc(&t.off, off.size());
-    if (!rc && sliced) rc = dalloc(&t.cols, nslots * 64);
     if (rc) return rc;
+    if (sliced && (dalloc(&t.vals, 4 * nslots * 64) || dalloc(&t.cols, nslots * 64) || dalloc(&t.off, off.size()))) {
+        // no room for the copy
+        (void)hipGetLastError();
+        g_err.clear();
+        dfree(t.vals);
+        dfree(t.cols);
+        dfree(t.off);
+        sliced = false;
+    }
     double *x = t.x, *y = t.y, *sums = t.sums;
     const double one = 1.0;
     hipError_t e = hipMemcpy(x, x0.data(), sizeof(double) * n2, hipMemcpyHostToDevice);

@@ -16,8 +16,8 @@ std::shared_ptr<Staging> staging();
 // stream st, complete on return.
 //
 // A fresh host array costs a page fault per 4 KB when it is first written, more than
-// its transfer: 131 MB took 42 ms as a copy into a staging vector and from there into
-// the array (32-45 ms copied there directly), and takes 7 ms here, where 8 threads
+// its transfer: 140 MB in four arrays took 42 ms as copies into staging vectors and from there
+// into the arrays (32-45 ms copied there directly), and take 12 ms here, where 8 threads
 // each copy what the DMA engine has put into their pinned buffers (1000 predictions of
 // 32000 samples, all told: 16.5 ms then, 5.7 ms now).  Below 4 MB, where
 // starting the threads costs as much, and without pinned memory the copy is direct.

@@ -77,8 +77,13 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
     if (!staging || width * rows < kDirect) return direct(to, from, pitch, width, rows, map, st);
     std::lock_guard<std::mutex> lk(staging->mu);
     char *buf = staging->get();
-    int device = 0;
-    if (!buf || hipGetDevice(&device) != hipSuccess) return direct(to, from, pitch, width, rows, map, st);
+    // the stream's device, which need not be the caller's
+    hipDevice_t device = 0;
+    int callers = 0;
+    if (!buf || hipStreamGetDevice(st, &device) != hipSuccess || hipGetDevice(&callers) != hipSuccess) {
+        (void)hipGetLastError();
+        return direct(to, from, pitch, width, rows, map, st);
+    }
 
     // pieces: parts of a row, or several whole rows
     const size_t per_row = (width + kPiece - 1) / kPiece, per_piece = per_row > 1 ? 1 : kPiece / width;
@@ -140,6 +145,7 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
     }
     work(0);
     for (int q = 1; q < started; ++q) th[q].join();
+    if (callers != device) (void)hipSetDevice(callers);
     const hipError_t e2 = hipStreamSynchronize(st);
     const hipError_t e = (hipError_t)error.load();
     return e != hipSuccess ? e : e2;
