@@ -545,6 +545,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_kernel(int M, int N, int K, i
                                                    lda, B, ldb, C, ldc, ep);
 }
 
+// EPI_ADAM of a layer that streams (STREAM).  Three waves per SIMD at most: its rate is that
+// of the memory with three blocks per CU as with four (180 us for 32000 x 1024), and the fourth
+// place, registers and LDS of a 64 x 64 block, is free for the products that run beside it,
+// which else wait for a block to end (training step, batch 64 / 256 / 512: 0.246 / 0.328 /
+// 0.469 -> 0.239 / 0.322 / 0.455 ms).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void gemm_adam_stream_kernel(
+    int M, int N, int K, int kchunk, const uint16_t *__restrict__ A, int lda, const uint16_t *__restrict__ B, int ldb,
+    float *__restrict__ C, int ldc, const EpiArgs ep)
+{
+    gemm_nt_tile<64, 64, 4, 2, EPI_ADAM, false, true>(blockIdx.x, blockIdx.y, 0, 1, M, N, K, kchunk, A, lda, B, ldb, C,
+                                                      ldc, ep);
+}
+
 // Several products with the Adam step (64 x 64 tiles) in one launch: block b takes a tile
 // of the product whose blocks first .. hold it.  The dW of the hidden layers, each too
 // small to fill the chip for longer than a launch takes.
@@ -669,8 +682,10 @@ __global__ void gather_rows_kernel(int batch, int width, int ld, const float *sr
 // What is left is the latency of the loads on a quarter of the chip.  HR = 256 (1024
 // threads, one pass for a batch of 256) is the faster form alone (13 us with HR = 64);
 // beside a kernel that fills the chip such a block waits for a whole CU to drain (150 us),
-// and HR = 64 (256 threads) starts in any free slot (20 to 30 us).
-constexpr int HC = 16, HLD = HC + 1, HP = 8;
+// and HR = 64 (256 threads) starts in any free slot (20 to 30 us).  HP parts are in flight per
+// pass: with 8 the kernel's 106 registers did not fit beside three blocks of the output
+// layer's step (below), with 4 its 72 do (also alone no slower).
+constexpr int HC = 16, HLD = HC + 1, HP = 4;
 template <bool BACK, int HR>
 __global__ __launch_bounds__(4 * HR) void hidden_kernel(int rows, int cols, int valid, const float *__restrict__ parts,
                                                     int nparts, size_t slice, float *__restrict__ z,
@@ -919,7 +934,8 @@ hipError_t gemm(hipStream_t st, int M, int N, int K, const uint16_t *A, int lda,
     case EPI_BIAS_GELU: SFG_GEMM_TILES(EPI_BIAS_GELU); break;
     case EPI_MSE: SFG_GEMM_TILES(EPI_MSE); break;
     case EPI_ADAM:
-        if (ep.stream) SFG_GEMM(64, 64, 4, 2, EPI_ADAM, false, true);
+        if (ep.stream)
+            hipLaunchKernelGGL(gemm_adam_stream_kernel, g, dim3(256), 0, st, M, N, K, kchunk, A, lda, B, ldb, C, ldc, ep);
         else SFG_GEMM(64, 64, 4, 2, EPI_ADAM);
         break;
     default:
