@@ -1022,7 +1022,6 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
         return fail(SFG_E_HIP, "run setup: %s", hipGetErrorString(es));
     }
     // lane grouping: shots per lane group and the padded shot stride
-    int sp = d->shots_per_lane_group;
     if (grid && n < 1 << 28 && grid_default(op, d)) {
         int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan);
         if (rc) {
@@ -1034,11 +1033,10 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
     }
     int variant = d->kernel_variant, xcd = d->xcd_remap;
     if (!r->plan) batched_default(op, d, nmedia > 1, &variant, &xcd);
-    if (r->plan) {
-        sp = 1;
-        r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
-    }
-    if (sp == 0) sp = d->nshots <= 1 ? 1 : d->nshots <= 4 ? 4 : d->nshots <= 16 ? 16 : 64;
+    if (r->plan) r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
+    const int lanes =
+        d->shots_per_lane_group ? d->shots_per_lane_group : d->nshots <= 1 ? 1 : d->nshots <= 4 ? 4 : d->nshots <= 16 ? 16 : 64;
+    const int sp = r->plan ? 1 : lanes;
     if (sp != 1 && sp != 4 && sp != 16 && sp != 32 && sp != 64) {
         run_free(r);
         return fail(SFG_E_ARG, "run: shots_per_lane_group must be 1, 4, 16, 32 or 64");
@@ -1052,7 +1050,9 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
         run_free(r);
         return fail(SFG_E_ARG, "run: node_num * padded shots must stay below 2^31");
     }
-    r->block = d->block > 0 ? d->block : (sp == 1 && n < 256 * 1024 ? 64 : 256);
+    // (the grid layout's steps take the patches' own blocks: its runs keep the block of
+    // their lane groups, which multi-runs compare)
+    r->block = d->block > 0 ? d->block : (lanes == 1 && n < 256 * 1024 ? 64 : 256);
     if (r->block % 64 != 0 || r->block > 256) {
         run_free(r);
         return fail(SFG_E_ARG, "run: block must be 64, 128, 192 or 256 threads (kernel launch bound)");
