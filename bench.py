@@ -380,11 +380,13 @@ def main():
         models = workloads.config4b(step_range=step_range)
         log(f"multi-model setup {time.time() - t_m:.1f}s: sizes {[c['size'] for c in models]}")
         keep, runs = [], []
-        # the multi-run kernel takes lane groups of 1, 32 or 64 shots; a lane's arithmetic does
-        # not depend on the grouping, so part 1 stays bit-identical to the single run
+        # part 1 in the launch of the single run (the library's own, 0, included); explicit
+        # groups of fewer than 32 shots as groups of 64, the smallest that share a launch.  A
+        # lane's arithmetic does not depend on the grouping, so part 1 stays bit-identical
         sp1 = kw.get("shots_per_lane_group", 64)
+        block = kw.get("block") or 256
         part1 = gpu.Run(op, md, case["src"], L, case["rec"], precision=prec, nsteps=nsteps,
-                        **dict(kw, shots_per_lane_group=sp1 if sp1 in (32, 64) else 64))
+                        **dict(kw, block=block, shots_per_lane_group=sp1 if sp1 in (0, 32, 64) else 64))
         runs.append(part1)
         for c in models:
             p = c["problem"]
@@ -394,7 +396,7 @@ def main():
             # single-shot models in the sliced layout (round-robin tiles), stepped by a
             # launch of single-shot forms of their own, after part 1's own step launch
             runs.append(gpu.Run(mop, mmd, c["src"], L, c["rec"], c["dt"], c["f0"], c["t0"], precision=prec,
-                                nsteps=c["nsteps"], block=kw.get("block", 256), shots_per_lane_group=1,
+                                nsteps=c["nsteps"], block=block, shots_per_lane_group=1,
                                 kernel_variant=8, xcd_remap=False))
         grp = gpu.Multi(runs)
         grp.advance(L)
@@ -434,7 +436,7 @@ def main():
         # schedule (cooperative launch per guard interval, tile queues, grid barrier)
         def part2_runs():
             return [gpu.Run(keep[2 * qi], keep[2 * qi + 1], c["src"], L, c["rec"], c["dt"], c["f0"], c["t0"],
-                            precision=prec, nsteps=c["nsteps"], block=kw.get("block", 256), shots_per_lane_group=1,
+                            precision=prec, nsteps=c["nsteps"], block=block, shots_per_lane_group=1,
                             kernel_variant=8, xcd_remap=False) for qi, c in enumerate(models)]
         best_s, tab_s = autotune.tune_multi_schedule(part2_runs, steps=min(300, L // 2), log=log)
         multi["part2_schedule"] = {"ms_per_step": {("per_step" if k == 0 else f"persistent_{k}_per_cu"): ms

@@ -32,8 +32,10 @@ def candidates(nshots, nodes=160801, patches=False):
         return dict(shots_per_lane_group=sp, block=block, kernel_variant=variant, xcd_remap=xcd, row_order=order,
                     sell_sigma=sigma)
 
-    # the library's own choice (the grid layout on meshes numbered line by line)
-    own = [c(0, 0, 0, True, "node")]
+    # the library's own choice (the grid layout on meshes numbered line by line), with the
+    # block named: it leaves the choice as it is, and a multi-run takes runs of one block,
+    # which the library picks by shots and mesh size where it is left out
+    own = [c(0, 256, 0, True, "node")]
     if nshots <= 1:
         # one row per lane: per-row layouts, the sliced layout (8) and, on meshes
         # with a line structure, the sliced layout with LDS-staged halos over

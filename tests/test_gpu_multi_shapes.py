@@ -85,3 +85,19 @@ def test_default_shapes_share_a_multi_run(prec, specs):
     assert_same(seismograms(makers, True), seismograms(makers, False))
     for h in keep:
         h.close()
+
+
+@pytest.mark.parametrize("shots", [1, 3, 64])
+def test_tuned_launch_shares_a_multi_run_with_sliced_models(shots):
+    """A launch the tuner returns names its block: runs of it go into one multi-run
+    with single-shot models that take the same block."""
+    from seisfem_amd import autotune
+    own = autotune.run_kwargs(dict(autotune.candidates(shots)[0], row_order=None, row_order_name="node"))
+    assert own["shots_per_lane_group"] == 0 and own["kernel_variant"] == 0
+    say(f"the library's own launch of {shots} shots beside sliced models")
+    model = dict(block=own["block"], shots_per_lane_group=1, kernel_variant=8, xcd_remap=False)
+    keep, makers = make_runs([(host.Q4, 30, 41, shots, False, own), (host.Q4, 20, 23, 1, False, model),
+                              (host.Q9, 9, 8, 1, False, model)], gpu.FP32_KAHAN16, 40)
+    assert_same(seismograms(makers, True), seismograms(makers, False))
+    for h in keep:
+        h.close()
