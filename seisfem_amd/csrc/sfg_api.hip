@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1928,7 +1929,7 @@ struct sfg_multi {
     // persistent schedule (sfg_multi_set_persistent): resident blocks of one
     // cooperative launch per guard interval, or 0 for the per-step launches
     int persist_blocks = 0;
-    const MultiGroup *persist = nullptr;
+    const MultiGroup *persist = nullptr; // grp[1] or mixed (single-shot runs only), or grp[0] beside grid[]
     bool persist_single = false; // only single-shot runs
     int *queue = nullptr;       // device int[16]: tile queues by step parity and XCD
     hipStream_t stream = nullptr;
@@ -2116,6 +2117,21 @@ extern "C" int sfg_multi_create(sfg_multi **out, sfg_run *const *runs, int nruns
     return SFG_OK;
 }
 
+// Whether a batched run in the grid layout is too small to fill the GPU alone, as its
+// 64-shot lane groups would be (see sfg_multi_create)
+static bool small_batch(const sfg_run *r)
+{
+    return r->nshots > 16 && (long long)((r->op->n + 3) / 4) * ((r->nshots + 63) / 64) < 256;
+}
+
+// LDS of the persistent launch of a group of grid runs (fields staged in two parts)
+static size_t persistent_lds(const sfg_multi *m, const MultiGroup &g)
+{
+    size_t lds = 0;
+    for (const sfg_run *r : g.runs) lds = std::max(lds, grid_lds_bytes(r->plan->g, false, m->prec == 0 ? 8 : 4));
+    return lds;
+}
+
 extern "C" int sfg_multi_advance(sfg_multi *m, int nsteps)
 {
     g_err.clear();
@@ -2124,12 +2140,22 @@ extern "C" int sfg_multi_advance(sfg_multi *m, int nsteps)
     const int steps = todo;
     HIPCHK(hipEventRecord(m->ev0, m->stream));
     while (todo > 0 && m->persist_blocks > 0) {
-        // one cooperative launch up to the next guard
+        // one cooperative launch (one per patch size of batched grid runs) up to the next guard
         const MultiGroup &g = *m->persist;
         const int seg = std::min(todo, m->guard_every - m->executed % m->guard_every);
-        HIPCHK(launch_multi_persistent(m->prec, g.args, g.tile_start, (int)g.runs.size(), g.ntiles, m->block,
-                                       m->persist_blocks, m->executed & 1, seg, m->queue, m->persist_single,
-                                       m->stream));
+        const MultiGroup *last = !g.runs.empty() ? &g : nullptr;
+        if (!m->persist_single)
+            for (const MultiGroup &x : m->grid)
+                if (!x.runs.empty() && last != &g) last = &x;
+        for (const MultiGroup &x : m->grid)
+            if (!m->persist_single && !x.runs.empty())
+                HIPCHK(launch_grid_persistent(m->prec, x.args, x.tile_start, (int)x.runs.size(), x.ntiles,
+                                              x.runs[0]->plan->g.most, m->persist_blocks, m->executed & 1, seg,
+                                              persistent_lds(m, x), last == &x, m->stream));
+        if (last == &g)
+            HIPCHK(launch_multi_persistent(m->prec, g.args, g.tile_start, (int)g.runs.size(), g.ntiles, m->block,
+                                           m->persist_blocks, m->executed & 1, seg, m->queue, m->persist_single,
+                                           m->stream));
         m->executed += seg;
         todo -= seg;
         if (m->executed % m->guard_every == 0 || m->executed == m->max_steps) {
@@ -2175,25 +2201,29 @@ extern "C" int sfg_multi_set_persistent(sfg_multi *m, int blocks_per_cu)
         m->persist_blocks = 0;
         return SFG_OK;
     }
-    // the runs of one shared launch: batched runs only, or single-shot runs in the
-    // per-row, sliced and grid layouts (the last in their per-row form)
-    const MultiGroup *g = nullptr;
-    bool ok = m->solo.empty() && m->grp[2].runs.empty();
-    bool grid = false;
+    // single-shot runs in the per-row, sliced and grid layouts (the last in their per-row
+    // form), in one launch; or batched runs too small to fill the GPU alone, those in lane
+    // groups in one launch, those in the grid layout in one per patch size
+    bool ok = m->solo.empty() && m->grp[2].runs.empty(), singles = !m->grp[1].runs.empty(), grid = false;
+    bool batches = !m->grp[0].runs.empty();
     for (const MultiGroup &q : m->grid)
         for (const sfg_run *r : q.runs) {
             grid = true;
-            ok = ok && r->S == 1;
+            (r->S == 1 ? singles : batches) = true;
+            ok = ok && (r->S == 1 || small_batch(r));
         }
-    if (ok && m->grp[1].runs.empty() && !grid) g = &m->grp[0];
-    else if (ok && m->grp[0].runs.empty()) g = grid ? &m->mixed : &m->grp[1];
-    else ok = false;
-    if (!ok)
-        return fail(SFG_E_ARG, "multi persistent: needs every run in one shared launch (single-shot runs in the "
-                               "per-row, sliced or grid layouts, or batched runs too small to fill the GPU alone)");
-    const bool single = g != &m->grp[0];
-    int per_cu = 0, dev = 0, cus = 0;
-    HIPCHK(multi_persistent_blocks_per_cu(m->prec, single, m->block, &per_cu));
+    if (!ok || singles == batches)
+        return fail(SFG_E_ARG, "multi persistent: needs single-shot runs in the per-row, sliced or grid layouts only, "
+                               "or batched runs too small to fill the GPU alone only");
+    const MultiGroup *g = batches ? &m->grp[0] : grid ? &m->mixed : &m->grp[1];
+    int per_cu = INT_MAX, dev = 0, cus = 0, q = 0;
+    if (singles || !g->runs.empty()) HIPCHK(multi_persistent_blocks_per_cu(m->prec, singles, m->block, &per_cu));
+    for (const MultiGroup &x : m->grid)
+        if (batches && !x.runs.empty()) {
+            if (persistent_lds(m, x) > 65536) HIPCHK(allow_grid_lds());
+            HIPCHK(grid_persistent_blocks_per_cu(m->prec, x.runs[0]->plan->g.most, persistent_lds(m, x), &q));
+            per_cu = std::min(per_cu, q);
+        }
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     if (blocks_per_cu > per_cu)
@@ -2215,7 +2245,7 @@ extern "C" int sfg_multi_set_persistent(sfg_multi *m, int blocks_per_cu)
         }
     }
     m->persist = g;
-    m->persist_single = single;
+    m->persist_single = singles;
     m->persist_blocks = blocks_per_cu * cus;
     return SFG_OK;
 }

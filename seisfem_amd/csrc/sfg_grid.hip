@@ -2,6 +2,8 @@
 // patches with the neighbours' fields in LDS and the matrices as stencil classes
 // (see GridArgs).  Same arithmetic per row as step_tile (sfg_kernels.hip): every
 // sum runs in column order, and the FPB4 form is bit-identical to the reference.
+#include <hip/hip_cooperative_groups.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -666,23 +668,17 @@ hipError_t launch_grid_step(int precision, bool cps, const void *sa, const void 
 #undef SFG_GS
 }
 
-// Several grid-layout runs in one launch per step (see multi_step_kernel): a
-// run's tiles are its (patch, shot) pairs, patches fastest.
+// One tile of a multi-run's grid launch: a run's tiles are its (patch, shot) pairs,
+// patches fastest.
 template <class T, int PREC, bool TOG>
-__global__ __launch_bounds__(GRID_BLOCK) void multi_grid_kernel(const GridRun<T> *__restrict__ runs,
-                                                                const int *__restrict__ tile_start, int nruns,
-                                                                int xcd_remap, int slot)
+__device__ __forceinline__ void multi_grid_tile(const GridRun<T> *__restrict__ runs, const int *__restrict__ tile_start,
+                                                int nruns, int t, int slot, int tile)
 {
-    const int t = begin_step(runs[0].a.ctrl, slot);
-    const unsigned int nb = gridDim.x;
-    unsigned int bid = blockIdx.x;
-    if (xcd_remap > 1) bid = xcd_striped(bid, nb, (unsigned int)(xcd_remap - 1));
-    else if (xcd_remap) bid = xcd_contiguous(bid, nb);
     int r = 0;
-    while (r + 1 < nruns && (int)bid >= tile_start[r + 1]) ++r;
+    while (r + 1 < nruns && tile >= tile_start[r + 1]) ++r;
     const StepArgs<T> &a = runs[r].a;
     const GridArgs<T> &g = runs[r].g;
-    const int local = (int)bid - tile_start[r], s = local / g.g.npatch, patch = local - s * g.g.npatch;
+    const int local = tile - tile_start[r], s = local / g.g.npatch, patch = local - s * g.g.npatch;
     if (a.S > 1 && s >= (t < a.nsteps_max ? ro(a.active)[t] : 0)) return;
 #define SFG_GT(C, M) grid_tile<T, PREC, C, M, TOG>(a, g, t, slot, patch, s, false)
     if (a.cps) {
@@ -695,6 +691,74 @@ __global__ __launch_bounds__(GRID_BLOCK) void multi_grid_kernel(const GridRun<T>
         else SFG_GT(false, GRID_ROWS);
     }
 #undef SFG_GT
+}
+
+// Several grid-layout runs in one launch per step (see multi_step_kernel).
+template <class T, int PREC, bool TOG>
+__global__ __launch_bounds__(GRID_BLOCK) void multi_grid_kernel(const GridRun<T> *__restrict__ runs,
+                                                                const int *__restrict__ tile_start, int nruns,
+                                                                int xcd_remap, int slot)
+{
+    const int t = begin_step(runs[0].a.ctrl, slot);
+    const unsigned int nb = gridDim.x;
+    unsigned int bid = blockIdx.x;
+    if (xcd_remap > 1) bid = xcd_striped(bid, nb, (unsigned int)(xcd_remap - 1));
+    else if (xcd_remap) bid = xcd_contiguous(bid, nb);
+    multi_grid_tile<T, PREC, TOG>(runs, tile_start, nruns, t, slot, (int)bid);
+}
+
+// Persistent form for small batches (see multi_persistent_kernel): a cooperative grid
+// steps nsteps steps, each block taking every gridDim.x-th tile (these runs have few and
+// equal tiles), with a grid-wide barrier between steps.  Fields are staged in two parts,
+// the form of less LDS, so that at least two blocks fit a CU.  The launch after which the
+// guard interval is over for every run (finish) hands the step count on.
+template <class T, int PREC>
+__global__ __launch_bounds__(GRID_BLOCK, 2) void multi_grid_persistent_kernel(const GridRun<T> *__restrict__ runs,
+                                                                              const int *__restrict__ tile_start,
+                                                                              int nruns, int ntiles, int slot,
+                                                                              int nsteps, int finish)
+{
+    cooperative_groups::grid_group grid = cooperative_groups::this_grid();
+    Ctrl *ctrl = runs[0].a.ctrl;
+    const int t0 = __hip_atomic_load(&ctrl->step[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < nsteps; ++k) {
+        for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+            multi_grid_tile<T, PREC, false>(runs, tile_start, nruns, t0 + k, (slot + k) & 1, tile);
+            __syncthreads(); // (the next tile overwrites the LDS)
+        }
+        grid.sync();
+    }
+    if (finish && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(&ctrl->step[slot ^ (nsteps & 1)], t0 + nsteps, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+static const void *grid_persistent_fn(int precision)
+{
+    switch (precision) {
+    case 0: return (const void *)multi_grid_persistent_kernel<double, 0>;
+    case 1: return (const void *)multi_grid_persistent_kernel<float, 1>;
+    case 2: return (const void *)multi_grid_persistent_kernel<float, 2>;
+    case 3: return (const void *)multi_grid_persistent_kernel<float, 3>;
+    default: return nullptr;
+    }
+}
+
+hipError_t grid_persistent_blocks_per_cu(int precision, int most, size_t lds, int *per_cu)
+{
+    const void *f = grid_persistent_fn(precision);
+    if (!f) return hipErrorInvalidValue;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, f, most, lds);
+}
+
+hipError_t launch_grid_persistent(int precision, const void *runs_dev, const int *tile_start_dev, int nruns, int ntiles,
+                                  int most, int blocks, int slot, int nsteps, size_t lds, bool finish, hipStream_t st)
+{
+    const void *f = grid_persistent_fn(precision);
+    if (!f) return hipErrorInvalidValue;
+    int fin = finish ? 1 : 0;
+    void *kargs[] = {(void *)&runs_dev, (void *)&tile_start_dev, (void *)&nruns, (void *)&ntiles,
+                     (void *)&slot, (void *)&nsteps, (void *)&fin};
+    return hipLaunchCooperativeKernel(f, dim3(blocks), dim3(most), kargs, (unsigned int)lds, st);
 }
 
 hipError_t launch_multi_grid(int precision, const void *runs_dev, const int *tile_start_dev, int nruns, int ntiles,
@@ -725,7 +789,8 @@ hipError_t allow_grid_lds()
                        SFG_GF(false, GRID_CLASS, false), SFG_GF(false, GRID_CLASS_S, false),
                        SFG_GF(false, GRID_ROWS, false), SFG_GF(true, GRID_CLASS, false),
                        SFG_GF(true, GRID_CLASS_S, false), SFG_GF(true, GRID_ROWS, false),
-                       (const void *)multi_grid_kernel<double, 0, true>, (const void *)multi_grid_kernel<double, 0, false>};
+                       (const void *)multi_grid_kernel<double, 0, true>, (const void *)multi_grid_kernel<double, 0, false>,
+                       grid_persistent_fn(0)};
 #undef SFG_GF
     hipError_t e = hipSuccess;
     for (const void *k : f)

@@ -214,6 +214,12 @@ hipError_t launch_grid_step(int precision, bool cps, const void *step_args, cons
 // runs of one patch size `most`
 hipError_t launch_multi_grid(int precision, const void *runs_dev, const int *tile_start_dev, int nruns, int ntiles,
                              int most, int xcd_remap, int slot, size_t lds_bytes, bool together, hipStream_t st);
+// Persistent schedule of small batches of one patch size: `blocks` resident blocks step
+// nsteps steps (cooperative launch); finish: the last launch of the guard interval
+hipError_t grid_persistent_blocks_per_cu(int precision, int most, size_t lds_bytes, int *per_cu);
+hipError_t launch_grid_persistent(int precision, const void *runs_dev, const int *tile_start_dev, int nruns, int ntiles,
+                                  int most, int blocks, int slot, int nsteps, size_t lds_bytes, bool finish,
+                                  hipStream_t st);
 // LDS of a patch: its table, and per halo node part A and (together) part B, else
 // the larger of the two (see LDS_A, LDS_B)
 inline size_t grid_lds_bytes(const GridShape &g, bool together, size_t w)

@@ -101,3 +101,36 @@ def test_tuned_launch_shares_a_multi_run_with_sliced_models(shots):
     assert_same(seismograms(makers, True), seismograms(makers, False))
     for h in keep:
         h.close()
+
+
+# batches too small to fill the GPU alone: default shapes in the grid layout with patches
+# of 64 and 128 rows (reach 1 and 2), and beside a lane-group launch
+@pytest.mark.parametrize("prec,specs", [
+    (gpu.FP64, [(host.Q4, 12, 13, 70, False, {}), (host.T6, 4, 5, 20, False, {}),
+                (host.Q4, 11, 11, 45, False, dict(block=256, shots_per_lane_group=32, kernel_variant=5))]),
+    (gpu.FP64, [(host.Q4, 12, 13, 70, False, {}), (host.Q9, 5, 6, 19, False, {})]),
+    (gpu.FP32_KAHAN16, [(host.Q4, 20, 9, 30, False, {}), (host.Q9, 6, 5, 40, False, {})])])
+def test_persistent_schedule_of_default_batches(prec, specs):
+    say(f"persistent schedule of default batches, precision {prec}: {[s[:5] for s in specs]}")
+    keep, makers = make_runs(specs, prec, 60)
+    ref = seismograms(makers, True)
+    for schedule in ([(1, 37), (1, 60)], [(2, 60)], [(0, 20), (2, 15), (0, 60)]):
+        assert_same(seismograms(makers, True, schedule), ref)
+    for h in keep:
+        h.close()
+
+
+def test_persistent_schedule_refuses_what_needs_launches_of_its_own():
+    """Few shots in a batch, and single shots beside batches, as without the grid layout."""
+    say("persistent schedule: refused combinations")
+    for specs in ([(host.Q4, 12, 13, 8, False, {})],
+                  [(host.Q4, 12, 13, 70, False, {}), (host.Q4, 12, 13, 1, False, dict(block=256))]):
+        keep, makers = make_runs(specs, gpu.FP64, 40)
+        runs = [mk() for mk in makers]
+        multi = gpu.Multi(runs)
+        with pytest.raises(gpu.NativeError) as e:
+            multi.set_persistent(1)
+        assert e.value.code == -1
+        multi.close()
+        for h in runs + keep:
+            h.close()
