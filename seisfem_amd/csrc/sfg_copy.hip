@@ -2,12 +2,11 @@
 #include "sfg_copy.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
-#include <exception>
 #include <mutex>
-#include <thread>
 #include <vector>
+
+#include "sfg_pieces.h"
 
 namespace sfg {
 
@@ -68,6 +67,60 @@ static hipError_t direct(char *dst, const char *src, size_t pitch, size_t width,
     return e != hipSuccess ? e : e2;
 }
 
+// The pieces of one download: parts of a row, or several whole rows
+struct Download : PiecePort {
+    hipDevice_t device = 0;
+    hipStream_t st = nullptr;
+    char *buf = nullptr, *to = nullptr;
+    const char *from = nullptr;
+    size_t pitch = 0, width = 0, rows = 0, per_row = 0, per_piece = 0;
+    const int *map = nullptr;
+    hipEvent_t done[kThreads][2] = {};
+
+    char *buffer(int q, int b) const { return buf + (size_t)(2 * q + b) * kPiece; }
+    size_t rows_of(size_t piece) const { return std::min(per_piece, rows - piece * per_piece); }
+    size_t bytes_of(size_t piece) const { return std::min(kPiece, width - piece % per_row * kPiece); }
+
+    int open(int q) override
+    {
+        hipError_t e = hipSetDevice(device);
+        for (int b = 0; b < 2 && e == hipSuccess; ++b) e = hipEventCreateWithFlags(&done[q][b], hipEventDisableTiming);
+        return e;
+    }
+    int issue(int q, int b, size_t piece) override
+    {
+        hipError_t e;
+        if (per_row > 1)
+            e = hipMemcpyAsync(buffer(q, b), from + piece / per_row * pitch + piece % per_row * kPiece, bytes_of(piece),
+                               hipMemcpyDeviceToHost, st);
+        else if (pitch == width)
+            e = hipMemcpyAsync(buffer(q, b), from + piece * per_piece * pitch, rows_of(piece) * width,
+                               hipMemcpyDeviceToHost, st);
+        else
+            e = hipMemcpy2DAsync(buffer(q, b), width, from + piece * per_piece * pitch, pitch, width, rows_of(piece),
+                                 hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipEventRecord(done[q][b], st) : e;
+    }
+    int wait(int q, int b) override { return hipEventSynchronize(done[q][b]); }
+    void take(int q, int b, size_t piece) override
+    {
+        const char *src = buffer(q, b);
+        auto place = [&](size_t row) { return to + (map ? (size_t)map[row] : row) * width; };
+        if (per_row > 1) {
+            std::memcpy(place(piece / per_row) + piece % per_row * kPiece, src, bytes_of(piece));
+        } else if (!map) {
+            std::memcpy(place(piece * per_piece), src, rows_of(piece) * width);
+        } else {
+            for (size_t r = 0; r < rows_of(piece); ++r) std::memcpy(place(piece * per_piece + r), src + r * width, width);
+        }
+    }
+    void close(int q) override
+    {
+        for (hipEvent_t &x : done[q])
+            if (x) (void)hipEventDestroy(x);
+    }
+};
+
 hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const void *src, size_t pitch, size_t width,
                     size_t rows, const int *map, hipStream_t st)
 {
@@ -85,69 +138,22 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
         return direct(to, from, pitch, width, rows, map, st);
     }
 
-    // pieces: parts of a row, or several whole rows
-    const size_t per_row = (width + kPiece - 1) / kPiece, per_piece = per_row > 1 ? 1 : kPiece / width;
-    const size_t pieces = per_row > 1 ? rows * per_row : (rows + per_piece - 1) / per_piece;
-    std::atomic<size_t> next{0};
-    std::atomic<int> error{hipSuccess};
-    auto work = [&](int q) {
-        hipError_t e = hipSetDevice(device);
-        hipEvent_t done[2] = {nullptr, nullptr};
-        for (int k = 0; k < 2 && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&done[k], hipEventDisableTiming);
-        size_t row[2], off[2], len[2];           // the piece on its way in each buffer
-        bool have[2] = {false, false};
-        auto issue = [&](int k) {
-            have[k] = false;
-            const size_t i = next++;
-            if (i >= pieces || e != hipSuccess || error.load() != hipSuccess) return;
-            char *b = buf + (size_t)(2 * q + k) * kPiece;
-            if (per_row > 1) {
-                row[k] = i / per_row;
-                off[k] = i % per_row * kPiece;
-                len[k] = std::min(kPiece, width - off[k]);
-                e = hipMemcpyAsync(b, from + row[k] * pitch + off[k], len[k], hipMemcpyDeviceToHost, st);
-            } else {
-                row[k] = i * per_piece;
-                off[k] = 0;
-                const size_t nr = std::min(per_piece, rows - row[k]);
-                len[k] = nr * width;
-                e = pitch == width ? hipMemcpyAsync(b, from + row[k] * pitch, len[k], hipMemcpyDeviceToHost, st)
-                                   : hipMemcpy2DAsync(b, width, from + row[k] * pitch, pitch, width, nr,
-                                                      hipMemcpyDeviceToHost, st);
-            }
-            if (e == hipSuccess) e = hipEventRecord(done[k], st);
-            have[k] = e == hipSuccess;
-        };
-        issue(0);
-        issue(1);
-        for (int k = 0; have[k]; k ^= 1) {
-            e = hipEventSynchronize(done[k]);
-            if (e != hipSuccess) break;
-            const char *b = buf + (size_t)(2 * q + k) * kPiece;
-            if (per_row > 1 || !map) {
-                std::memcpy(to + (map ? (size_t)map[row[k]] : row[k]) * width + off[k], b, len[k]);
-            } else {
-                for (size_t r = 0; r < len[k] / width; ++r)
-                    std::memcpy(to + (size_t)map[row[k] + r] * width, b + r * width, width);
-            }
-            issue(k);
-        }
-        for (hipEvent_t &x : done)
-            if (x) (void)hipEventDestroy(x);
-        if (e != hipSuccess) error.store(e);
-    };
-    std::thread th[kThreads];
-    int started = 1;
-    try {
-        for (; started < kThreads; ++started) th[started] = std::thread(work, started);
-    } catch (const std::exception &) {
-        // fewer helpers: the pieces are handed out as they are asked for
-    }
-    work(0);
-    for (int q = 1; q < started; ++q) th[q].join();
+    Download d;
+    d.device = device;
+    d.st = st;
+    d.buf = buf;
+    d.to = to;
+    d.from = from;
+    d.pitch = pitch;
+    d.width = width;
+    d.rows = rows;
+    d.map = map;
+    d.per_row = (width + kPiece - 1) / kPiece;
+    d.per_piece = d.per_row > 1 ? 1 : kPiece / width;
+    const size_t pieces = d.per_row > 1 ? rows * d.per_row : (rows + d.per_piece - 1) / d.per_piece;
+    const hipError_t e = (hipError_t)deliver(d, pieces, kThreads);
     if (callers != device) (void)hipSetDevice(callers);
-    const hipError_t e2 = hipStreamSynchronize(st);
-    const hipError_t e = (hipError_t)error.load();
+    const hipError_t e2 = hipStreamSynchronize(st);   // (nothing is left in flight to the buffers)
     return e != hipSuccess ? e : e2;
 }
 
