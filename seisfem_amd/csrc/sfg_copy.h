@@ -6,8 +6,9 @@
 
 namespace sfg {
 
-// Pinned staging buffers of the process, held by the objects that download
-// through them and freed with the last of these.
+// Pinned staging buffers of the process (at most 4 x 16 MB, one set for each download
+// under way), held by the objects that download through them and freed with the last of
+// these.
 struct Staging;
 std::shared_ptr<Staging> staging();
 

@@ -14,28 +14,43 @@ namespace {
 constexpr int kThreads = 8;
 constexpr size_t kPiece = (size_t)1 << 20;   // bytes of one transfer; two buffers per thread
 constexpr size_t kDirect = (size_t)4 << 20;  // smaller results are copied directly
+// Downloads that have pinned buffers at a time (16 MB each, allocated when so many overlap);
+// others are copied directly.  Threads that read back at the same time run side by side:
+// with one set they took turns, and a small result waited for the largest (4.5 MB beside
+// 131 MB 4.7 ms, with sets of their own 0.9; four threads of 131 MB each 17 ms, 15).
+constexpr int kSets = 4;
 std::mutex g_mu;
 std::weak_ptr<Staging> g_staging;
 } // namespace
 
+// Sets of buffers, one for each download under way
 struct Staging {
-    std::mutex mu;                           // one download at a time
-    char *buf = nullptr;
-    bool tried = false;
-    char *get()
+    struct Set {
+        std::mutex mu;                       // held by the download that uses it
+        char *buf = nullptr;
+        bool tried = false;
+    } sets[kSets];
+    // a free set's pinned buffers, locked by lk until the download ends; null: none free, or no memory
+    char *get(std::unique_lock<std::mutex> &lk)
     {
-        if (!tried) {
-            tried = true;
-            if (hipHostMalloc((void **)&buf, 2 * kThreads * kPiece, hipHostMallocPortable) != hipSuccess) {
-                (void)hipGetLastError();
-                buf = nullptr;
+        for (Set &x : sets) {
+            lk = std::unique_lock<std::mutex>(x.mu, std::try_to_lock);
+            if (!lk.owns_lock()) continue;
+            if (!x.tried) {
+                x.tried = true;
+                if (hipHostMalloc((void **)&x.buf, 2 * kThreads * kPiece, hipHostMallocPortable) != hipSuccess) {
+                    (void)hipGetLastError();
+                    x.buf = nullptr;
+                }
             }
+            if (x.buf) return x.buf;
         }
-        return buf;
+        return nullptr;
     }
     ~Staging()
     {
-        if (buf) (void)hipHostFree(buf);
+        for (Set &x : sets)
+            if (x.buf) (void)hipHostFree(x.buf);
     }
 };
 
@@ -128,8 +143,8 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
     char *to = (char *)dst;
     const char *from = (const char *)src;
     if (!staging || width * rows < kDirect) return direct(to, from, pitch, width, rows, map, st);
-    std::lock_guard<std::mutex> lk(staging->mu);
-    char *buf = staging->get();
+    std::unique_lock<std::mutex> lk;
+    char *buf = staging->get(lk);
     // the stream's device, which need not be the caller's
     hipDevice_t device = 0;
     int callers = 0;
