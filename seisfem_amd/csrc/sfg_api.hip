@@ -209,7 +209,18 @@ extern "C" void abc_mpml(int node_num, int element_num, int element_order, int *
 // ---------------------------------------------------------------------------
 // operators
 
-// Grid layout of one operator for patches of at most `most` rows (GridArgs).
+// Values of a grid layout in one precision
+struct GridValues {
+    void *tab = nullptr, *mval = nullptr;
+    ~GridValues()
+    {
+        dfree(tab);
+        dfree(mval);
+    }
+};
+
+// Grid layout of one operator for patches of at most `most` rows (GridArgs).  A run holds
+// the layout and the values it reads; the operator keeps both for its later runs.
 struct GridPlan {
     int most = 0, align = 0;    // rows of a patch; nodes that lines and patches start on a multiple of (0: any)
     bool ok = false;            // false: the operator does not fit the layout
@@ -220,12 +231,10 @@ struct GridPlan {
     int nitems = 0;             // stencils in the tables
     long long nentries = 0;     // table entries
     long long nslots = 0;       // slots of 64 per-row values
-    void *tab[2] = {nullptr, nullptr}, *mval[2] = {nullptr, nullptr}; // FP64, FP32
-    bool vals[2] = {false, false};
+    std::shared_ptr<const GridValues> vals[2]; // FP64, FP32
     ~GridPlan()
     {
         for (int *q : {rows, cls, slice, smax, toff, moff, sdel}) dfree(q); // (toff holds tlen, trep and tdst too)
-        for (int k = 0; k < 2; ++k) { dfree(tab[k]); dfree(mval[k]); }
     }
 };
 
@@ -240,7 +249,7 @@ struct sfg_operator {
     // grid layouts of this operator, built by the first run that takes one and
     // shared by its later runs (grid_plan); freed with the operator
     mutable std::mutex grid_mu;
-    mutable std::vector<std::unique_ptr<GridPlan>> grid;
+    mutable std::vector<std::shared_ptr<GridPlan>> grid;
     mutable int grid_tried = 0;         // lines looked for
     mutable GridShape lines;            // line, lines, hx, hy (line = 0: none)
 };
@@ -585,58 +594,76 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
         }
         if (P.nslots > 0x7fffffffLL / (7 * 64)) return SFG_OK;
         if ((rc = upload(&P.moff, moff, st))) return rc;
-        if (mode == GRID_ROWS && (rc = dalloc(&P.sdel, (size_t)P.nslots * 64))) return rc;
     }
     HIPCHK(hipStreamSynchronize(st));
     P.ok = true;
     return SFG_OK;
 }
 
-// The operator's grid layout for patches of at most `most` rows with the values
-// of one precision, built on first use (on `st`, which it waits for).  *out =
-// null when the operator does not fit the layout (no line structure).
-static int grid_plan(const sfg_operator *op, int most, int align, bool f32, hipStream_t st, const GridPlan **out)
+// The operator's grid layout for patches of at most `most` rows, without values, built
+// on first use (on `st`, which it waits for; the caller holds grid_mu).  *out = null
+// when the operator does not fit the layout (no line structure).
+static int grid_plan(const sfg_operator *op, int most, int align, hipStream_t st, std::shared_ptr<GridPlan> *out)
 {
-    *out = nullptr;
-    std::lock_guard<std::mutex> lk(op->grid_mu);
-    GridPlan *P = nullptr;
-    for (auto &p : op->grid)
-        if (p->most == most && p->align == align) P = p.get();
+    out->reset();
+    std::shared_ptr<GridPlan> P;
+    for (const auto &p : op->grid)
+        if (p->most == most && p->align == align) P = p;
     if (!P) {
-        std::unique_ptr<GridPlan> fresh(new GridPlan);
-        fresh->most = most;
-        fresh->align = align;
-        int rc = build_grid(op, *fresh, st);
-        if (rc) return rc;
-        P = fresh.get();
-        op->grid.push_back(std::move(fresh));
-    }
-    if (!P->ok) return SFG_OK;
-    const int k = f32 ? 1 : 0, w = f32 ? 4 : 8;
-    if (!P->vals[k]) {
-        const void *v = f32 ? (const void *)op->v32 : (const void *)op->v64;
-        int rc;
-        char *tv = nullptr, *mv = nullptr;
-        dfree(P->tab[k]); // (of an attempt that ran out of memory)
-        dfree(P->mval[k]);
-        if ((rc = dalloc(&tv, (size_t)P->nentries * 8 * w))) return rc;
-        P->tab[k] = tv;
-        if (P->mode != GRID_CLASS) {
-            const size_t per = P->mode == GRID_ROWS ? 7 : 1;
-            if ((rc = dalloc(&mv, (size_t)P->nslots * 64 * per * w))) return rc;
-            P->mval[k] = mv;
+        try {
+            P = std::make_shared<GridPlan>();
+            P->most = most;
+            P->align = align;
+            int rc = build_grid(op, *P, st);
+            if (rc) return rc;
+            op->grid.push_back(P);
+        } catch (const std::bad_alloc &) {
+            return fail(SFG_E_NOMEM, "grid layout: out of host memory");
         }
-        if (P->nitems)
-            HIPCHK(launch_grid_table(P->nitems, P->trep, P->tdst, op->rp, op->ci, P->g.line, P->g.W, v, (size_t)op->nnz,
-                                     w, tv, st));
-        if (P->mode != GRID_CLASS)
-            HIPCHK(launch_grid_values(P->g.npatch * (P->g.most / 64), P->mode, P->rows, P->moff, P->smax, op->rp,
-                                      op->ci, P->g.line, P->g.W, v, (size_t)op->nnz, w, mv, P->sdel, st));
-        HIPCHK(hipStreamSynchronize(st));
-        P->vals[k] = true;
     }
-    *out = P;
+    if (P->ok) *out = P;
     return SFG_OK;
+}
+
+// The layout's values in one precision, filled on first use (on `st`, which it waits
+// for; the caller holds grid_mu).
+static int grid_values(const sfg_operator *op, GridPlan &P, bool f32, hipStream_t st,
+                       std::shared_ptr<const GridValues> *out)
+{
+    const int k = f32 ? 1 : 0, w = f32 ? 4 : 8;
+    if (!P.vals[k]) {
+        const void *v = f32 ? (const void *)op->v32 : (const void *)op->v64;
+        auto x = std::make_shared<GridValues>();
+        int rc;
+        if ((rc = dalloc((char **)&x->tab, (size_t)P.nentries * 8 * w))) return rc;
+        if (P.mode != GRID_CLASS) {
+            const size_t per = P.mode == GRID_ROWS ? 7 : 1;
+            if ((rc = dalloc((char **)&x->mval, (size_t)P.nslots * 64 * per * w))) return rc;
+            if (P.mode == GRID_ROWS && !P.sdel && (rc = dalloc(&P.sdel, (size_t)P.nslots * 64))) return rc;
+        }
+        if (P.nitems)
+            HIPCHK(launch_grid_table(P.nitems, P.trep, P.tdst, op->rp, op->ci, P.g.line, P.g.W, v, (size_t)op->nnz, w,
+                                     x->tab, st));
+        if (P.mode != GRID_CLASS)
+            HIPCHK(launch_grid_values(P.g.npatch * (P.g.most / 64), P.mode, P.rows, P.moff, P.smax, op->rp, op->ci,
+                                      P.g.line, P.g.W, v, (size_t)op->nnz, w, x->mval, P.sdel, st));
+        HIPCHK(hipStreamSynchronize(st));
+        P.vals[k] = std::move(x);
+    }
+    *out = P.vals[k];
+    return SFG_OK;
+}
+
+// Gives back the layouts and values that no run holds.
+static void release_grids(const sfg_operator *op)
+{
+    std::lock_guard<std::mutex> lk(op->grid_mu);
+    for (auto &p : op->grid) {
+        for (auto &v : p->vals)
+            if (v.use_count() == 1) v.reset();
+        if (p.use_count() == 1) p.reset();
+    }
+    op->grid.erase(std::remove(op->grid.begin(), op->grid.end(), nullptr), op->grid.end());
 }
 
 // ---------------------------------------------------------------------------
@@ -775,31 +802,32 @@ static void batched_default(const sfg_operator *op, const sfg_shot_desc *d, bool
     *xcd = std::max(1, (line[0] + 16) / 32);     // 4 rows a block, 8 XCDs
 }
 
-// The layout the library takes for `nshots` shots (null: none).  With several shots
+// The layout the library takes for `nshots` shots, and its values (null: none).  With several shots
 // lines and patches start on 128-byte boundaries (64 with small patches): the state
 // then streams through HBM, and a line written in two parts costs its read back
 // (128 shots Q4 400 x 400 FP32 844 -> 804 us per step, 37 shots Q9 97 x 111 132 -> 124).
-static int choose_grid(const sfg_operator *op, int nshots, bool f32, hipStream_t st, const GridPlan **out)
+static int choose_grid(const sfg_operator *op, int nshots, bool f32, hipStream_t st,
+                       std::shared_ptr<const GridPlan> *plan, std::shared_ptr<const GridValues> *vals)
 {
-    int rc = SFG_OK;
+    std::lock_guard<std::mutex> lk(op->grid_mu);
+    int rc = find_lines(op, st);
+    if (rc || op->lines.line == 0) return rc;
+    std::shared_ptr<GridPlan> P;
     auto get = [&](int most) {
-        rc = grid_plan(op, most, nshots > 1 ? (most == 256 && f32 ? 32 : 16) : 0, f32, st, out);
-        return rc == SFG_OK && *out;
+        rc = grid_plan(op, most, nshots > 1 ? (most == 256 && f32 ? 32 : 16) : 0, st, &P);
+        return rc == SFG_OK && P;
     };
-    *out = nullptr;
-    int reach;
-    {
-        std::lock_guard<std::mutex> lk(op->grid_mu);
-        if ((rc = find_lines(op, st))) return rc;
-        if (op->lines.line == 0) return SFG_OK;
-        reach = std::max(op->lines.hx, op->lines.hy);
-    }
-    if (!get(grid_rows(op->n, nshots, reach)) && rc == SFG_OK) (void)get(256);
+    if (!get(grid_rows(op->n, nshots, std::max(op->lines.hx, op->lines.hy))) && rc == SFG_OK) (void)get(256);
+    if (rc || !P) return rc;
     // with all seven values per row the matrices are read again for every shot, which
     // lane groups of many shots do not (T6 120 x 120 FP64, 64 shots: 922 us per step
     // against 687; Q9 100 x 100 FP64, 24 shots: 331 / 481)
-    if (*out && (*out)->mode == GRID_ROWS && nshots > 32) *out = nullptr;
-    return rc;
+    if (P->mode == GRID_ROWS && nshots > 32) return SFG_OK;
+    // (padded lines may exceed the index range where lane groups do not)
+    if ((size_t)P->g.pitch * P->g.lines * nshots >= (size_t)1 << 31) return SFG_OK;
+    if ((rc = grid_values(op, *P, f32, st, vals))) return rc;
+    *plan = P;
+    return SFG_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -846,7 +874,8 @@ struct sfg_run {
     // grid layout (default launch shape on meshes numbered line by line): the
     // per-step launches take launch_grid_step with these; a64 / a32 keep a
     // per-row form that steps a single-shot run's state alike (persistent schedule)
-    const GridPlan *plan = nullptr;
+    std::shared_ptr<const GridPlan> plan;
+    std::shared_ptr<const GridValues> vals;
     int np = 0;                 // padded nodes per field
     unsigned char *info = nullptr;
     int *bkind = nullptr;
@@ -1024,13 +1053,11 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
     }
     // lane grouping: shots per lane group and the padded shot stride
     if (grid && n < 1 << 28 && grid_default(op, d)) {
-        int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan);
+        int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan, &r->vals);
         if (rc) {
             run_free(r);
             return rc;
         }
-        // (padded lines may exceed the index range where lane groups do not)
-        if (r->plan && (size_t)r->plan->g.pitch * r->plan->g.lines * d->nshots >= (size_t)1 << 31) r->plan = nullptr;
     }
     int variant = d->kernel_variant, xcd = d->xcd_remap;
     if (!r->plan) batched_default(op, d, nmedia > 1, &variant, &xcd);
@@ -1526,8 +1553,8 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
         fill(r->a32, (float *)r->state, (float *)r->comp, op->v32, md->coef32, [](double v) { return (float)v; }),
             r->a32.Ap = op->p32, r->a32.sell_val = (const float *)r->sell_val;
 
-    if (const GridPlan *P = r->plan) {
-        auto fill_grid = [&](auto &g, int k, auto *tab, auto *mval) {
+    if (const GridPlan *P = r->plan.get()) {
+        auto fill_grid = [&](auto &g, auto *tab, auto *mval) {
             g.g = P->g;
             g.mode = P->mode;
             g.toff = P->toff;
@@ -1542,11 +1569,11 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
             g.sdel = P->sdel;
             g.info = r->info;
             g.bkind = r->bkind;
-            g.tab = (decltype(tab))P->tab[k];
-            g.mval = (decltype(mval))P->mval[k];
+            g.tab = (decltype(tab))r->vals->tab;
+            g.mval = (decltype(mval))r->vals->mval;
         };
-        if (r->prec == 0) fill_grid(r->g64, 0, (const double *)nullptr, (const double *)nullptr);
-        else fill_grid(r->g32, 1, (const float *)nullptr, (const float *)nullptr);
+        if (r->prec == 0) fill_grid(r->g64, (const double *)nullptr, (const double *)nullptr);
+        else fill_grid(r->g32, (const float *)nullptr, (const float *)nullptr);
         const bool tog = grid_together(r->prec, std::max(P->g.hx, P->g.hy), (long long)P->g.npatch * r->S);
         r->g64.together = r->g32.together = tog;
         r->grid_lds = grid_lds_bytes(P->g, tog, w);
@@ -1575,13 +1602,15 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
     return SFG_OK;
 }
 
-// (the grid layout's tables and padded lines may need more memory than lane groups do)
+// (the grid layout's tables and padded lines may need more memory than lane groups do:
+// these then have what it had taken, except what other runs hold)
 static int run_create_impl(sfg_run **out, const sfg_operator *op, const sfg_medium *const *media, int nmedia,
                            const sfg_shot_desc *d)
 {
     int rc = run_create_as(out, op, media, nmedia, d, true);
     if (rc == SFG_E_NOMEM) {
         (void)hipGetLastError();
+        release_grids(op);
         rc = run_create_as(out, op, media, nmedia, d, false);
     }
     return rc;
