@@ -219,8 +219,10 @@ __device__ __forceinline__ void grid_tile(const StepArgs<T> &a, const GridArgs<T
     const int wlen = wave_info & 0xff;           // longest row of the wave
     const bool uniform = (wave_info & 0x100) != 0;
     // the row's stencil: first table entry, nonzeros; its own halo position
-    const int e0 = key & 0xfff, own = key >> 12 & 0xfff, rlen = key >> 24;
+    // (a lane without a row stands at the wave's first one: it walks along, see walk)
     const bool valid = row >= 0;
+    const int own0 = __builtin_amdgcn_readfirstlane(key >> 12 & 0xfff);
+    const int e0 = key & 0xfff, own = valid ? key >> 12 & 0xfff : own0, rlen = key >> 24;
     const int r = valid ? row : 0;
     // byte offsets of the row in the state (lines `pitch` nodes apart) and among the coefficients
     const int oy = (own * g.magic) >> 16, sr = valid ? (y0 + oy) * gs.pitch + x0 + own - oy * W : 0;
@@ -316,10 +318,13 @@ __device__ __forceinline__ void grid_tile(const StepArgs<T> &a, const GridArgs<T
     // lanes with v_readlane (through the scalar cache, which every launch finds cold, a
     // nonzero took 500-1000 cycles, and a scalar load in flight turns every LDS wait
     // into a full drain); the lanes of other waves read their own entries of the table.
+    // v_readlane must not read a lane that is switched off, so a wave of one class walks with
+    // all its lanes, also those that are not `on`, whose products are not used.
     auto walk = [&](bool on, auto np, auto &&nz) __attribute__((always_inline)) {
         constexpr int NP = decltype(np)::value;
-        if (!on || wlen == 0) return;
+        if (wlen == 0 || __builtin_amdgcn_ballot_w64(on) == 0) return;
         if constexpr (MODE == GRID_ROWS) {
+            if (!on) return;
             constexpr int AHEAD = EXACT ? 2 : 4;
             const size_t m0 = (size_t)ro(g.moff)[wid];
             for (int k0 = 0; k0 < wlen; k0 += AHEAD) {
@@ -398,7 +403,7 @@ __device__ __forceinline__ void grid_tile(const StepArgs<T> &a, const GridArgs<T
                     nz(x[b], MODE == GRID_CLASS_S ? mk : st.value(0, k), st.value(1, k), st.value(2, k), st.value(3, k),
                        st.value(4, k), st.value(5, k), st.value(6, k));
                 });
-            } else {
+            } else if (on) {
                 const Entry<T> *e = tab + e0;
                 Entry<T> c = e[0], next;
                 all(rlen, [&](int k, auto, T mk) __attribute__((always_inline)) {
