@@ -1732,10 +1732,11 @@ extern "C" int sfg_run_seismograms(sfg_run *r, double *u, double *w)
     HIPCHK(hipStreamSynchronize(r->stream));
     const size_t per = (size_t)r->max_steps * r->rec_num;
     if (per == 0) return SFG_OK;
+    std::vector<char> scratch;
     HIPCHK(download(r->staging, u, r->seis_u, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
-                    r->stream));
+                    r->stream, &scratch));
     HIPCHK(download(r->staging, w, r->seis_w, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
-                    r->stream));
+                    r->stream, &scratch));
     return SFG_OK;
 }
 

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <cstddef>
 #include <memory>
+#include <vector>
 
 namespace sfg {
 
@@ -21,8 +22,9 @@ std::shared_ptr<Staging> staging();
 // into the arrays (32-45 ms copied there directly), and take 12 ms here, where 8 threads
 // each copy what the DMA engine has put into their pinned buffers (1000 predictions of
 // 32000 samples, all told: 16.5 ms then, 5.7 ms now).  Below 4 MB, where
-// starting the threads costs as much, and without pinned memory the copy is direct.
+// starting the threads costs as much, and without pinned memory the copy is direct; rows
+// to be copied apart then pass through scratch, which a caller of many downloads keeps.
 hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const void *src, size_t pitch, size_t width,
-                    size_t rows, const int *map, hipStream_t st);
+                    size_t rows, const int *map, hipStream_t st, std::vector<char> *scratch = nullptr);
 
 } // namespace sfg

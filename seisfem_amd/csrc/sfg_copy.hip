@@ -65,21 +65,23 @@ std::shared_ptr<Staging> staging()
     return s;
 }
 
+// One transfer, whatever the number of rows: rows in a pitch come over with what lies
+// between them and are copied apart here (a 2D copy into pageable memory moves row by row,
+// 7 us each: 1024 rows of 52 bytes 7.0 ms against 0.04).
 static hipError_t direct(char *dst, const char *src, size_t pitch, size_t width, size_t rows, const int *map,
-                         hipStream_t st)
+                         hipStream_t st, std::vector<char> *scratch)
 {
-    hipError_t e;
-    std::vector<char> rowsv;
-    if (map) rowsv.resize(width * rows);     // one transfer, whatever the number of rows
-    char *to = map ? rowsv.data() : dst;
-    if (pitch == width)
-        e = hipMemcpyAsync(to, src, width * rows, hipMemcpyDeviceToHost, st);
-    else
-        e = hipMemcpy2DAsync(to, width, src, pitch, width, rows, hipMemcpyDeviceToHost, st);
+    const size_t bytes = (rows - 1) * pitch + width;
+    std::vector<char> own;
+    std::vector<char> &rowsv = scratch ? *scratch : own;
+    const bool apart = map || pitch != width;
+    if (apart && rowsv.size() < bytes) rowsv.resize(bytes);
+    const hipError_t e = hipMemcpyAsync(apart ? rowsv.data() : dst, src, bytes, hipMemcpyDeviceToHost, st);
     const hipError_t e2 = hipStreamSynchronize(st);
-    if (map && e == hipSuccess && e2 == hipSuccess)
-        for (size_t i = 0; i < rows; ++i) std::memcpy(dst + (size_t)map[i] * width, to + i * width, width);
-    return e != hipSuccess ? e : e2;
+    if (e != hipSuccess || e2 != hipSuccess) return e != hipSuccess ? e : e2;
+    for (size_t i = 0; apart && i < rows; ++i)
+        std::memcpy(dst + (map ? (size_t)map[i] : i) * width, rowsv.data() + i * pitch, width);
+    return hipSuccess;
 }
 
 // The pieces of one download: parts of a row, or several whole rows
@@ -137,12 +139,12 @@ struct Download : PiecePort {
 };
 
 hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const void *src, size_t pitch, size_t width,
-                    size_t rows, const int *map, hipStream_t st)
+                    size_t rows, const int *map, hipStream_t st, std::vector<char> *scratch)
 {
     if (width == 0 || rows == 0) return hipStreamSynchronize(st);
     char *to = (char *)dst;
     const char *from = (const char *)src;
-    if (!staging || width * rows < kDirect) return direct(to, from, pitch, width, rows, map, st);
+    if (!staging || width * rows < kDirect) return direct(to, from, pitch, width, rows, map, st, scratch);
     std::unique_lock<std::mutex> lk;
     char *buf = staging->get(lk);
     // the stream's device, which need not be the caller's
@@ -150,7 +152,7 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
     int callers = 0;
     if (!buf || hipStreamGetDevice(st, &device) != hipSuccess || hipGetDevice(&callers) != hipSuccess) {
         (void)hipGetLastError();
-        return direct(to, from, pitch, width, rows, map, st);
+        return direct(to, from, pitch, width, rows, map, st, scratch);
     }
 
     Download d;

@@ -1483,6 +1483,7 @@ extern "C" int sfg_mlp_predict(sfg_mlp *m, const float *X, int n, float *Y, doub
     MCHK(hipMalloc((void **)&Xd, sizeof(float) * (size_t)n * m->nin));
     MCHK(hipMemcpy(Xd, X, sizeof(float) * (size_t)n * m->nin, hipMemcpyHostToDevice));
     std::vector<int> idx(B);
+    std::vector<char> scratch;
     hipEvent_t e0, e1;
     MCHK(hipEventCreate(&e0));
     MCHK(hipEventCreate(&e1));
@@ -1498,7 +1499,7 @@ extern "C" int sfg_mlp_predict(sfg_mlp *m, const float *X, int n, float *Y, doub
         if (rc) { (void)hipFree(Xd); return rc; }
         // the outputs of the models go straight into the caller's rows
         MCHK(sfg::download(m->staging, Y + (size_t)s0 * m->nout, m->y, sizeof(float) * m->pout[L],
-                           sizeof(float) * m->nout, cnt, nullptr, m->st));
+                           sizeof(float) * m->nout, cnt, nullptr, m->st, &scratch));
         float ms = 0.f;
         MCHK(hipEventElapsedTime(&ms, e0, e1));
         total += ms;
