@@ -1733,10 +1733,10 @@ extern "C" int sfg_run_seismograms(sfg_run *r, double *u, double *w)
     const size_t per = (size_t)r->max_steps * r->rec_num;
     if (per == 0) return SFG_OK;
     std::vector<char> scratch;
-    HIPCHK(download(r->staging, u, r->seis_u, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
-                    r->stream, &scratch));
-    HIPCHK(download(r->staging, w, r->seis_w, sizeof(double) * per, sizeof(double) * per, r->nshots, r->perm.data(),
-                    r->stream, &scratch));
+    const int *map = std::is_sorted(r->perm.begin(), r->perm.end()) ? nullptr : r->perm.data(); // null: as they lie
+    const size_t row = sizeof(double) * per;
+    HIPCHK(download(r->staging, u, r->seis_u, row, row, r->nshots, map, r->stream, &scratch));
+    HIPCHK(download(r->staging, w, r->seis_w, row, row, r->nshots, map, r->stream, &scratch));
     return SFG_OK;
 }
 

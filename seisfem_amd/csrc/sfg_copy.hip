@@ -13,42 +13,60 @@ namespace sfg {
 namespace {
 constexpr int kThreads = 8;
 constexpr size_t kPiece = (size_t)1 << 20;   // bytes of one transfer; two buffers per thread
-constexpr size_t kDirect = (size_t)4 << 20;  // smaller results are copied directly
 // Downloads that have pinned buffers at a time (16 MB each, allocated when so many overlap);
 // others are copied directly.  Threads that read back at the same time run side by side:
 // with one set they took turns, and a small result waited for the largest (4.5 MB beside
 // 131 MB 4.7 ms, with sets of their own 0.9; four threads of 131 MB each 17 ms, 15).
 constexpr int kSets = 4;
+// Results below kDirect are copied directly; those of up to kSmall through a small set
+// (the runtime's own staging takes two to five times as long there); those below kOne by the
+// caller's thread alone, through a set if there is one (a new one costs a page fault per 4 KB
+// too); larger ones by all threads.  us into memory in use / fresh memory, copied directly,
+// through a set by one thread, by 8 threads: 16 KB 18 / 15, 12 / 14, 67 / 93; 128 KB 62 /
+// 31, 14 / 30, 103 / 100; 1 MB 67 / 252, 61 / 244, 110 / 361; 4 MB 243 / 990, 220 / 940, 254 /
+// 736; 16 MB 927 / 3699, 823 / 3557, 645 / 1185.
+constexpr size_t kDirect = (size_t)64 << 10;
+constexpr size_t kSmall = (size_t)256 << 10;
+constexpr size_t kOne = (size_t)4 << 20;
 std::mutex g_mu;
 std::weak_ptr<Staging> g_staging;
 } // namespace
 
-// Sets of buffers, one for each download under way
+// Sets of pinned buffers, each used by one download at a time
 struct Staging {
     struct Set {
         std::mutex mu;                       // held by the download that uses it
         char *buf = nullptr;
         bool tried = false;
-    } sets[kSets];
-    // a free set's pinned buffers, locked by lk until the download ends; null: none free, or no memory
-    char *get(std::unique_lock<std::mutex> &lk)
-    {
-        for (Set &x : sets) {
-            lk = std::unique_lock<std::mutex>(x.mu, std::try_to_lock);
-            if (!lk.owns_lock()) continue;
-            if (!x.tried) {
-                x.tried = true;
-                if (hipHostMalloc((void **)&x.buf, 2 * kThreads * kPiece, hipHostMallocPortable) != hipSuccess) {
+        // the buffers, locked by lk until the download ends; null: in use, no memory, or (make
+        // false) not allocated yet
+        char *take(std::unique_lock<std::mutex> &lk, size_t bytes, bool make)
+        {
+            lk = std::unique_lock<std::mutex>(mu, std::try_to_lock);
+            if (!lk.owns_lock()) return nullptr;
+            if (make && !tried) {
+                tried = true;
+                if (hipHostMalloc((void **)&buf, bytes, hipHostMallocPortable) != hipSuccess) {
                     (void)hipGetLastError();
-                    x.buf = nullptr;
+                    buf = nullptr;
                 }
             }
-            if (x.buf) return x.buf;
+            return buf;
         }
+    } small, sets[kSets];
+    // pinned memory for a result of so many bytes (null: none)
+    char *get(std::unique_lock<std::mutex> &lk, size_t bytes)
+    {
+        if (bytes < kDirect) return nullptr;
+        if (bytes <= kSmall)
+            if (char *b = small.take(lk, kSmall, true)) return b;
+        for (Set &x : sets)
+            if (char *b = x.take(lk, 2 * kThreads * kPiece, bytes >= kOne)) return b;
         return nullptr;
     }
     ~Staging()
     {
+        if (small.buf) (void)hipHostFree(small.buf);
         for (Set &x : sets)
             if (x.buf) (void)hipHostFree(x.buf);
     }
@@ -67,20 +85,22 @@ std::shared_ptr<Staging> staging()
 
 // One transfer, whatever the number of rows: rows in a pitch come over with what lies
 // between them and are copied apart here (a 2D copy into pageable memory moves row by row,
-// 7 us each: 1024 rows of 52 bytes 7.0 ms against 0.04).
-static hipError_t direct(char *dst, const char *src, size_t pitch, size_t width, size_t rows, const int *map,
-                         hipStream_t st, std::vector<char> *scratch)
+// 7 us each: 1024 rows of 52 bytes 7.0 ms against 0.04).  buf: pinned memory of that size, or null.
+static hipError_t in_one(char *dst, const char *src, size_t pitch, size_t width, size_t rows, const int *map,
+                         hipStream_t st, char *buf, std::vector<char> *scratch)
 {
     const size_t bytes = (rows - 1) * pitch + width;
-    std::vector<char> own;
-    std::vector<char> &rowsv = scratch ? *scratch : own;
     const bool apart = map || pitch != width;
-    if (apart && rowsv.size() < bytes) rowsv.resize(bytes);
-    const hipError_t e = hipMemcpyAsync(apart ? rowsv.data() : dst, src, bytes, hipMemcpyDeviceToHost, st);
-    const hipError_t e2 = hipStreamSynchronize(st);
-    if (e != hipSuccess || e2 != hipSuccess) return e != hipSuccess ? e : e2;
-    for (size_t i = 0; apart && i < rows; ++i)
-        std::memcpy(dst + (map ? (size_t)map[i] : i) * width, rowsv.data() + i * pitch, width);
+    std::vector<char> own;
+    if (apart && !buf) {
+        std::vector<char> &v = scratch ? *scratch : own;
+        if (v.size() < bytes) v.resize(bytes);
+        buf = v.data();
+    }
+    const hipError_t e = hipMemcpyWithStream(buf ? buf : dst, src, bytes, hipMemcpyDeviceToHost, st);
+    if (e != hipSuccess) return e;
+    if (!apart && buf) std::memcpy(dst, buf, bytes);
+    for (size_t i = 0; apart && i < rows; ++i) std::memcpy(dst + (map ? (size_t)map[i] : i) * width, buf + i * pitch, width);
     return hipSuccess;
 }
 
@@ -144,15 +164,16 @@ hipError_t download(const std::shared_ptr<Staging> &staging, void *dst, const vo
     if (width == 0 || rows == 0) return hipStreamSynchronize(st);
     char *to = (char *)dst;
     const char *from = (const char *)src;
-    if (!staging || width * rows < kDirect) return direct(to, from, pitch, width, rows, map, st, scratch);
+    const size_t bytes = (rows - 1) * pitch + width;
     std::unique_lock<std::mutex> lk;
-    char *buf = staging->get(lk);
+    char *buf = staging ? staging->get(lk, bytes) : nullptr;
+    if (!buf || bytes < kOne) return in_one(to, from, pitch, width, rows, map, st, buf, scratch);
     // the stream's device, which need not be the caller's
     hipDevice_t device = 0;
     int callers = 0;
-    if (!buf || hipStreamGetDevice(st, &device) != hipSuccess || hipGetDevice(&callers) != hipSuccess) {
+    if (hipStreamGetDevice(st, &device) != hipSuccess || hipGetDevice(&callers) != hipSuccess) {
         (void)hipGetLastError();
-        return direct(to, from, pitch, width, rows, map, st, scratch);
+        return in_one(to, from, pitch, width, rows, map, st, nullptr, scratch);
     }
 
     Download d;
