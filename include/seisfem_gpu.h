@@ -146,9 +146,9 @@ typedef struct {
     int kernel_variant;        /* 0 = chosen by the library: with shots_per_lane_group 0, row_order NULL
                                   and block 0 or 256, meshes numbered line by line take the grid
                                   layout (patches of rows with their neighbours' fields in LDS, the
-                                  matrices as a table of the distinct row stencils; FP64, and the FP32
-                                  forms unless 64-shot lane groups would be mostly full) or 64-shot
-                                  lane groups with 3 or 5 and XCD stripes; else 1.  1 = packed values + 2-way gather, 2 = separate value
+                                  matrices as a table of the distinct row stencils) or, where more
+                                  than 16 shots keep 64-shot lane groups busy enough, those, with 3
+                                  or 5 and XCD stripes once the state streams through HBM; else 1.  1 = packed values + 2-way gather, 2 = separate value
                                   arrays, 3 = 1 + streaming hints on data used once per step,
                                   4 = 3 + own-row fields kept from the diagonal gather and own-row
                                   accelerations (p in the FP32 forms) / Kahan terms loaded first,

@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -360,7 +361,8 @@ static std::vector<int> line_candidates(const sfg_operator *op)
 
 // Patch shape: the one whose blocks touch the fewest 64-byte pieces of the
 // state: 10 staged words per halo node and 28 own words per row (in and out).
-static void choose_patch(GridShape &g, int most, int align)
+// Returns those bytes (8 a word); g.npatch stays 0 when no shape fits.
+static double choose_patch(GridShape &g, int most, int align)
 {
     double best = 1e300;
     GridShape b = g;
@@ -386,6 +388,7 @@ static void choose_patch(GridShape &g, int most, int align)
         if (cost < best) best = cost, b = c;
     }
     g = b;
+    return best;
 }
 
 // Most classes a table may hold (their entries, at most 25 each, are numbered in
@@ -740,6 +743,9 @@ extern "C" void sfg_medium_destroy(sfg_medium *md)
     delete md;
 }
 
+// words of Kahan terms per node of one buffer
+static size_t comp_fields(int prec) { return prec == 3 ? 3 : prec == 2 ? 6 : 0; }
+
 // ---- launch shape left to the library (shots_per_lane_group, kernel_variant,
 // row_order and a block other than 256 not given) ------------------------------
 
@@ -765,67 +771,134 @@ static int grid_rows(int nodes, int nshots, int reach)
     return reach > 1 ? (rows <= 131072 ? 128 : 256) : (rows <= 65536 ? 64 : 256);
 }
 
-// Whether a descriptor that leaves the launch shape to the library may take the grid
-// layout.  FP64 does for any number of shots.  In the FP32 forms 64-shot lane groups
-// that are mostly full (at least three quarters) need fewer instructions for the same
-// bytes, except for long rows (Q9: 16 nonzeros on average).  us per step, grid / best
-// lane-group launch: Q4 300 x 300 FP64 8 shots 93 / 257, 64 shots 628 / 769; FP32 +
-// Kahan (bfloat16 terms) 8 shots 28 / 85, 24 shots 98 / 170, 64 shots 251 / 233, 128
-// shots 490 / 455; Q4 200 x 200 72 shots 153 / 202, 96 shots 200 / 203; Q9 120 x 120 24
-// shots 92 / 180, 128 shots 476 / 493; T6 120 x 120 128 shots 467 / 423; a medium per
-// shot, 128 shots: Q4 200 x 200 258 / 233, Q9 100 x 100 336 / 374.
-static bool grid_default(const sfg_operator *op, const sfg_shot_desc *d)
+// Whether a descriptor leaves the launch shape to the library.
+static bool default_shape(const sfg_shot_desc *d)
 {
-    if (d->shots_per_lane_group != 0 || d->kernel_variant != 0 || d->row_order ||
-        (d->block != 0 && d->block != GRID_BLOCK))
-        return false;
-    const int groups = (d->nshots + 63) / 64;
-    return d->precision == 0 || 4 * d->nshots <= 3 * 64 * groups || op->nnz > 14LL * op->n;
+    return d->shots_per_lane_group == 0 && d->kernel_variant == 0 && !d->row_order &&
+           (d->block == 0 || d->block == GRID_BLOCK);
+}
+
+// What a run's shots ask of a layout
+struct RunLoad {
+    int prec = 0, shots = 0;
+    bool media = false;         // a medium per shot
+    double active = 0, lanes = 0; // shot-steps, and those of 64-shot lane groups that step until their last shot ends
+    double bytes = 0;           // state (both buffers) and coefficients of a medium per shot, in 64-shot lane groups
+};
+static RunLoad run_load(int n, int prec, bool media, std::vector<int> steps)
+{
+    RunLoad l;
+    l.prec = prec;
+    l.shots = (int)steps.size();
+    l.media = media;
+    std::sort(steps.begin(), steps.end(), std::greater<int>());
+    for (size_t s = 0; s < steps.size(); ++s) {
+        l.active += steps[s];
+        if (s % 64 == 0) l.lanes += 64.0 * steps[s];
+    }
+    l.bytes = (double)n * ((l.shots + 63) / 64 * 64) * (prec == 0 ? 8.0 : 4.0) *
+              (2.0 * NFIELD + 2.0 * comp_fields(prec) + (media ? 12.0 : 0.0));
+    return l;
+}
+// State in lane groups from which it streams through HBM: 4/3 of the Infinity Cache (below,
+// the hints of data used once cost more than they save; see batched_default)
+static const double kStreams = 340e6;
+
+// Whether the grid layout in patches of shape g (of `cost`, see choose_patch) is taken for
+// a run of more than 16 shots rather than 64-shot lane groups.  A grid step costs by its
+// active shots, lane groups by their lanes until the last shot of each has ended; an active
+// shot costs more in the grid layout where patches fit the lines badly: measured, `rho` of
+// its cost in a full lane group grows with the bytes its patches touch (rows of up to 14
+// nonzeros), or with the places they leave empty (FP64, and Q9 with 16 nonzeros on average,
+// where reach 2 makes narrow meshes fill little).  us per step, grid / lane groups: FP32 + Kahan
+// (bfloat16 terms), all shots active, 64 shots Q4 40 x 40 10.8 / 13.6, Q4 150 x 100 39.7 / 44.6,
+// T6 60 x 50 46 / 45, T6 12 x 60 22.6 / 18.2, Q9 60 x 50 49 / 54, Q9 8 x 100 32.5 / 23.1, 128
+// shots Q4 300 x 300 490 / 455, Q9 120 x 120 476 / 493, T6 120 x 120 467 / 423; shots of uneven
+// length (half to all of the steps), 64 shots Q4 150 x 100 32 / 43, Q4 300 x 300 188 / 218,
+// T6 12 x 60 19.1 / 18.4, Q9 8 x 100 26.7 / 22.2, 128 shots Q4 150 x 100 87 / 92, Q4 300 x
+// 300 364 / 383, T6 120 x 100 304 / 303; 32 of 64 lanes Q4 200 x 200 59 / 82, T6 60 x 50 29 /
+// 39, Q9 8 x 100 14.9 / 20.3; FP64, 64 shots Q4 300 x 300 628 / 769, 128 shots Q4 150 x 100
+// 242 / 288, T6 60 x 50 225 / 284, Q9 8 x 100 111 / 95.
+static bool grid_pays(const sfg_operator *op, const RunLoad &l, const GridShape &g, double cost)
+{
+    if (l.shots <= 16) return true; // (lane groups of 16 or fewer: 8 shots Q4 300 x 300 FP64 93 / 257, FP32 28 / 85)
+    const double fill = (double)op->n / ((double)g.npatch * g.most);
+    const bool stream = l.bytes > kStreams, long_rows = op->nnz > 14LL * op->n;
+    const double steps = l.lanes > 0 ? l.active / l.lanes : 1.0;
+    if (l.prec == 0) return 0.5 / std::pow(fill, 1.4) * steps <= 1.0;
+    if (long_rows) {
+        // (from eight blocks of 256 rows per CU on a further block waits for a place)
+        const double blocks = (double)g.npatch * l.shots * (l.lanes > 0 ? l.active / l.lanes : 1.0);
+        return 0.6 / std::pow(fill, 1.4) * (blocks > 2048 ? 1.15 : 1.0) * steps <= 1.0;
+    }
+    const double bytes = cost / ((double)op->n * 8.0 * 38.0);   // touched over needed
+    return stream ? 0.78 * bytes * steps <= 0.9 : 0.68 * bytes * steps <= 0.84;
 }
 
 // Variant and XCD map of 64-shot lane groups whose launch shape is left to the
-// library, on meshes numbered line by line: XCD stripes of an eighth of a line (a
-// row's neighbours on the adjacent lines then come from the same L2); streaming
-// hints on large meshes of few nonzeros a row, three nonzeros in flight elsewhere.  us
-// per step, FP32 + Kahan (bfloat16 terms): variant 1 in contiguous ranges 855, 3 in
-// stripes 759, 5 in stripes 812 (128 shots Q4 400 x 400); 3 / 5 in stripes 455 / 487
-// (Q4 300 x 300), 92 / 88 (Q4 100 x 120), 499 / 493 (Q9 120 x 120), 426 / 423 (T6 120 x
-// 120), and 246 / 233 with a medium per shot (Q4 200 x 200).
-static void batched_default(const sfg_operator *op, const sfg_shot_desc *d, bool media, int *variant, int *xcd)
+// library, on meshes numbered line by line, where the state streams through HBM: XCD
+// stripes of an eighth of a line (a row's neighbours on the adjacent lines then come from
+// the same L2); streaming hints on large meshes of few nonzeros a row, three nonzeros in
+// flight elsewhere.  us per step, FP32 + Kahan (bfloat16 terms): variant 1 in contiguous
+// ranges 855, 3 in stripes 759, 5 in stripes 812 (128 shots Q4 400 x 400); 3 / 5 in stripes
+// 455 / 487 (Q4 300 x 300), 92 / 88 (Q4 100 x 120), 499 / 493 (Q9 120 x 120), 426 / 423
+// (T6 120 x 120), and 246 / 233 with a medium per shot (Q4 200 x 200).  In the caches
+// variant 1 is the faster one: 64 shots Q4 150 x 100 (226 MB) 45 / 58, T6 60 x 50 (181 MB) 45 /
+// 57, 128 shots Q4 40 x 40 (50 MB) 18.5 / 25; equal at 64 shots Q4 100 x 250 (337 MB) 71 / 73.
+static void batched_default(const sfg_operator *op, const sfg_shot_desc *d, const RunLoad &l, int *variant, int *xcd)
 {
-    if (d->shots_per_lane_group != 0 || d->kernel_variant != 0 || d->xcd_remap != 0 || d->row_order || d->nshots <= 16 ||
-        (d->block != 0 && d->block != 256))
-        return;
+    if (!default_shape(d) || d->xcd_remap != 0 || d->nshots <= 16 || l.bytes <= kStreams) return;
     const std::vector<int> line = line_candidates(op);
     if (line.empty()) return;
-    *variant = (media || op->nnz > 10LL * op->n || op->n < 65536) ? 5 : 3;
+    *variant = (l.media || op->nnz > 10LL * op->n || op->n < 65536) ? 5 : 3;
     *xcd = std::max(1, (line[0] + 16) / 32);     // 4 rows a block, 8 XCDs
 }
 
-// The layout the library takes for `nshots` shots, and its values (null: none).  With several shots
-// lines and patches start on 128-byte boundaries (64 with small patches): the state
-// then streams through HBM, and a line written in two parts costs its read back
-// (128 shots Q4 400 x 400 FP32 844 -> 804 us per step, 37 shots Q9 97 x 111 132 -> 124).
-static int choose_grid(const sfg_operator *op, int nshots, bool f32, hipStream_t st,
-                       std::shared_ptr<const GridPlan> *plan, std::shared_ptr<const GridValues> *vals)
+// Nodes that the lines and patches of a run of several shots start on a multiple of: 128
+// bytes (64 with small patches).  Once the state streams through HBM a line written in two
+// parts costs its read back (128 shots Q4 400 x 400 FP32 844 -> 804 us per step, 37 shots Q9
+// 97 x 111 132 -> 124); in the caches it is a tenth (150 x 100 64 shots 42.7 -> 39.7), and the
+// padding of a short line costs more than that (64 shots Q4 16 x 300, 17 nodes padded to 32,
+// FP64 42.7 -> 71, 128 shots Q4 40 x 40 FP32 16.2 -> 21).
+static int grid_align(const GridShape &lines, const RunLoad &l, int most)
+{
+    if (l.shots <= 1) return 0;
+    const double state = (double)lines.line * lines.lines * l.shots * (l.prec == 0 ? 8.0 : 4.0) *
+                         (2.0 * NFIELD + 2.0 * comp_fields(l.prec) + 4.0);
+    for (int a = most == 256 && l.prec != 0 ? 32 : 16; a >= 16; a /= 2) {
+        const double pitch = (lines.line + a - 1) / a * a;
+        if (pitch <= (state > 256e6 ? 1.3 : 1.08) * lines.line) return a;
+    }
+    return 0;
+}
+
+// The layout the library takes for a run, and its values (null: none).
+static int choose_grid(const sfg_operator *op, const RunLoad &l, hipStream_t st, std::shared_ptr<const GridPlan> *plan,
+                       std::shared_ptr<const GridValues> *vals)
 {
     std::lock_guard<std::mutex> lk(op->grid_mu);
     int rc = find_lines(op, st);
     if (rc || op->lines.line == 0) return rc;
     std::shared_ptr<GridPlan> P;
     auto get = [&](int most) {
-        rc = grid_plan(op, most, nshots > 1 ? (most == 256 && f32 ? 32 : 16) : 0, st, &P);
+        const int align = grid_align(op->lines, l, most);
+        GridShape g = op->lines;
+        g.most = most;
+        const double cost = choose_patch(g, most, align);
+        if (g.npatch == 0 || !grid_pays(op, l, g, cost)) return false;
+        rc = grid_plan(op, most, align, st, &P);
         return rc == SFG_OK && P;
     };
-    if (!get(grid_rows(op->n, nshots, std::max(op->lines.hx, op->lines.hy))) && rc == SFG_OK) (void)get(256);
+    const int most = grid_rows(op->n, l.shots, std::max(op->lines.hx, op->lines.hy));
+    if (!get(most) && rc == SFG_OK && most != 256) (void)get(256);
     if (rc || !P) return rc;
     // with all seven values per row the matrices are read again for every shot, which
     // lane groups of many shots do not (T6 120 x 120 FP64, 64 shots: 922 us per step
     // against 687; Q9 100 x 100 FP64, 24 shots: 331 / 481)
-    if (P->mode == GRID_ROWS && nshots > 32) return SFG_OK;
+    if (P->mode == GRID_ROWS && l.shots > 32) return SFG_OK;
     // (padded lines may exceed the index range where lane groups do not)
-    if ((size_t)P->g.pitch * P->g.lines * nshots >= (size_t)1 << 31) return SFG_OK;
-    if ((rc = grid_values(op, *P, f32, st, vals))) return rc;
+    if ((size_t)P->g.pitch * P->g.lines * l.shots >= (size_t)1 << 31) return SFG_OK;
+    if ((rc = grid_values(op, *P, l.prec != 0, st, vals))) return rc;
     *plan = P;
     return SFG_OK;
 }
@@ -834,7 +907,6 @@ static int choose_grid(const sfg_operator *op, int nshots, bool f32, hipStream_t
 // runs
 
 // 4- or 8-byte words per (node, shot) of one Kahan-term buffer
-static size_t comp_fields(int prec) { return prec == 3 ? 3 : prec == 2 ? 6 : 0; }
 
 struct sfg_run {
     const sfg_operator *op = nullptr;
@@ -1052,15 +1124,16 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
         return fail(SFG_E_HIP, "run setup: %s", hipGetErrorString(es));
     }
     // lane grouping: shots per lane group and the padded shot stride
-    if (grid && n < 1 << 28 && grid_default(op, d)) {
-        int rc = choose_grid(op, d->nshots, r->prec != 0, r->stream, &r->plan, &r->vals);
+    const RunLoad load = run_load(n, r->prec, r->cps, steps);
+    if (grid && n < 1 << 28 && default_shape(d)) {
+        int rc = choose_grid(op, load, r->stream, &r->plan, &r->vals);
         if (rc) {
             run_free(r);
             return rc;
         }
     }
     int variant = d->kernel_variant, xcd = d->xcd_remap;
-    if (!r->plan) batched_default(op, d, nmedia > 1, &variant, &xcd);
+    if (!r->plan) batched_default(op, d, load, &variant, &xcd);
     if (r->plan) r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
     const int lanes =
         d->shots_per_lane_group ? d->shots_per_lane_group : d->nshots <= 1 ? 1 : d->nshots <= 4 ? 4 : d->nshots <= 16 ? 16 : 64;
