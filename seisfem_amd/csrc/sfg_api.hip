@@ -782,27 +782,33 @@ static bool default_shape(const sfg_shot_desc *d)
 struct RunLoad {
     int prec = 0, shots = 0;
     bool media = false;         // a medium per shot
-    double active = 0, lanes = 0; // shot-steps, and those of 64-shot lane groups that step until their last shot ends
-    double bytes = 0;           // state (both buffers) and coefficients of a medium per shot, in 64-shot lane groups
+    double active = 0, lanes = 0; // shot-steps, and those of lane groups that step until their last shot ends
+    double bytes = 0;           // state (both buffers) and coefficients of a medium per shot
 };
+
+// Shots per lane group where it is left to the library
+static int lane_group(int nshots) { return nshots <= 1 ? 1 : nshots <= 4 ? 4 : nshots <= 16 ? 16 : 64; }
+
 static RunLoad run_load(int n, int prec, bool media, std::vector<int> steps)
 {
     RunLoad l;
     l.prec = prec;
     l.shots = (int)steps.size();
     l.media = media;
+    const int G = lane_group(l.shots);
     std::sort(steps.begin(), steps.end(), std::greater<int>());
-    for (size_t s = 0; s < steps.size(); ++s) {
+    for (int s = 0; s < l.shots; ++s) {
         l.active += steps[s];
-        if (s % 64 == 0) l.lanes += 64.0 * steps[s];
+        if (s % G == 0) l.lanes += (double)G * steps[s];
     }
-    l.bytes = (double)n * ((l.shots + 63) / 64 * 64) * (prec == 0 ? 8.0 : 4.0) *
+    l.bytes = (double)n * l.shots * (prec == 0 ? 8.0 : 4.0) *
               (2.0 * NFIELD + 2.0 * comp_fields(prec) + (media ? 12.0 : 0.0));
     return l;
 }
-// State in lane groups from which it streams through HBM: 4/3 of the Infinity Cache (below,
-// the hints of data used once cost more than they save; see batched_default)
-static const double kStreams = 340e6;
+// Whether the state streams through HBM in lane groups: somewhat more of it than the 256 MB
+// Infinity Cache holds (with less, the hints of data used once cost more than they save;
+// see batched_default)
+static bool streams(const RunLoad &l) { return l.bytes > (l.prec == 0 ? 300e6 : 340e6); }
 
 // Whether the grid layout in patches of shape g (of `cost`, see choose_patch) is taken for
 // a run of more than 16 shots rather than 64-shot lane groups.  A grid step costs by its
@@ -823,7 +829,7 @@ static bool grid_pays(const sfg_operator *op, const RunLoad &l, const GridShape 
 {
     if (l.shots <= 16) return true; // (lane groups of 16 or fewer: 8 shots Q4 300 x 300 FP64 93 / 257, FP32 28 / 85)
     const double fill = (double)op->n / ((double)g.npatch * g.most);
-    const bool stream = l.bytes > kStreams, long_rows = op->nnz > 14LL * op->n;
+    const bool long_rows = op->nnz > 14LL * op->n;
     const double steps = l.lanes > 0 ? l.active / l.lanes : 1.0;
     if (l.prec == 0) return 0.5 / std::pow(fill, 1.4) * steps <= 1.0;
     if (long_rows) {
@@ -832,7 +838,30 @@ static bool grid_pays(const sfg_operator *op, const RunLoad &l, const GridShape 
         return 0.6 / std::pow(fill, 1.4) * (blocks > 2048 ? 1.15 : 1.0) * steps <= 1.0;
     }
     const double bytes = cost / ((double)op->n * 8.0 * 38.0);   // touched over needed
-    return stream ? 0.78 * bytes * steps <= 0.9 : 0.68 * bytes * steps <= 0.84;
+    if (streams(l)) return 0.78 * bytes * steps <= 0.9;
+    return op->nnz > 10LL * op->n ? 0.64 * bytes * steps <= 0.96 : 0.68 * bytes * steps <= 0.84;
+}
+
+// The same where all seven values are stored per row (GRID_ROWS): the matrices are then
+// read again for every shot, which full lane groups do not.  us per step, grid / lane groups,
+// all shots active: FP64 16 shots Q4 150 x 100 54 / 41, Q4 300 x 300 289 / 273, T6 60 x 50 60 / 52,
+// Q9 120 x 100 273 / 255; FP32 + Kahan (bfloat16 terms) 16 shots Q4 300 x 300 143 / 127, T6 60 x
+// 50 25 / 25, Q9 120 x 100 (25 MB of matrices) 134 / 74, 32 shots Q4 150 x 100 44 / 38, Q9 120 x
+// 100 260 / 186; on smaller meshes 16 shots Q4 40 x 40 FP64 10.5 / 14.2, Q9 20 x 20 FP32 11.5 /
+// 17.4.  Groups that are not full: FP64 8 shots Q4 300 x 300 154 / 256, 20 shots Q9 120 x 100 339 /
+// 565, FP32 8 shots Q9 120 x 100 53 / 75, 20 shots 166 / 195.  4 shots: Q4 150 x 100 FP64 18 / 19, Q9
+// 120 x 100 FP32 32 / 36.  64 shots T6 120 x 120 FP64 922 / 687.
+static bool rows_pay(const sfg_operator *op, const RunLoad &l)
+{
+    if (l.shots <= 4 || l.lanes == 0) return true;
+    if (l.shots > 32) return false;
+    const bool large = (double)op->n * l.shots > 1e5;
+    const bool heavy = l.prec != 0 && op->nnz > 14LL * op->n && op->nnz * 28.0 > 16e6;
+    double rho; // cost of an active shot, that of one in a full lane group being 1
+    if (l.shots <= 16) rho = !large ? 1.0 : heavy ? 1.85 : 1.3;
+    else if (l.prec == 0) rho = 1.9;
+    else rho = !large ? 1.4 : heavy ? 2.8 : 2.3;
+    return rho * l.active <= l.lanes;
 }
 
 // Variant and XCD map of 64-shot lane groups whose launch shape is left to the
@@ -844,10 +873,12 @@ static bool grid_pays(const sfg_operator *op, const RunLoad &l, const GridShape 
 // 455 / 487 (Q4 300 x 300), 92 / 88 (Q4 100 x 120), 499 / 493 (Q9 120 x 120), 426 / 423
 // (T6 120 x 120), and 246 / 233 with a medium per shot (Q4 200 x 200).  In the caches
 // variant 1 is the faster one: 64 shots Q4 150 x 100 (226 MB) 45 / 58, T6 60 x 50 (181 MB) 45 /
-// 57, 128 shots Q4 40 x 40 (50 MB) 18.5 / 25; equal at 64 shots Q4 100 x 250 (337 MB) 71 / 73.
+// 57, 128 shots Q4 40 x 40 (50 MB) 18.5 / 25; about equal at 64 shots Q4 100 x 250 (FP32, 337
+// MB) 71 / 73, 128 shots T6 60 x 50 (363 MB) 93 / 89; FP64 T6 60 x 50 48 shots (244 MB) 120 /
+// 133, 64 shots (325 MB) 154 / 140.
 static void batched_default(const sfg_operator *op, const sfg_shot_desc *d, const RunLoad &l, int *variant, int *xcd)
 {
-    if (!default_shape(d) || d->xcd_remap != 0 || d->nshots <= 16 || l.bytes <= kStreams) return;
+    if (!default_shape(d) || d->xcd_remap != 0 || d->nshots <= 16 || !streams(l)) return;
     const std::vector<int> line = line_candidates(op);
     if (line.empty()) return;
     *variant = (l.media || op->nnz > 10LL * op->n || op->n < 65536) ? 5 : 3;
@@ -892,10 +923,7 @@ static int choose_grid(const sfg_operator *op, const RunLoad &l, hipStream_t st,
     const int most = grid_rows(op->n, l.shots, std::max(op->lines.hx, op->lines.hy));
     if (!get(most) && rc == SFG_OK && most != 256) (void)get(256);
     if (rc || !P) return rc;
-    // with all seven values per row the matrices are read again for every shot, which
-    // lane groups of many shots do not (T6 120 x 120 FP64, 64 shots: 922 us per step
-    // against 687; Q9 100 x 100 FP64, 24 shots: 331 / 481)
-    if (P->mode == GRID_ROWS && l.shots > 32) return SFG_OK;
+    if (P->mode == GRID_ROWS && !rows_pay(op, l)) return SFG_OK;
     // (padded lines may exceed the index range where lane groups do not)
     if ((size_t)P->g.pitch * P->g.lines * l.shots >= (size_t)1 << 31) return SFG_OK;
     if ((rc = grid_values(op, *P, l.prec != 0, st, vals))) return rc;
@@ -1135,8 +1163,7 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
     int variant = d->kernel_variant, xcd = d->xcd_remap;
     if (!r->plan) batched_default(op, d, load, &variant, &xcd);
     if (r->plan) r->np = (r->plan->g.pitch * r->plan->g.lines + 31) / 32 * 32;
-    const int lanes =
-        d->shots_per_lane_group ? d->shots_per_lane_group : d->nshots <= 1 ? 1 : d->nshots <= 4 ? 4 : d->nshots <= 16 ? 16 : 64;
+    const int lanes = d->shots_per_lane_group ? d->shots_per_lane_group : lane_group(d->nshots);
     const int sp = r->plan ? 1 : lanes;
     if (sp != 1 && sp != 4 && sp != 16 && sp != 32 && sp != 64) {
         run_free(r);
