@@ -177,7 +177,7 @@ int sfg_run_create(sfg_run **run, const sfg_operator *op, const sfg_medium *md,
                    const sfg_shot_desc *desc);
 /* As sfg_run_create, with one medium per shot (media[nshots], all built on
  * op): many models of one mesh share the seven operator matrices while each
- * shot reads its own coefficients (stored [coef][node][shot] on the device).
+ * shot reads its own coefficients (copied at creation).
  * The reference runs one model per process; this batches them. */
 int sfg_run_create_media(sfg_run **run, const sfg_operator *op, const sfg_medium *const *media,
                          const sfg_shot_desc *desc);

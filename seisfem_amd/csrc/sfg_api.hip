@@ -1523,44 +1523,31 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
         return fail(SFG_E_HIP, "run setup: %s", hipGetErrorString(e));
     }
     if (r->cps) {
-        // one medium per shot: coefficients and flags become [.][node][shot] arrays
-        // in the internal (step-sorted) shot order
+        // one medium per shot: coefficients and flags become arrays of all shots in the
+        // internal (step-sorted) shot order
         std::vector<const void *> csrc(d->nshots), fsrc(d->nshots);
         for (int s = 0; s < d->nshots; ++s) {
             const sfg_medium *m = media[r->perm[s]];
             csrc[s] = r->prec == 0 ? (const void *)m->coef64 : (const void *)m->coef32;
             fsrc[s] = m->flag;
         }
-        if (r->plan) {
-            // shot-major, each shot's arrays as its medium holds them
-            const size_t nc = (size_t)NCOEF * n;
-            if ((rc = dalloc((char **)&r->coefp, nc * r->S * w)) || (rc = dalloc(&r->flagp, (size_t)n * r->S))) {
-                run_free(r);
-                return rc;
-            }
-            for (int s = 0; s < d->nshots && e == hipSuccess; ++s) {
-                e = hipMemcpyAsync((char *)r->coefp + s * nc * w, csrc[s], nc * w, hipMemcpyDeviceToDevice, r->stream);
-                if (e == hipSuccess)
-                    e = hipMemcpyAsync(r->flagp + (size_t)s * n, fsrc[s], sizeof(int) * (size_t)n,
-                                       hipMemcpyDeviceToDevice, r->stream);
-            }
-            if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-        } else {
-            const void **dsrc = nullptr;
-            if ((rc = dalloc((char **)&r->coefp, (size_t)NCOEF * F * w)) || (rc = dalloc(&r->flagp, F)) ||
-                (rc = dalloc((char **)&dsrc, sizeof(void *) * 2 * d->nshots))) {
-                dfree(dsrc);
-                run_free(r);
-                return rc;
-            }
-            e = hipMemcpy(dsrc, csrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
-            if (e == hipSuccess)
-                e = hipMemcpy(dsrc + d->nshots, fsrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = launch_pack_per_shot(dsrc, d->nshots, NCOEF, n, r->S, (int)w, r->coefp, r->stream);
-            if (e == hipSuccess) e = launch_pack_per_shot(dsrc + d->nshots, d->nshots, 1, n, r->S, 4, r->flagp, r->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+        // [.][node][shot], or (grid layout) [shot][.][node], each shot's as its medium holds them
+        const size_t per = r->plan ? (size_t)n * r->S : F;
+        const void **dsrc = nullptr;
+        if ((rc = dalloc((char **)&r->coefp, (size_t)NCOEF * per * w)) || (rc = dalloc(&r->flagp, per)) ||
+            (rc = dalloc((char **)&dsrc, sizeof(void *) * 2 * d->nshots))) {
             dfree(dsrc);
+            run_free(r);
+            return rc;
         }
+        const bool sm = r->plan != nullptr;
+        e = hipMemcpy(dsrc, csrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
+        if (e == hipSuccess)
+            e = hipMemcpy(dsrc + d->nshots, fsrc.data(), sizeof(void *) * d->nshots, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = launch_pack_per_shot(dsrc, d->nshots, NCOEF, n, r->S, (int)w, sm, r->coefp, r->stream);
+        if (e == hipSuccess) e = launch_pack_per_shot(dsrc + d->nshots, d->nshots, 1, n, r->S, 4, sm, r->flagp, r->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+        dfree(dsrc);
         if (e != hipSuccess) {
             run_free(r);
             return fail(SFG_E_HIP, "run setup (per-shot media): %s", hipGetErrorString(e));

@@ -304,9 +304,10 @@ hipError_t launch_sell_values(const void *vals, size_t nnz, const int *src, size
 // pattern rp/ci, else 0
 hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, size_t cs, size_t is, size_t ss,
                            const int *rp, const int *ci, int *pml, hipStream_t st);
-// dst[c][i][s] = srcs[min(s, nsrc-1)][c*n + i] for c < ncoef, i < n, s < S; elem = 4 or 8 bytes
+// dst[c][i][s] (shot_major: dst[s][c][i]) = srcs[min(s, nsrc-1)][c*n + i] for c < ncoef, i < n,
+// s < S; elem = 4 or 8 bytes
 hipError_t launch_pack_per_shot(const void *const *srcs_dev, int nsrc, int ncoef, int n, int S, int elem,
-                                void *dst, hipStream_t st);
+                                bool shot_major, void *dst, hipStream_t st);
 hipError_t launch_elastic_slices(int n, const int *rp, const int *ci, const double *A, size_t nnz, const int *off,
                                  size_t nslots, int *cols, double *vals, hipStream_t st);
 hipError_t launch_elastic_apply(int n, const int *rp, const int *off, size_t nslots, const int *cols,

@@ -1280,14 +1280,18 @@ __global__ void fill_zero_kernel(uint32_t *p, size_t nwords)
         p[i] = 0u;
 }
 
+// (pml zeroed beforehand; a thread takes one row of one shot, those that find a profile
+// store the same value)
 template <class T>
 __global__ void pml_rows_kernel(const T *coef, int n, int ns, size_t cs, size_t is, size_t ss, int *pml)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const size_t total = (size_t)n * ns;
+    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
+        const size_t i = ss == 1 ? q / ns : q % n, s = ss == 1 ? q % ns : q / n;
         int any = 0;
-        for (int c = DX; c <= DYYP; ++c)
-            for (int s = 0; s < ns; ++s) any |= coef[c * cs + i * is + s * ss] != T(0);
-        pml[i] = any ? 2 : 0;
+#pragma unroll
+        for (int c = DX; c <= DYYP; ++c) any |= coef[c * cs + i * is + s * ss] != T(0);
+        if (any) pml[i] = 2;
     }
 }
 
@@ -1309,13 +1313,15 @@ hipError_t launch_pml_rows(int precision, const void *coef, int n, int ns, size_
 {
     const int blocks = (n + 255) / 256 < 4096 ? (n + 255) / 256 : 4096;
     if (n <= 0) return hipSuccess;
+    hipError_t e = launch_fill_zero(pml, sizeof(int) * (size_t)n, st);
+    if (e != hipSuccess) return e;
+    const size_t pairs = ((size_t)n * ns + 255) / 256;
+    const dim3 g(pairs < 4096 ? (unsigned int)pairs : 4096);
     if (precision == 0)
-        hipLaunchKernelGGL(pml_rows_kernel<double>, dim3(blocks), dim3(256), 0, st, (const double *)coef, n, ns, cs,
-                           is, ss, pml);
+        hipLaunchKernelGGL(pml_rows_kernel<double>, g, dim3(256), 0, st, (const double *)coef, n, ns, cs, is, ss, pml);
     else
-        hipLaunchKernelGGL(pml_rows_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float *)coef, n, ns, cs,
-                           is, ss, pml);
-    hipError_t e = hipGetLastError();
+        hipLaunchKernelGGL(pml_rows_kernel<float>, g, dim3(256), 0, st, (const float *)coef, n, ns, cs, is, ss, pml);
+    e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(pml_ring_kernel, dim3(blocks), dim3(256), 0, st, n, rp, ci, pml);
     return hipGetLastError();
@@ -1346,25 +1352,25 @@ hipError_t launch_medium_f32(int n, const double *coef64, const int *flag, float
 // Per-shot coefficients: shot-innermost copy of each medium's [ncoef][n] array.
 // Padded shots (s >= nsrc) repeat the last medium so every lane reads finite data.
 template <class E>
-__global__ void pack_per_shot_kernel(const E *const *srcs, int nsrc, int ncoef, int n, int S, E *dst)
+__global__ void pack_per_shot_kernel(const E *const *srcs, int nsrc, int ncoef, int n, int S, bool shot_major, E *dst)
 {
-    const size_t total = (size_t)ncoef * n * S;
+    const size_t per = (size_t)ncoef * n, total = per * S;
     for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < total; q += (size_t)gridDim.x * blockDim.x) {
-        const int s = (int)(q % S);
-        const size_t ci = q / S; // c * n + i
+        const int s = (int)(shot_major ? q / per : q % S);
+        const size_t ci = shot_major ? q - s * per : q / S; // c * n + i
         dst[q] = srcs[s < nsrc ? s : nsrc - 1][ci];
     }
 }
 
 hipError_t launch_pack_per_shot(const void *const *srcs_dev, int nsrc, int ncoef, int n, int S, int elem,
-                                void *dst, hipStream_t st)
+                                bool shot_major, void *dst, hipStream_t st)
 {
     if (elem == 8)
         hipLaunchKernelGGL(pack_per_shot_kernel<uint64_t>, dim3(2048), dim3(256), 0, st,
-                           (const uint64_t *const *)srcs_dev, nsrc, ncoef, n, S, (uint64_t *)dst);
+                           (const uint64_t *const *)srcs_dev, nsrc, ncoef, n, S, shot_major, (uint64_t *)dst);
     else if (elem == 4)
         hipLaunchKernelGGL(pack_per_shot_kernel<uint32_t>, dim3(2048), dim3(256), 0, st,
-                           (const uint32_t *const *)srcs_dev, nsrc, ncoef, n, S, (uint32_t *)dst);
+                           (const uint32_t *const *)srcs_dev, nsrc, ncoef, n, S, shot_major, (uint32_t *)dst);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
