@@ -1936,11 +1936,16 @@ extern "C" int sfg_estimate_dt(const sfg_operator *op, const sfg_medium *md, int
     }
     for (auto &v : x0) v /= std::sqrt(nrm);
     // Iterations are launched in batches, whose norms come back together: one at a time
-    // each waited for its own norm (200 x 150 Q4: 25 us an iteration, 9 in batches).  A batch is a quarter of the iterations so far, so that those past the end, whose
-    // norms are not looked at, stay few.  sums: |y|^2 of each iteration of this batch and the
-    // one before it (in turn in each half), after the start vector's.
+    // each waited for its own norm (200 x 150 Q4: 25 us an iteration, 9 in batches).  A batch
+    // is a quarter of the iterations so far, so that those past the end, whose norms are not
+    // looked at, stay few.  sums: |y|^2 of each iteration of this batch and the one before it
+    // (in turn in each half), after the start vector's.
     const int most = 64;
-    std::vector<int> off((n + 63) / 64);  // first slot of each slice of 64 rows
+    // The values in slices of 64 rows cost a pass over the matrices, which fewer than four
+    // iterations do not earn (one iteration Q4 40 x 40 0.06 ms, 0.09 with slices, Q9 250 x 250 1.6
+    // and 2.0; five are faster with them)
+    bool sliced = max_iter >= 4;
+    std::vector<int> off(sliced ? (n + 63) / 64 : 0);  // first slot of each slice
     size_t nslots = 0;
     for (size_t c = 0; c < off.size(); ++c) {
         off[c] = (int)nslots;
@@ -1950,7 +1955,7 @@ extern "C" int sfg_estimate_dt(const sfg_operator *op, const sfg_medium *md, int
     }
     // (a few rows far longer than the others would pad the slices to many times the matrix:
     // such an operator is read in the order of its CSR arrays)
-    bool sliced = nslots * 64 <= 4 * (size_t)op->nnz;
+    sliced = sliced && nslots * 64 <= 4 * (size_t)op->nnz;
     struct Tmp { // device memory of this call
         double *x = nullptr, *y = nullptr, *sums = nullptr, *vals = nullptr;
         int *off = nullptr, *cols = nullptr;
