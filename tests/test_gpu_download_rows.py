@@ -52,3 +52,39 @@ def test_padded_rows_take_the_time_of_packed_ones():
         ms[nin] = median_ms(lambda: net.layer(0))
         net.close()
     assert ms[13] < 10 * ms[32] + 0.5, ms
+
+
+# below, at and above the sizes where the way of a copy changes (64 KB, 256 KB, 4 MB), shots in
+# the caller's order and not, with and without the large pinned buffers of an earlier download
+@pytest.mark.parametrize("large_first", [False, True])
+@pytest.mark.parametrize("shots,steps,nrec", [(3, 20, 100), (4, 40, 60), (7, 40, 400), (9, 160, 400)])
+def test_seismograms_of_all_sizes(shots, steps, nrec, large_first):
+    from seisfem_amd import gpu, host
+    en, x, y = host.mesh_structured(host.Q4, 20, 20, 0.0, 200.0, 0.0, 200.0)
+    vp, rho = np.full(x.size, 3000.0), np.full(x.size, 2000.0)
+    prob = host.build_problem(host.Q4, en, x, y, rho, host.elastic_constants(rho, vp, vp / 1.73), vp, 10.0, 5, 5, 1,
+                              bbox=(0.0, 200.0, 0.0, 200.0))
+    op = gpu.Operator(prob["node_num"], prob["csr"])
+    md = gpu.Medium(op, prob["c"], prob["mass_lump"], prob["dirichlet"], prob["mpml"])
+    say(f"{shots} shots of {steps} steps at {nrec} receivers, large buffers first: {large_first}")
+    net = surrogate.MLP(13, 1100, 1, 1100, batch=32, seed=1)
+    if large_first:
+        net.layer(1)                                 # 4.8 MB
+    src = (150 + 11 * np.arange(shots)).astype(np.int32)
+    rec = np.arange(nrec, dtype=np.int32)
+    for order in (np.full(shots, steps), steps - (np.arange(shots) * 5) % 9):
+        nsteps = order.astype(np.int32)
+        run = gpu.Run(op, md, src, steps, rec, 5.0e-4, 25.0, 0.01, nsteps=nsteps, guard_every=40)
+        run.advance(steps)
+        u, w = run.seismograms()
+        run.close()
+        assert np.max(np.abs(u)) > 0
+        for s in range(shots):
+            one = gpu.Run(op, md, src[s:s + 1], steps, rec[s::50], 5.0e-4, 25.0, 0.01, nsteps=nsteps[s:s + 1],
+                          guard_every=40)
+            one.advance(steps)
+            u1, w1 = one.seismograms()
+            one.close()
+            assert np.array_equal(u[s, :, s::50], u1[0]) and np.array_equal(w[s, :, s::50], w1[0]), s
+    for h in (net, md, op):
+        h.close()
