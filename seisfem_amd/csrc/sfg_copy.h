@@ -7,8 +7,8 @@
 
 namespace sfg {
 
-// Pinned staging buffers of the process (four sets of 16 MB and a small one, a set for each download under
-// way), held by the objects that download through them and freed with the last of
+// Pinned staging buffers of the process (at most four sets of 16 MB, one for each download
+// under way), held by the objects that download through them and freed with the last of
 // these.
 struct Staging;
 std::shared_ptr<Staging> staging();

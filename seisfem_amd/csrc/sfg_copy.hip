@@ -18,15 +18,13 @@ constexpr size_t kPiece = (size_t)1 << 20;   // bytes of one transfer; two buffe
 // with one set they took turns, and a small result waited for the largest (4.5 MB beside
 // 131 MB 4.7 ms, with sets of their own 0.9; four threads of 131 MB each 17 ms, 15).
 constexpr int kSets = 4;
-// Results below kDirect are copied directly; those of up to kSmall through a small set
-// (the runtime's own staging takes two to five times as long there); those below kOne by the
-// caller's thread alone, through a set if there is one (a new one costs a page fault per 4 KB
-// too); larger ones by all threads.  us into memory in use / fresh memory, copied directly,
-// through a set by one thread, by 8 threads: 16 KB 18 / 15, 12 / 14, 67 / 93; 128 KB 62 /
-// 31, 14 / 30, 103 / 100; 1 MB 67 / 252, 61 / 244, 110 / 361; 4 MB 243 / 990, 220 / 940, 254 /
-// 736; 16 MB 927 / 3699, 823 / 3557, 645 / 1185.
+// Results below kDirect are copied directly; those below kOne by the caller's thread alone,
+// through a set if there is one (a new one costs its allocation, 20 us to a millisecond, and a
+// page fault per 4 KB); larger ones by all threads.  us into memory in use / fresh memory,
+// copied directly, through a set by one thread, by 8 threads: 16 KB 18 / 15, 12 / 14, 67 /
+// 93; 128 KB 62 / 31, 14 / 30, 103 / 100; 1 MB 67 / 252, 61 / 244, 110 / 361; 4 MB 243 / 990,
+// 220 / 940, 254 / 736; 16 MB 927 / 3699, 823 / 3557, 645 / 1185.
 constexpr size_t kDirect = (size_t)64 << 10;
-constexpr size_t kSmall = (size_t)256 << 10;
 constexpr size_t kOne = (size_t)4 << 20;
 std::mutex g_mu;
 std::weak_ptr<Staging> g_staging;
@@ -40,33 +38,30 @@ struct Staging {
         bool tried = false;
         // the buffers, locked by lk until the download ends; null: in use, no memory, or (make
         // false) not allocated yet
-        char *take(std::unique_lock<std::mutex> &lk, size_t bytes, bool make)
+        char *take(std::unique_lock<std::mutex> &lk, bool make)
         {
             lk = std::unique_lock<std::mutex>(mu, std::try_to_lock);
             if (!lk.owns_lock()) return nullptr;
             if (make && !tried) {
                 tried = true;
-                if (hipHostMalloc((void **)&buf, bytes, hipHostMallocPortable) != hipSuccess) {
+                if (hipHostMalloc((void **)&buf, 2 * kThreads * kPiece, hipHostMallocPortable) != hipSuccess) {
                     (void)hipGetLastError();
                     buf = nullptr;
                 }
             }
             return buf;
         }
-    } small, sets[kSets];
+    } sets[kSets];
     // pinned memory for a result of so many bytes (null: none)
     char *get(std::unique_lock<std::mutex> &lk, size_t bytes)
     {
         if (bytes < kDirect) return nullptr;
-        if (bytes <= kSmall)
-            if (char *b = small.take(lk, kSmall, true)) return b;
         for (Set &x : sets)
-            if (char *b = x.take(lk, 2 * kThreads * kPiece, bytes >= kOne)) return b;
+            if (char *b = x.take(lk, bytes >= kOne)) return b;
         return nullptr;
     }
     ~Staging()
     {
-        if (small.buf) (void)hipHostFree(small.buf);
         for (Set &x : sets)
             if (x.buf) (void)hipHostFree(x.buf);
     }
