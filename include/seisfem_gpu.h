@@ -214,7 +214,8 @@ int sfg_run_energy(sfg_run *run, double *energy, int max_checks);
  * run's stream over the last sfg_run_advance call (0 if unavailable). */
 double sfg_run_last_ms_per_step(const sfg_run *run);
 /* Algorithmic HBM bytes of one step kernel launch (operator + coefficients +
- * state traffic of the active shots). */
+ * state traffic of the active shots), those of the reference's form in every
+ * layout: the grid layout reads few matrix bytes where rows share stencils. */
 double sfg_run_step_bytes(const sfg_run *run, int active_shots);
 void sfg_run_destroy(sfg_run *run);
 
@@ -224,8 +225,9 @@ void sfg_run_destroy(sfg_run *run);
  * uneven size and step count) so that they step together: each step, every
  * batched run large enough to fill the GPU alone takes its own step launch,
  * the smaller batched runs (32 or 64 shots per lane group) share one launch,
- * and the single-shot runs share one launch per layout (kernel variant 9 in a
- * launch of its own, with the largest halo's LDS); all of them read one device
+ * the single-shot runs share one launch per layout (kernel variant 9 in a
+ * launch of its own, with the largest halo's LDS), and the runs in the grid
+ * layout one per patch size (64, 128 or 256 rows); all of them read one device
  * step counter and the launches of guard_every steps are captured in one
  * hipGraph.  The runs must share precision, max_steps (use per-shot nsteps for
  * uneven lengths), block size and guard interval and not have stepped yet.
@@ -241,9 +243,10 @@ double sfg_multi_last_ms_per_step(const sfg_multi *multi);
  * cooperative launch per guard interval, in which blocks_per_cu x (CU count)
  * resident blocks take each step's tiles from a queue and meet at a grid-wide
  * barrier between steps; 0 returns to the graph-replayed per-step launches.
- * Results are identical bit for bit.  Needs every run in one shared launch
- * (single-shot runs in the per-row or sliced layouts, or only batched runs
- * too small to fill the GPU alone); fails if that many blocks cannot be
+ * Results are identical bit for bit.  Needs single-shot runs in the per-row,
+ * sliced or grid layouts only (which share one launch), or only batched runs
+ * too small to fill the GPU alone (those in lane groups share one, those in
+ * the grid layout one per patch size); fails if that many blocks cannot be
  * resident at once.  No counterpart in the reference. */
 int sfg_multi_set_persistent(sfg_multi *multi, int blocks_per_cu);
 /* Algorithmic bytes of the launch of step `step` (shots still active then). */

@@ -1,7 +1,8 @@
 // Grid layout of the step kernel: meshes numbered line by line, stepped in
 // patches with the neighbours' fields in LDS and the matrices as stencil classes
-// (see GridArgs).  Same arithmetic per row as step_tile (sfg_kernels.hip): every
-// sum runs in column order, and the FPB4 form is bit-identical to the reference.
+// (see GridArgs).  Same arithmetic per row as step_tile (sfg_kernels.hip), which a change
+// here has to follow (the persistent schedule steps the same runs by either): every
+// sum runs in column order, and the FP64 form is bit-identical to the reference.
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
@@ -87,7 +88,7 @@ struct alignas(8 * sizeof(T)) Entry {
 // Values of T per halo position in LDS: part A holds U, W, Lx1..4, Ly1..4, part B
 // the split displacements and velocities.  Strides of an odd number of 16-byte
 // words keep the 16-byte reads of neighbouring positions on different banks (FP32:
-// 12 = 3 words; FPB4: 10 and 14 = 5 and 7 words; part B in FP32 is 3 words as is).
+// 12 = 3 words; FP64: 10 and 14 = 5 and 7 words; part B in FP32 is 3 words as is).
 template <class T> constexpr int LDS_A = sizeof(T) == 4 ? 12 : 10;
 template <class T> constexpr int LDS_B = sizeof(T) == 4 ? 12 : 14;
 
@@ -148,10 +149,13 @@ struct Stencil {
 // row forms the products that rows outside the damping layers need (and S5, S6
 // where the patch has M-PML rows).  Only patches with M-PML rows also stage the 12
 // split displacements and velocities (part B): with TOG beside part A, all products
-// in one walk; else over it after a barrier, in a second walk of the M-PML rows.  A row outside the layers multiplies those products by
-// exact zeros, in FPB4 too: leaving them at zero changes no bit of U and W (a sum
-// plus a signed zero is unchanged, and the displacements, which start at +0, never
-// become -0).  The patch's class table precedes them in LDS.
+// in one walk; else over it after a barrier, in a second walk of the M-PML rows.  A row
+// outside the layers multiplies those products by exact zeros, in FP64 too: while the
+// fields are finite, leaving them at zero changes no bit of U and W (a sum plus a signed
+// zero is unchanged, and the displacements, which start at +0, never become -0).  Once a
+// split field has overflowed the reference's form has a NaN there (zero times infinity)
+// and this one has not; the energy guard ends such a run either way.  The patch's class
+// table precedes them in LDS.
 template <class T, int PREC, bool CPS, int MODE, bool TOG>
 __device__ __forceinline__ void grid_tile(const StepArgs<T> &a, const GridArgs<T> &g, int t, int slot, int patch, int s,
                                           bool lead)
@@ -783,7 +787,7 @@ hipError_t launch_multi_grid(int precision, const void *runs_dev, const int *til
     return hipGetLastError();
 }
 
-// FPB4 patches may take more than the default 64 KB of dynamic LDS
+// FP64 patches may take more than the default 64 KB of dynamic LDS
 // (GRID_HALO_MAX x 24 values x 8 bytes + GRID_TABLE entries of 64 bytes = 122 KB)
 hipError_t allow_grid_lds()
 {

@@ -187,7 +187,7 @@ struct GridArgs {
     int mode;
     int np;                     // padded nodes: field stride of a shot
     int magic;                  // q / W == q * magic >> 16 for halo positions q
-    int together;               // 1: a patch stages all its fields at once (FP64; the FP32 forms always do)
+    int together;               // 1: a patch stages all its fields at once (grid_together)
     int steps0;                 // executed steps of shot 0 (single-shot runs)
     const int *rows;            // [npatch * most] row at each place, -1 = none
     const int *cls;             // [npatch * most] first entry of the row's class in its patch's table | its
