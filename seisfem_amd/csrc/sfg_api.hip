@@ -227,6 +227,7 @@ struct GridPlan {
     bool ok = false;            // false: the operator does not fit the layout
     GridShape g;
     int mode = GRID_ROWS, magic = 0;
+    // (rows holds cls, slice and smax too, toff holds tlen, trep and tdst)
     int *rows = nullptr, *cls = nullptr, *slice = nullptr, *smax = nullptr, *toff = nullptr, *tlen = nullptr,
         *trep = nullptr, *tdst = nullptr, *moff = nullptr, *sdel = nullptr;
     int nitems = 0;             // stencils in the tables
@@ -235,7 +236,7 @@ struct GridPlan {
     std::shared_ptr<const GridValues> vals[2]; // FP64, FP32
     ~GridPlan()
     {
-        for (int *q : {rows, cls, slice, smax, toff, moff, sdel}) dfree(q); // (toff holds tlen, trep and tdst too)
+        for (int *q : {rows, toff, moff, sdel}) dfree(q);
     }
 };
 
@@ -477,49 +478,78 @@ static bool patch_tables(GridShape &g, const std::vector<int> &cptr, const std::
     return true;
 }
 
-template <class T>
-static int upload(T **p, const std::vector<T> &v, hipStream_t st)
-{
-    int rc = dalloc(p, v.size());
-    if (rc) return rc;
-    if (!v.empty()) HIPCHK(hipMemcpyAsync(*p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice, st));
-    HIPCHK(hipStreamSynchronize(st));
-    return SFG_OK;
-}
+// Device scratch and host staging of one search for a layout.  Transfers and allocations of
+// a plan are small and each costs its latency (for 1681 nodes more than its kernels), so what
+// goes together is packed, and the stream is waited for once at the end (a new operator of
+// 3913 nodes: 220 us with an allocation per array and a wait per transfer, 170 so).
+struct GridBuild {
+    hipStream_t st = nullptr;
+    bool used = false;          // st has work that reads the members below
+    // device: the reach's flags, hashes without and with M, rows' classes, classes' first rows and entries
+    char *mem = nullptr;
+    int *flags = nullptr, *key = nullptr;
+    unsigned long long *h = nullptr;
+    bool hashed = false, fetched = false;
+    std::vector<unsigned long long> host; // flags (two words) and hashes as they come back
+    std::vector<int> keys, packed, tables, smax, moff;
+    explicit GridBuild(hipStream_t s) : st(s) {}
+    ~GridBuild()
+    {
+        if (used) (void)hipStreamSynchronize(st);
+        dfree(mem);
+    }
+    int alloc(int n)
+    {
+        if (mem) return SFG_OK;
+        int rc = dalloc(&mem, 16 + sizeof(unsigned long long) * 2 * n + sizeof(int) * ((size_t)n + 2 * kGridClasses + 1));
+        if (rc) return rc;
+        flags = (int *)mem;
+        h = (unsigned long long *)(mem + 16);
+        key = (int *)(h + 2 * (size_t)n);
+        return SFG_OK;
+    }
+};
+// Nodes up to which the hashes come back with the flags of the reach (16 bytes a node)
+static const int kHashesAhead = 32768;
 
 // The mesh's lines and the reach of its columns, found once per operator (the
 // caller holds grid_mu).
-static int find_lines(const sfg_operator *op, hipStream_t st)
+static int find_lines(const sfg_operator *op, GridBuild &b)
 {
     if (op->grid_tried) return SFG_OK;
-    int *flags = nullptr, f[4];
-    int rc = dalloc(&flags, 4);
-    if (rc) return rc;
-    hipError_t e = hipSuccess;
-    for (int l : line_candidates(op)) {
-        e = launch_fill_zero(flags, sizeof f, st);
-        if (e == hipSuccess) e = launch_grid_reach(op->n, op->rp, op->ci, l, flags, flags + 2, st);
-        if (e == hipSuccess) e = hipMemcpyAsync(f, flags, sizeof f, hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess || f[2] != 0) continue;
+    const std::vector<int> lines = line_candidates(op);
+    const size_t n = op->n;
+    int rc;
+    if (!lines.empty() && (rc = b.alloc(op->n))) return rc;
+    for (int l : lines) {
+        const bool ahead = !b.fetched && n <= (size_t)kHashesAhead;
+        b.host.resize(std::max(b.host.size(), ahead ? 2 + 2 * n : (size_t)2));
+        b.used = true;
+        HIPCHK(launch_fill_zero(b.flags, 4 * sizeof(int), b.st));
+        HIPCHK(launch_grid_reach(op->n, op->rp, op->ci, l, b.flags, b.flags + 2, b.st));
+        if (ahead) HIPCHK(launch_grid_hash(op->n, op->rp, op->ci, op->v64, (size_t)op->nnz, b.h, b.st));
+        HIPCHK(hipMemcpyAsync(b.host.data(), b.mem, 16 + (ahead ? 16 * n : 0), hipMemcpyDeviceToHost, b.st));
+        HIPCHK(hipStreamSynchronize(b.st));
+        if (ahead) b.hashed = b.fetched = true;
+        int f[4];
+        std::memcpy(f, b.host.data(), sizeof f);
+        if (f[2] != 0) continue;
         op->lines.line = l;
         op->lines.lines = op->n / l;
         op->lines.hx = f[0];
         op->lines.hy = f[1];
         break;
     }
-    dfree(flags);
-    if (e != hipSuccess) return fail(SFG_E_HIP, "grid layout: %s", hipGetErrorString(e));
     op->grid_tried = 1;
     return SFG_OK;
 }
 
-static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
+// (the caller waits for b.st)
+static int build_grid(const sfg_operator *op, GridPlan &P, GridBuild &b)
 {
     const int n = op->n;
+    const hipStream_t st = b.st;
     P.ok = false;
-    int rc = find_lines(op, st);
-    if (rc) return rc;
     GridShape g = op->lines;
     if (g.line == 0) return SFG_OK;
     g.most = P.most;
@@ -532,40 +562,42 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
     P.g = g;
     const int nw = g.npatch * (g.most / 64);
     const size_t nrows = (size_t)g.npatch * g.most;
-    struct Tmp { // device scratch of this call: hashes; rows' classes, classes' first rows and entries
-        int *key = nullptr;
-        unsigned long long *h = nullptr;
-        ~Tmp() { dfree(key); dfree(h); }
-    } tmp;
-    // (transfers of a plan are small and each costs its latency: what goes together is
-    // packed.  The flags of the check lie behind the keys that come back with them.)
-    if ((rc = dalloc(&tmp.h, 2 * (size_t)n)) || (rc = dalloc(&tmp.key, (size_t)n + 2 * kGridClasses + 1)) ||
-        (rc = dalloc(&P.rows, nrows)) || (rc = dalloc(&P.cls, nrows + 4)) || (rc = dalloc(&P.slice, nw)) ||
-        (rc = dalloc(&P.smax, nw)))
-        return rc;
+    int rc;
+    // (the flags of the check lie behind the keys that come back with them)
+    if ((rc = b.alloc(n)) || (rc = dalloc(&P.rows, 2 * nrows + 4 + 2 * (size_t)nw))) return rc;
+    P.cls = P.rows + nrows;
+    P.slice = P.cls + nrows + 4;
+    P.smax = P.slice + nw;
     int *const flags = P.cls + nrows;
+    b.used = true;
+    if (!b.hashed) HIPCHK(launch_grid_hash(n, op->rp, op->ci, op->v64, (size_t)op->nnz, b.h, st));
+    b.hashed = true;
+    if (!b.fetched) b.host.resize(2 + 2 * (size_t)n);
     // the most compact mode whose tables fit
-    std::vector<unsigned long long> h(n);
-    HIPCHK(launch_grid_hash(n, op->rp, op->ci, op->v64, (size_t)op->nnz, tmp.h, st));
-    std::vector<int> cls, rep, keys(nrows + 4), packed, cptr, toff, tlen, trep, tdst;
+    std::vector<int> cls, rep, cptr, toff, tlen, trep, tdst;
+    std::vector<int> &keys = b.keys;
+    keys.resize(nrows + 4);
     int mode = GRID_ROWS;
     for (int m = GRID_CLASS; m < GRID_ROWS && mode == GRID_ROWS; ++m) {
-        HIPCHK(hipMemcpyAsync(h.data(), tmp.h + (m == GRID_CLASS ? n : 0), sizeof(unsigned long long) * n,
-                              hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        if (!group_rows(h.data(), n, cls, rep)) continue;
+        const size_t half = m == GRID_CLASS ? n : 0;
+        unsigned long long *const h = b.host.data() + 2 + half;
+        if (!b.fetched) {
+            HIPCHK(hipMemcpyAsync(h, b.h + half, sizeof(unsigned long long) * n, hipMemcpyDeviceToHost, st));
+            HIPCHK(hipStreamSynchronize(st));
+        }
+        if (!group_rows(h, n, cls, rep)) continue;
         const int nclass = (int)rep.size();
         cptr.assign(nclass + 1, 0);
         for (int c = 0; c < nclass; ++c) cptr[c + 1] = cptr[c] + op->hrp[rep[c] + 1] - op->hrp[rep[c]];
-        packed = cls;
-        packed.insert(packed.end(), rep.begin(), rep.end());
-        packed.insert(packed.end(), cptr.begin(), cptr.end());
-        int *const drep = tmp.key + n, *const dcptr = drep + nclass;
+        b.packed = cls;
+        b.packed.insert(b.packed.end(), rep.begin(), rep.end());
+        b.packed.insert(b.packed.end(), cptr.begin(), cptr.end());
+        int *const drep = b.key + n, *const dcptr = drep + nclass;
         HIPCHK(launch_fill_zero(flags, 4 * sizeof(int), st));
-        HIPCHK(hipMemcpyAsync(tmp.key, packed.data(), sizeof(int) * packed.size(), hipMemcpyHostToDevice, st));
-        HIPCHK(launch_grid_check(n, op->rp, op->ci, op->v64, (size_t)op->nnz, m == GRID_CLASS ? 0 : 1, tmp.key, drep,
+        HIPCHK(hipMemcpyAsync(b.key, b.packed.data(), sizeof(int) * b.packed.size(), hipMemcpyHostToDevice, st));
+        HIPCHK(launch_grid_check(n, op->rp, op->ci, op->v64, (size_t)op->nnz, m == GRID_CLASS ? 0 : 1, b.key, drep,
                                  flags, st));
-        HIPCHK(launch_grid_sort(g, m, op->rp, tmp.key, dcptr, P.rows, P.cls, P.slice, P.smax, st));
+        HIPCHK(launch_grid_sort(g, m, op->rp, b.key, dcptr, P.rows, P.cls, P.slice, P.smax, st));
         HIPCHK(hipMemcpyAsync(keys.data(), P.cls, sizeof(int) * keys.size(), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         if (keys[nrows] == 0 && patch_tables(g, cptr, rep, keys, toff, tlen, trep, tdst, &P.nentries)) mode = m;
@@ -574,13 +606,14 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
     if (mode == GRID_ROWS) {
         g.table = 0;
         P.nentries = 0;
-        HIPCHK(launch_grid_sort(g, mode, op->rp, tmp.key, nullptr, P.rows, P.cls, P.slice, P.smax, st));
+        HIPCHK(launch_grid_sort(g, mode, op->rp, b.key, nullptr, P.rows, P.cls, P.slice, P.smax, st));
     } else {
         P.nitems = (int)trep.size();
         HIPCHK(hipMemcpyAsync(P.cls, keys.data(), sizeof(int) * nrows, hipMemcpyHostToDevice, st));
-        packed = toff;
-        for (const std::vector<int> *v : {&tlen, &trep, &tdst}) packed.insert(packed.end(), v->begin(), v->end());
-        if ((rc = upload(&P.toff, packed, st))) return rc;
+        b.tables = toff;
+        for (const std::vector<int> *v : {&tlen, &trep, &tdst}) b.tables.insert(b.tables.end(), v->begin(), v->end());
+        if ((rc = dalloc(&P.toff, b.tables.size()))) return rc;
+        HIPCHK(hipMemcpyAsync(P.toff, b.tables.data(), sizeof(int) * b.tables.size(), hipMemcpyHostToDevice, st));
         P.tlen = P.toff + toff.size();
         P.trep = P.tlen + tlen.size();
         P.tdst = P.trep + trep.size();
@@ -588,52 +621,50 @@ static int build_grid(const sfg_operator *op, GridPlan &P, hipStream_t st)
     P.g = g;
     HIPCHK(launch_grid_place(g, P.rows, P.cls, st));
     if (mode != GRID_CLASS) {
-        std::vector<int> smax(nw), moff(nw);
-        HIPCHK(hipMemcpyAsync(smax.data(), P.smax, sizeof(int) * nw, hipMemcpyDeviceToHost, st));
+        b.smax.resize(nw);
+        b.moff.resize(nw);
+        HIPCHK(hipMemcpyAsync(b.smax.data(), P.smax, sizeof(int) * nw, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         for (int w = 0; w < nw; ++w) {
-            moff[w] = (int)P.nslots;
-            P.nslots += smax[w];
+            b.moff[w] = (int)P.nslots;
+            P.nslots += b.smax[w];
         }
         if (P.nslots > 0x7fffffffLL / (7 * 64)) return SFG_OK;
-        if ((rc = upload(&P.moff, moff, st))) return rc;
+        if ((rc = dalloc(&P.moff, nw))) return rc;
+        HIPCHK(hipMemcpyAsync(P.moff, b.moff.data(), sizeof(int) * nw, hipMemcpyHostToDevice, st));
     }
-    HIPCHK(hipStreamSynchronize(st));
     P.ok = true;
     return SFG_OK;
 }
 
 // The operator's grid layout for patches of at most `most` rows, without values, built
-// on first use (on `st`, which it waits for; the caller holds grid_mu).  *out = null
+// on first use (on b.st, which the caller waits for; it holds grid_mu).  *out = null
 // when the operator does not fit the layout (no line structure).
-static int grid_plan(const sfg_operator *op, int most, int align, hipStream_t st, std::shared_ptr<GridPlan> *out)
+static int grid_plan(const sfg_operator *op, int most, int align, GridBuild &b, std::shared_ptr<GridPlan> *out)
 {
     out->reset();
     std::shared_ptr<GridPlan> P;
     for (const auto &p : op->grid)
         if (p->most == most && p->align == align) P = p;
     if (!P) {
-        try {
-            P = std::make_shared<GridPlan>();
-            P->most = most;
-            P->align = align;
-            int rc = build_grid(op, *P, st);
-            if (rc) return rc;
-            op->grid.push_back(P);
-        } catch (const std::bad_alloc &) {
-            return fail(SFG_E_NOMEM, "grid layout: out of host memory");
-        }
+        P = std::make_shared<GridPlan>();
+        P->most = most;
+        P->align = align;
+        int rc = build_grid(op, *P, b);
+        if (rc) return rc;
+        op->grid.push_back(P);
     }
     if (P->ok) *out = P;
     return SFG_OK;
 }
 
-// The layout's values in one precision, filled on first use (on `st`, which it waits
-// for; the caller holds grid_mu).
-static int grid_values(const sfg_operator *op, GridPlan &P, bool f32, hipStream_t st,
+// The layout's values in one precision, filled on first use (on b.st, which the caller
+// waits for; it holds grid_mu).
+static int grid_values(const sfg_operator *op, GridPlan &P, bool f32, GridBuild &b,
                        std::shared_ptr<const GridValues> *out)
 {
     const int k = f32 ? 1 : 0, w = f32 ? 4 : 8;
+    const hipStream_t st = b.st;
     if (!P.vals[k]) {
         const void *v = f32 ? (const void *)op->v32 : (const void *)op->v64;
         auto x = std::make_shared<GridValues>();
@@ -644,13 +675,13 @@ static int grid_values(const sfg_operator *op, GridPlan &P, bool f32, hipStream_
             if ((rc = dalloc((char **)&x->mval, (size_t)P.nslots * 64 * per * w))) return rc;
             if (P.mode == GRID_ROWS && !P.sdel && (rc = dalloc(&P.sdel, (size_t)P.nslots * 64))) return rc;
         }
+        b.used = true;
         if (P.nitems)
             HIPCHK(launch_grid_table(P.nitems, P.trep, P.tdst, op->rp, op->ci, P.g.line, P.g.W, v, (size_t)op->nnz, w,
                                      x->tab, st));
         if (P.mode != GRID_CLASS)
             HIPCHK(launch_grid_values(P.g.npatch * (P.g.most / 64), P.mode, P.rows, P.moff, P.smax, op->rp, op->ci,
                                       P.g.line, P.g.W, v, (size_t)op->nnz, w, x->mval, P.sdel, st));
-        HIPCHK(hipStreamSynchronize(st));
         P.vals[k] = std::move(x);
     }
     *out = P.vals[k];
@@ -908,7 +939,8 @@ static int choose_grid(const sfg_operator *op, const RunLoad &l, hipStream_t st,
                        std::shared_ptr<const GridValues> *vals)
 {
     std::lock_guard<std::mutex> lk(op->grid_mu);
-    int rc = find_lines(op, st);
+    GridBuild b(st);
+    int rc = find_lines(op, b);
     if (rc || op->lines.line == 0) return rc;
     std::shared_ptr<GridPlan> P;
     auto get = [&](int most) {
@@ -917,7 +949,7 @@ static int choose_grid(const sfg_operator *op, const RunLoad &l, hipStream_t st,
         g.most = most;
         const double cost = choose_patch(g, most, align);
         if (g.npatch == 0 || !grid_pays(op, l, g, cost)) return false;
-        rc = grid_plan(op, most, align, st, &P);
+        rc = grid_plan(op, most, align, b, &P);
         return rc == SFG_OK && P;
     };
     const int most = grid_rows(op->n, l.shots, std::max(op->lines.hx, op->lines.hy));
@@ -926,7 +958,9 @@ static int choose_grid(const sfg_operator *op, const RunLoad &l, hipStream_t st,
     if (P->mode == GRID_ROWS && !rows_pay(op, l)) return SFG_OK;
     // (padded lines may exceed the index range where lane groups do not)
     if ((size_t)P->g.pitch * P->g.lines * l.shots >= (size_t)1 << 31) return SFG_OK;
-    if ((rc = grid_values(op, *P, l.prec != 0, st, vals))) return rc;
+    if ((rc = grid_values(op, *P, l.prec != 0, b, vals))) return rc;
+    if (b.used) HIPCHK(hipStreamSynchronize(st));
+    b.used = false;
     *plan = P;
     return SFG_OK;
 }
@@ -1154,7 +1188,12 @@ static int run_create_as(sfg_run **out, const sfg_operator *op, const sfg_medium
     // lane grouping: shots per lane group and the padded shot stride
     const RunLoad load = run_load(n, r->prec, r->cps, steps);
     if (grid && n < 1 << 28 && default_shape(d)) {
-        int rc = choose_grid(op, load, r->stream, &r->plan, &r->vals);
+        int rc;
+        try {
+            rc = choose_grid(op, load, r->stream, &r->plan, &r->vals);
+        } catch (const std::bad_alloc &) {
+            rc = fail(SFG_E_NOMEM, "grid layout: out of host memory");
+        }
         if (rc) {
             run_free(r);
             return rc;
